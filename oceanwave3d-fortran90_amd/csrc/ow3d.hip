@@ -1057,9 +1057,13 @@ extern "C" long long ow3d_estimate_bytes(const ow3d_config *cfg) {
         std::vector<Grid> lev;
         if (!mg_levels(g, cfg->mg_maxgrids, lev, err())) return -1;
         const long long p = cfg->mg_precision == 0 ? 8 : 4, pc = cfg->mg_precision == 2 ? 2 : p;
+        ow3d_tank probe;   // the hierarchy and the settings that needs_b and needs_r read
+        probe.cfg = *cfg;
+        probe.levels = lev;
         for (size_t k = 0; k < lev.size(); k++) {
             const Grid &L = lev[k];
-            b += p * ((long long)L.n * 4 + 6LL * L.nxy + 12LL * (L.nxg + L.nyg + L.nzg)) + 8LL * (L.nxg + L.nyg + L.nzg);
+            b += p * ((long long)L.n * (2 + needs_b(&probe, (int)k) + needs_r(&probe, (int)k)) + 6LL * L.nxy + 12LL * (L.nxg + L.nyg + L.nzg)) + 8LL * (L.nxg + L.nyg + L.nzg);
+            if (k > 0 && has_records(L)) b += p * (long long)(p == 8 ? line_records<double>(L.nxg, L.nyg, L.nzg) : line_records<float>(L.nxg, L.nyg, L.nzg));
             if (k == 0) b += pc * (long long)L.n * (long long)minv_pitch((int)L.n);
         }
     }

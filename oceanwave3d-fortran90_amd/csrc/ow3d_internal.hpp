@@ -96,8 +96,20 @@ struct MgLevel {
     // restriction from this level onto the next coarser one in the same case: per coarse column (row) the
     // weights of the 3-point smoothing on the fine grid, (d_lo, d_lo + d_hi, d_hi, 1 / (2 (d_lo + d_hi))) in T
     DevBuf<T> rxw, ryw;
+    DevBuf<T> fac;   // records of the columns (LineRecord) for the sweeps
     LvArgs<T> args{};
 };
+
+// Levels above the coarsest whose columns' records are kept for the sweeps: all x-z levels and 3D ones of up to
+// SWEEP_RECORD_POINTS points (larger 3D levels take k_mg_sweep_tiled, which forms its line matrices).
+constexpr size_t SWEEP_RECORD_POINTS = size_t(1) << 20;
+inline bool has_records(const Grid &g) { return g.ny == 1 || g.n <= SWEEP_RECORD_POINTS; }
+// Values of a level's column records (LineRecord).
+template <typename T>
+size_t line_records(int nxg, int nyg, int nzg) {
+    const size_t w = 16 / sizeof(T), n = ((size_t)3 * nzg + 3 + w - 1) / w * w;
+    return n * LineRecord<T, 3>::count(nxg, nyg);
+}
 
 inline int grid_blocks(size_t n, int bs = 256) {
     size_t b = (n + bs - 1) / bs;
@@ -134,10 +146,11 @@ struct ow3d_tank {
     std::vector<Grid> levels;
     std::vector<std::unique_ptr<MgLevel<double>>> mg64;
     std::vector<std::unique_ptr<MgLevel<float>>> mg32;
+    long bot_lim = 0;                 // points a level handed to the one-workgroup bottom kernel may have (0: off)
     int bot_top = -1;                 // finest level handled by the one-workgroup bottom kernel (-1: none)
     bool fused_rb = true;             // one launch per zebra sweep (red and black halves) on the upper levels
     // launch choices (ow3d_tune): matvec variant 0 column kernel, widest tile / 1 column kernel, 8-row
-    // tiles / 2 point kernel; zebra-sweep block size 0 auto (1024 threads below 256 tiles) / 256 / 1024
+    // tiles / 2 point kernel; zebra-sweep block size 0 / 256 / 1024 (kept for callers; the sweeps have one block size)
     int mv_variant = 0;
     int rb_threads = 0;
     BottomArgs<double> bot64{};
@@ -196,6 +209,11 @@ int launch_matvec(const ow3d_tank *t, const double *phi, double *y, hipStream_t 
 bool matvec_supported(int nzg, int A);
 // multigrid (ow3d_mg.hip): hierarchy set-up for t->cfg and u = M^-1 r on device vectors
 int mg_setup(ow3d_tank *t);
+// Buffers of level k that some path uses (t->levels, t->fused_rb and t->bot_lim are set): the right-hand side, except
+// on an FP64 finest level whose first sweep reads the residual itself, and the residual, except where it goes into its
+// restriction in one launch.
+bool needs_b(const ow3d_tank *t, int k);
+bool needs_r(const ow3d_tank *t, int k);
 int precond(ow3d_tank *t, const double *r, double *u, hipStream_t s);
 // per-precision parts (ow3d_mg64.hip, ow3d_mg32.hip)
 int mg_build64(ow3d_tank *t);

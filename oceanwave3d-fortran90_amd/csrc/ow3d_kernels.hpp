@@ -17,6 +17,25 @@ __host__ __device__ constexpr int cmin(int a, int b) { return a < b ? a : b; }
 __host__ __device__ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 __host__ __device__ constexpr int cclamp(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
+// a b + c with one rounding.  The smoother's column code writes its roundings out (contraction off): FP32 V
+// cycles are only linear to rounding, so that a product fused in one form of a kernel and not in another would
+// move a mixed-precision solution by up to 1e-8.
+__device__ __forceinline__ float fma1(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma1(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// c ? a : b of two values (a conditional on array elements would select their address and put the array in scratch)
+template <typename T>
+__device__ __forceinline__ T pick(bool c, T a, T b) { return c ? a : b; }
+
+// Barrier that orders the block's LDS accesses only.  __syncthreads() also waits for every HBM load and store in
+// flight; here loads issued early stay in flight across it, and nothing waits for stores that no thread of the
+// block reads back.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Kernels launched inside a device-driven Laplace solve take the solve's "done" flag and return at once
 // when it is set, so a fixed launch sequence (a captured graph) costs almost nothing after convergence.
 // nullptr: always run.
@@ -1615,6 +1634,7 @@ struct LvArgs {
     // first derivative (-cx1, 0, cx1), second derivative (cx2, cxc, cx2)
     int uni;
     T cx1, cx2, cxc, cy1, cy2, cyc;
+    const T *fac;           // records of the columns (LineRecord); nullptr: the sweep forms their line matrices
 };
 
 // Level coefficients as the column kernels read them: 3-point stencil rows sx(i), sy(j), sz(k) (first then
@@ -1723,26 +1743,39 @@ __device__ __forceinline__ void low_coefs(const CA &C, int i, int j, int k, T &s
 // rows with the neighbouring columns frozen (read through X(k, i, j)); the new column goes to out[0..NZ).
 // Couplings to same-colour columns (|di| or |dj| = 2, from the corner-shifted first pass on the sigma
 // ghost level) are left out, so that all columns of one colour can be relaxed at once.
-// Tridiagonal solve of a zebra column given its rows (lo, di, up, rh; e2 = third entry of the bottom row).
+// Tridiagonal solve of a zebra column given its rows (lo, di, up, rh; e2 = third entry of the bottom row): the
+// elimination factors f[k] (f[0]: of row 1 from the bottom row) and reciprocal pivots of the matrix (up[0] is
+// updated), then the substitution.  The surface row is the identity.
 template <typename T, int NZ>
-__device__ __forceinline__ void zebra_thomas(T (&lo)[NZ], T (&di)[NZ], T (&up)[NZ], T (&rh)[NZ], T e2, T *out) {
-    {   // eliminate the bottom row's third entry with row 1 (no-op when it is zero)
-        const T f = e2 != T(0) ? e2 / up[1] : T(0);
-        di[0] -= f * lo[1]; up[0] -= f * di[1]; rh[0] -= f * rh[1];
-    }
-    T inv[NZ];   // reciprocal pivots: one division per level
+__device__ __forceinline__ void line_factor(T (&lo)[NZ], T (&di)[NZ], T (&up)[NZ], T e2, T (&f)[NZ], T (&inv)[NZ]) {
+#pragma clang fp contract(off)
+    f[0] = e2 != T(0) ? e2 / up[1] : T(0);   // no-op when the entry is zero
+    di[0] = fma1(-f[0], lo[1], di[0]); up[0] = fma1(-f[0], di[1], up[0]);
     inv[0] = T(1) / di[0];
 #pragma unroll
-    for (int k = 1; k < NZ; k++) {
-        const T f = lo[k] * inv[k - 1];
-        di[k] -= f * up[k - 1];
-        rh[k] -= f * rh[k - 1];
+    for (int k = 1; k < NZ - 1; k++) {
+        f[k] = lo[k] * inv[k - 1];
+        di[k] = fma1(-f[k], up[k - 1], di[k]);
         inv[k] = T(1) / di[k];
     }
-    T xn = rh[NZ - 1] * inv[NZ - 1];
-    out[NZ - 1] = xn;
+}
+template <typename T, int NZ>
+__device__ __forceinline__ void line_solve(const T (&f)[NZ], const T (&up)[NZ], const T (&inv)[NZ], T (&rh)[NZ], T (&x)[NZ]) {
+#pragma clang fp contract(off)
+    rh[0] = fma1(-f[0], rh[1], rh[0]);
 #pragma unroll
-    for (int k = NZ - 2; k >= 0; k--) { xn = (rh[k] - up[k] * xn) * inv[k]; out[k] = xn; }
+    for (int k = 1; k < NZ - 1; k++) rh[k] = fma1(-f[k], rh[k - 1], rh[k]);
+    x[NZ - 1] = rh[NZ - 1];
+#pragma unroll
+    for (int k = NZ - 2; k >= 0; k--) x[k] = fma1(-up[k], x[k + 1], rh[k]) * inv[k];
+}
+template <typename T, int NZ>
+__device__ __forceinline__ void zebra_thomas(T (&lo)[NZ], T (&di)[NZ], T (&up)[NZ], T (&rh)[NZ], T e2, T *out) {
+    T f[NZ], inv[NZ], x[NZ];
+    line_factor<T, NZ>(lo, di, up, e2, f, inv);
+    line_solve<T, NZ>(f, up, inv, rh, x);
+#pragma unroll
+    for (int k = 0; k < NZ; k++) out[k] = x[k];
 }
 
 // zebra_column for a column at least two columns away from every wall (2 <= i <= nxg-3, and the same in
@@ -1925,199 +1958,6 @@ __device__ __forceinline__ void zebra_column(const LvArgs<T> &L, const CA &C, in
     zebra_thomas<T, NZ>(lo, di, up, rh, e2, out);
 }
 
-// Row k of the zebra line system of column (i, j) (the same rows zebra_column assembles): lo, di, up on
-// levels k-1, k, k+1, the right-hand side with the neighbouring columns moved over, and for the bottom
-// ghost row (k = 0) its third entry e2 (level 2).  nz = column depth.
-template <typename T, class XA, class CA>
-__device__ __forceinline__ void zebra_row(const LvArgs<T> &L, const CA &C, int i, int j, int k, int nz, const XA &X, T bk,
-                                          T &lo, T &di, T &up, T &rh, T &e2) {
-    const int nxg = L.nxg, nyg = L.nyg;
-    const bool d3 = L.dim3;
-    lo = T(0); up = T(0); e2 = T(0);
-    if (k == nz - 1) { di = T(1); rh = bk; return; }
-    const int wsx = cclamp(i - 1, 0, nxg - 3), wsy = d3 ? cclamp(j - 1, 0, nyg - 3) : 0;
-    const T *SX1 = C.sx(i), *SX2 = SX1 + 3;
-    const T *SY1 = C.sy(j), *SY2 = SY1 + 3;
-    if (k == 0) {
-        const T *Sz = C.sz(1);
-        T s2, s3, s4, s5;
-        low_coefs<T>(C, i, j, 1, s2, s3, s4, s5);
-        const T hx = C.col(1, i, j), hy = d3 ? C.col(2, i, j) : T(0);
-        const T cz = s5 + hx * s2 + hy * s4;
-        T a1 = cz * Sz[1], off = T(0);
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            const bool self = wsx + m == i;
-            const T v = X(1, self ? i : wsx + m, j);
-            a1 += self ? hx * SX1[m] : T(0);
-            off += self ? T(0) : hx * SX1[m] * v;
-        }
-        if (d3) {
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                const bool self = wsy + m == j;
-                const T v = X(1, i, self ? j : wsy + m);
-                a1 += self ? hy * SY1[m] : T(0);
-                off += self ? T(0) : hy * SY1[m] * v;
-            }
-        }
-        di = cz * Sz[0]; up = a1; e2 = cz * Sz[2];
-        rh = bk - off;
-        return;
-    }
-    int shx = 0; if (wsx == 0) shx = 1; if (wsx + 2 == nxg - 1) shx = -1;
-    int shy = 0;
-    if (d3) { if (wsy == 0) shy = 1; if (wsy + 2 == nyg - 1) shy = -1; }
-    const T *Z1 = C.sz(k), *Z2 = Z1 + 3;
-    T s2, s3, s4, s5;
-    low_coefs<T>(C, i, j, k, s2, s3, s4, s5);
-    const T czz = s2 * s2 + s4 * s4 + s5 * s5;
-    T a[3];
-#pragma unroll
-    for (int m = 0; m < 3; m++) a[m] = s3 * Z1[m] + czz * Z2[m];
-    T off = T(0);
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        const bool self = wsx + m == i;
-        const T v = X(k, self ? i : wsx + m, j);
-        a[1] += self ? SX2[m] : T(0);
-        off += self ? T(0) : SX2[m] * v;
-    }
-#pragma unroll
-    for (int mz = 0; mz < 3; mz++) {
-        const int kk = k - 1 + mz;
-        const int sh = (kk == 0) ? shx : 0;
-        const T *S1 = (kk == 0) ? C.sx(i - shx) : SX1;
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            const T w = T(2) * s2 * Z1[mz] * S1[m];
-            const int ii = wsx + sh + m;
-            const bool self = ii == i, skip = self || ii - i == 2 || i - ii == 2;
-            const T v = X(kk, skip ? i : ii, j);
-            a[mz] += self ? w : T(0);
-            off += skip ? T(0) : w * v;
-        }
-    }
-    if (d3) {
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            const bool self = wsy + m == j;
-            const T v = X(k, i, self ? j : wsy + m);
-            a[1] += self ? SY2[m] : T(0);
-            off += self ? T(0) : SY2[m] * v;
-        }
-#pragma unroll
-        for (int mz = 0; mz < 3; mz++) {
-            const int kk = k - 1 + mz;
-            const int sh = (kk == 0) ? shy : 0;
-            const T *S1 = (kk == 0) ? C.sy(j - shy) : SY1;
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                const T w = T(2) * s4 * Z1[mz] * S1[m];
-                const int jj = wsy + sh + m;
-                const bool self = jj == j, skip = self || jj - j == 2 || j - jj == 2;
-                const T v = X(kk, i, skip ? j : jj);
-                a[mz] += self ? w : T(0);
-                off += skip ? T(0) : w * v;
-            }
-        }
-    }
-    lo = a[0]; di = a[1]; up = a[2];
-    rh = bk - off;
-}
-
-// zebra_row for a column at least two columns from every wall (no clamped or shifted windows): the
-// column's level-0 value is at c in LDS, x- and y-neighbours at fixed offsets SXS and SYS.  Same terms in
-// the same order as zebra_row.
-template <typename T, int SXS, int SYS, class CA>
-__device__ __forceinline__ void zebra_row_interior(const CA &C, bool d3, int i, int j, int k, int nz, const T *c, T bk,
-                                                   T &lo, T &di, T &up, T &rh, T &e2) {
-    lo = T(0); up = T(0); e2 = T(0);
-    if (k == nz - 1) { di = T(1); rh = bk; return; }
-    const T *SX1 = C.sx(i), *SX2 = SX1 + 3;
-    const T *SY1 = C.sy(j), *SY2 = SY1 + 3;
-    const T *xm = c - SXS, *xp = c + SXS, *ym = c - SYS, *yp = c + SYS;
-    if (k == 0) {
-        const T *Sz = C.sz(1);
-        T s2, s3, s4, s5;
-        low_coefs<T>(C, i, j, 1, s2, s3, s4, s5);
-        const T hx = C.col(1, i, j), hy = d3 ? C.col(2, i, j) : T(0);
-        const T cz = s5 + hx * s2 + hy * s4;
-        T a1 = cz * Sz[1], off = T(0);
-        off += hx * SX1[0] * xm[1];
-        a1 += hx * SX1[1];
-        off += hx * SX1[2] * xp[1];
-        if (d3) {
-            off += hy * SY1[0] * ym[1];
-            a1 += hy * SY1[1];
-            off += hy * SY1[2] * yp[1];
-        }
-        di = cz * Sz[0]; up = a1; e2 = cz * Sz[2];
-        rh = bk - off;
-        return;
-    }
-    const T *Z1 = C.sz(k), *Z2 = Z1 + 3;
-    T s2, s3, s4, s5;
-    low_coefs<T>(C, i, j, k, s2, s3, s4, s5);
-    const T czz = s2 * s2 + s4 * s4 + s5 * s5;
-    T a[3];
-#pragma unroll
-    for (int m = 0; m < 3; m++) a[m] = s3 * Z1[m] + czz * Z2[m];
-    T off = T(0);
-    off += SX2[0] * xm[k];
-    a[1] += SX2[1];
-    off += SX2[2] * xp[k];
-#pragma unroll
-    for (int mz = 0; mz < 3; mz++) {
-        const int kk = k - 1 + mz;
-        off += T(2) * s2 * Z1[mz] * SX1[0] * xm[kk];
-        a[mz] += T(2) * s2 * Z1[mz] * SX1[1];
-        off += T(2) * s2 * Z1[mz] * SX1[2] * xp[kk];
-    }
-    if (d3) {
-        off += SY2[0] * ym[k];
-        a[1] += SY2[1];
-        off += SY2[2] * yp[k];
-#pragma unroll
-        for (int mz = 0; mz < 3; mz++) {
-            const int kk = k - 1 + mz;
-            off += T(2) * s4 * Z1[mz] * SY1[0] * ym[kk];
-            a[mz] += T(2) * s4 * Z1[mz] * SY1[1];
-            off += T(2) * s4 * Z1[mz] * SY1[2] * yp[kk];
-        }
-    }
-    lo = a[0]; di = a[1]; up = a[2];
-    rh = bk - off;
-}
-
-// Row k (1 <= k <= nz - 2) of an interior column (2 <= i <= nxg - 3, 2 <= j <= nyg - 3) on a uniform
-// horizontal grid: zebra_row_interior with the level's constant centred stencils, so each mixed-derivative
-// coupling is 2 s2 cx1 sum_m Z1[m] (x[i+1] - x[i-1]) on the three sigma levels around k (the centre
-// weight of the first derivative is zero).  c points at the column's level 0 in LDS.
-template <typename T, int SXS, int SYS, class CA>
-__device__ __forceinline__ void zebra_row_uniform(const LvArgs<T> &L, const CA &C, bool d3, int i, int j, int k, const T *c,
-                                                  T bk, T &lo, T &di, T &up, T &rh) {
-    const T *Z1 = C.sz(k), *Z2 = Z1 + 3;
-    const T om = T(1) - C.zs(k);
-    const T s2 = om * C.col(3, i, j), s3 = om * C.col(5, i, j), s5 = C.col(0, i, j);
-    const T *xm = c - SXS, *xp = c + SXS;
-    const T gx = (Z1[0] * (xp[k - 1] - xm[k - 1]) + Z1[1] * (xp[k] - xm[k])) + Z1[2] * (xp[k + 1] - xm[k + 1]);
-    T off = L.cx2 * (xm[k] + xp[k]) + (T(2) * L.cx1) * s2 * gx;
-    T czz = s2 * s2 + s5 * s5, dc = L.cxc;
-    if (d3) {
-        const T s4 = om * C.col(4, i, j);
-        const T *ym = c - SYS, *yp = c + SYS;
-        const T gy = (Z1[0] * (yp[k - 1] - ym[k - 1]) + Z1[1] * (yp[k] - ym[k])) + Z1[2] * (yp[k + 1] - ym[k + 1]);
-        off += L.cy2 * (ym[k] + yp[k]) + (T(2) * L.cy1) * s4 * gy;
-        czz += s4 * s4;
-        dc += L.cyc;
-    }
-    lo = s3 * Z1[0] + czz * Z2[0];
-    di = (s3 * Z1[1] + czz * Z2[1]) + dc;
-    up = s3 * Z1[2] + czz * Z2[2];
-    rh = bk - off;
-}
-
 // Residual o = b - L x of column (i, j) of a level (all row kinds: interior, bottom ghost, surface,
 // wall ghost columns, corners), x read through X(k, i, j).
 template <typename T, int NZ, class XA, class CA>
@@ -2287,266 +2127,928 @@ __global__ __launch_bounds__(128) void k_mg_zebra_t(LvArgs<T> L, int colour, T *
     }
 }
 
-// One full zebra sweep (red columns, then black columns) in one launch, out of place (xin -> xout: a
-// block's staged neighbours must not change while other blocks write their results).  A block owns a
-// TX x TY tile of interior columns and stages it with a two-column halo.  Each half-sweep runs in two
-// phases: the rows of all columns of the colour are assembled in parallel (one thread per (column,
-// level) row, into LDS), then one thread per column runs the tridiagonal solve.  The red half-sweep
-// covers the tile and its one-column ring (a red column reads only black neighbours, which do not change
-// in the red half-sweep, so the ring gets exactly the values the owning blocks compute); the black
-// half-sweep covers the tile and reads those red values.  The wall ghost pass before the sweep is done
-// on the staged window and the one after it for the ghost points next to the tile, so one launch does
-// (ghost pass, red, black, ghost pass) with x read once and written once.
-//
-// MODE 1: the first sweep of a preconditioner application, from x = 0 with the right-hand side given as
-// the FP64 residual r0: x is not read, b = (T) r0 is staged from r0 and written to bout for the points the
-// tile owns (its columns and the ghost points the post-sweep ghost pass gives it), which together cover
-// the level; this replaces the separate pass b = (T) r, x = 0 before the V cycle.
-// MODE 2: the last sweep of an application: the owned points of the result go to uout as FP64 (the
-// preconditioner's output) instead of to xout; this replaces the separate output conversion.
+// Columns between HBM and registers, two values per load or store where every column starts on an even element.
+template <typename S>
+struct alignas(2 * sizeof(S)) ColPair { S a, b; };
+template <int NZ, typename S, typename T>
+__device__ __forceinline__ void load_column(const S *__restrict__ p, T (&v)[NZ]) {
+    if constexpr (NZ % 2 == 0) {
+        const ColPair<S> *q = reinterpret_cast<const ColPair<S> *>(p);
+#pragma unroll
+        for (int k = 0; k < NZ / 2; k++) { const ColPair<S> w = q[k]; v[2 * k] = (T)w.a; v[2 * k + 1] = (T)w.b; }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NZ; k++) v[k] = (T)p[k];
+    }
+}
+// N values (a multiple of 16 bytes) from a 16-byte aligned address.
+template <int N, typename T>
+__device__ __forceinline__ void load_record(const T *__restrict__ p, T (&v)[N]) {
+    constexpr int W = 16 / sizeof(T);
+    struct alignas(16) Quad { T e[W]; };
+    static_assert(N % W == 0, "whole 16-byte loads");
+#pragma unroll
+    for (int q = 0; q < N / W; q++) {
+        const Quad w = reinterpret_cast<const Quad *>(p)[q];
+#pragma unroll
+        for (int e = 0; e < W; e++) v[q * W + e] = w.e[e];
+    }
+}
+template <int NZ, typename T, typename O>
+__device__ __forceinline__ void store_column(O *__restrict__ p, const T (&v)[NZ]) {
+    if constexpr (NZ % 2 == 0) {
+        ColPair<O> *q = reinterpret_cast<ColPair<O> *>(p);
+#pragma unroll
+        for (int k = 0; k < NZ / 2; k++) q[k] = ColPair<O>{(O)v[2 * k], (O)v[2 * k + 1]};
+    } else {
+#pragma unroll
+        for (int k = 0; k < NZ; k++) p[k] = (O)v[k];
+    }
+}
+
+// Line system of an interior column (two columns or more from every wall) on a uniform horizontal grid: the
+// matrix rows, and the right-hand side with the neighbours' terms.  Each mixed-derivative coupling is
+// 2 s2 cx1 sum_m Z1[m] (x[i+1] - x[i-1]) on the three sigma levels around k (the centre weight of the first
+// derivative is zero), and the differences and sums of the two neighbours are formed once per level, not once per
+// row that uses them.  c: the column's level 0 in LDS, neighbours at +- SXS and +- SYS; cp: the column's six
+// planes; S1x, S1y: its first-derivative rows (bottom row).
+template <typename T, int NZ, bool D3>
+__device__ __forceinline__ void line_matrix_uniform(const LvArgs<T> &L, const T (&cp)[6], const T (&S1x)[3], const T (&S1y)[3],
+                                                    T (&lo)[NZ], T (&di)[NZ], T (&up)[NZ], T &e2) {
+#pragma clang fp contract(off)
+    {
+        const T *Sz = L.sz + 6;
+        const T om = T(1) - L.zs[1];
+        const T s2 = om * cp[3], s4 = om * cp[4], s5 = cp[0];
+        const T hx = cp[1], hy = D3 ? cp[2] : T(0);
+        const T cz = fma1(hy, s4, fma1(hx, s2, s5));
+        T a1 = fma1(cz, Sz[1], hx * S1x[1]);
+        if constexpr (D3) a1 = fma1(hy, S1y[1], a1);
+        lo[0] = T(0); di[0] = cz * Sz[0]; up[0] = a1; e2 = cz * Sz[2];
+    }
+#pragma unroll
+    for (int k = 1; k < NZ - 1; k++) {
+        const T *Z1 = L.sz + k * 6, *Z2 = Z1 + 3;
+        const T om = T(1) - L.zs[k];
+        const T s2 = om * cp[3], s3 = om * cp[5], s5 = cp[0];
+        T czz = fma1(s2, s2, s5 * s5), dc = L.cxc;
+        if constexpr (D3) {
+            const T s4 = om * cp[4];
+            czz = fma1(s4, s4, czz);
+            dc += L.cyc;
+        }
+        lo[k] = fma1(s3, Z1[0], czz * Z2[0]);
+        di[k] = fma1(s3, Z1[1], czz * Z2[1]) + dc;
+        up[k] = fma1(s3, Z1[2], czz * Z2[2]);
+    }
+}
+// bw: the bottom row's weights of the west, east, south and north neighbour; c3, c4: h_x / h, h_y / h.
+template <typename T, int NZ, bool D3, int SXS, int SYS>
+__device__ __forceinline__ void line_rhs_uniform(const LvArgs<T> &L, T c3, T c4, const T (&bw)[4], const T *c, const T (&b)[NZ], T (&rh)[NZ]) {
+#pragma clang fp contract(off)
+    T sx[NZ], gx[NZ], sy[NZ], gy[NZ];   // sums and differences of the x- and y-neighbours
+#pragma unroll
+    for (int k = 0; k < NZ; k++) {
+        const T xm = c[k - SXS], xp = c[k + SXS];
+        sx[k] = xm + xp; gx[k] = xp - xm;
+        T ym = T(0), yp = T(0);
+        if constexpr (D3) {
+            ym = c[k - SYS]; yp = c[k + SYS];
+            sy[k] = ym + yp; gy[k] = yp - ym;
+        }
+        if (k == 1) {
+            T off = fma1(bw[1], xp, bw[0] * xm);
+            if constexpr (D3) {
+                off = fma1(bw[2], ym, off);
+                off = fma1(bw[3], yp, off);
+            }
+            rh[0] = b[0] - off;
+        }
+    }
+#pragma unroll
+    for (int k = 1; k < NZ - 1; k++) {
+        const T *Z1 = L.sz + k * 6;
+        const T om = T(1) - L.zs[k];
+        const T s2 = om * c3;
+        const T g = fma1(Z1[2], gx[k + 1], fma1(Z1[0], gx[k - 1], Z1[1] * gx[k]));
+        T off = fma1(L.cx2, sx[k], ((T(2) * L.cx1) * s2) * g);
+        if constexpr (D3) {
+            const T s4 = om * c4;
+            const T q = fma1(Z1[2], gy[k + 1], fma1(Z1[0], gy[k - 1], Z1[1] * gy[k]));
+            off += fma1(L.cy2, sy[k], ((T(2) * L.cy1) * s4) * q);
+        }
+        rh[k] = b[k] - off;
+    }
+    rh[NZ - 1] = b[NZ - 1];
+}
+
+// Rows of a column's 3-point x and y windows (centred: beside a wall the ghost column is the outer neighbour), and
+// the first row of the wall node beside it (of the high wall where there is none).
+template <typename T, bool D3>
+struct LineRows {
+    T X1[3], X2[3], XW[3], Y1[3], Y2[3], YW[3];
+    __device__ __forceinline__ void load(const LvArgs<T> &L, int i, int j) {
+        const int iw = i == 1 ? 0 : L.nxg - 1, jw = j == 1 ? 0 : L.nyg - 1;
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            X1[m] = L.sx[i * 6 + m]; X2[m] = L.sx[i * 6 + 3 + m]; XW[m] = L.sx[iw * 6 + m];
+            if constexpr (D3) { Y1[m] = L.sy[j * 6 + m]; Y2[m] = L.sy[j * 6 + 3 + m]; YW[m] = L.sy[jw * 6 + m]; }
+        }
+    }
+    // Weights of the mixed derivative on the sigma ghost level: beside a wall its window is shifted one column
+    // inwards and takes the wall node's row (ConstructTableCrossDerivatives.f90:173-186); the coupling to the
+    // column two away is left out (all columns of a colour are relaxed at once).
+    __device__ __forceinline__ static void ghost_level(const T (&S)[3], const T (&W)[3], int i, int n, T (&g)[3]) {
+        const bool lo = i == 1, hi = !lo && i == n - 2;
+        g[0] = pick(lo, T(0), pick(hi, W[1], S[0]));
+        g[1] = pick(lo, W[0], pick(hi, W[2], S[1]));
+        g[2] = pick(lo, W[1], pick(hi, T(0), S[2]));
+    }
+};
+// Line system of any column from its rows: columns next to a wall, and every column of a non-uniform grid.
+template <typename T, int NZ, bool D3>
+__device__ __forceinline__ void line_matrix_general(const LvArgs<T> &L, int i, int j, const LineRows<T, D3> &R, const T (&cp)[6], T (&lo)[NZ],
+                                                    T (&di)[NZ], T (&up)[NZ], T &e2) {
+#pragma clang fp contract(off)
+    T XG[3], YG[3];
+    R.ghost_level(R.X1, R.XW, i, L.nxg, XG);
+    if constexpr (D3) R.ghost_level(R.Y1, R.YW, j, L.nyg, YG);
+    {
+        const T *Sz = L.sz + 6;
+        const T om = T(1) - L.zs[1];
+        const T s2 = om * cp[3], s4 = om * cp[4], s5 = cp[0];
+        const T hx = cp[1], hy = D3 ? cp[2] : T(0);
+        const T cz = fma1(hy, s4, fma1(hx, s2, s5));
+        T a1 = cz * Sz[1] + hx * R.X1[1];
+        if constexpr (D3) a1 = a1 + hy * R.Y1[1];
+        lo[0] = T(0); di[0] = cz * Sz[0]; up[0] = a1; e2 = cz * Sz[2];
+    }
+#pragma unroll
+    for (int k = 1; k < NZ - 1; k++) {
+        const T *Z1 = L.sz + k * 6, *Z2 = Z1 + 3;
+        const T om = T(1) - L.zs[k];
+        const T s2 = om * cp[3], s4 = om * cp[4], s3 = om * cp[5], s5 = cp[0];
+        const T czz = fma1(s5, s5, fma1(s2, s2, s4 * s4));
+        T a[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) a[m] = fma1(s3, Z1[m], czz * Z2[m]);
+        a[1] += R.X2[1];
+#pragma unroll
+        for (int m = 0; m < 3; m++) a[m] = a[m] + (T(2) * s2 * Z1[m]) * (k - 1 + m == 0 ? XG[1] : R.X1[1]);
+        if constexpr (D3) {
+            a[1] += R.Y2[1];
+#pragma unroll
+            for (int m = 0; m < 3; m++) a[m] = a[m] + (T(2) * s4 * Z1[m]) * (k - 1 + m == 0 ? YG[1] : R.Y1[1]);
+        }
+        lo[k] = a[0]; di[k] = a[1]; up[k] = a[2];
+    }
+}
+template <typename T, int NZ, bool D3, int SXS, int SYS>
+__device__ __forceinline__ void line_rhs_general(const LvArgs<T> &L, int i, int j, const LineRows<T, D3> &R, T c3, T c4, const T (&bw)[4],
+                                                 const T *c, const T (&b)[NZ], T (&rh)[NZ]) {
+#pragma clang fp contract(off)
+    T XG[3], YG[3], xm[NZ], xp[NZ], ym[NZ], yp[NZ];
+    R.ghost_level(R.X1, R.XW, i, L.nxg, XG);
+    if constexpr (D3) R.ghost_level(R.Y1, R.YW, j, L.nyg, YG);
+#pragma unroll
+    for (int k = 0; k < NZ; k++) {
+        xm[k] = c[k - SXS]; xp[k] = c[k + SXS];
+        if constexpr (D3) { ym[k] = c[k - SYS]; yp[k] = c[k + SYS]; }
+    }
+    {
+        T off = bw[0] * xm[1];
+        off = off + bw[1] * xp[1];
+        if constexpr (D3) {
+            off = off + bw[2] * ym[1];
+            off = off + bw[3] * yp[1];
+        }
+        rh[0] = b[0] - off;
+    }
+#pragma unroll
+    for (int k = 1; k < NZ - 1; k++) {
+        const T *Z1 = L.sz + k * 6;
+        const T om = T(1) - L.zs[k];
+        const T s2 = om * c3, s4 = om * c4;
+        T off = R.X2[0] * xm[k];
+        off = off + R.X2[2] * xp[k];
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            const int kk = k - 1 + m;
+            const T w = T(2) * s2 * Z1[m];
+            off = off + (w * (kk == 0 ? XG[0] : R.X1[0])) * xm[kk];
+            off = off + (w * (kk == 0 ? XG[2] : R.X1[2])) * xp[kk];
+        }
+        if constexpr (D3) {
+            off = off + R.Y2[0] * ym[k];
+            off = off + R.Y2[2] * yp[k];
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                const int kk = k - 1 + m;
+                const T w = T(2) * s4 * Z1[m];
+                off = off + (w * (kk == 0 ? YG[0] : R.Y1[0])) * ym[kk];
+                off = off + (w * (kk == 0 ? YG[2] : R.Y1[2])) * yp[kk];
+            }
+        }
+        rh[k] = b[k] - off;
+    }
+    rh[NZ - 1] = b[NZ - 1];
+}
+
+// line_rhs_general by two lanes per column, 32 apart: `hi` of them forms the upper half of the rows (half the time of
+// the longest path of a small level's sweep; the rows of a wall column are about three times an interior
+// column's).  The lower lanes receive all rows.
+template <typename T, int NZ, bool D3, int SXS, int SYS>
+__device__ __forceinline__ void line_rhs_pair(const LvArgs<T> &L, int i, int j, bool hi, const LineRows<T, D3> &R, T c3, T c4, const T (&bw)[4],
+                                              const T *c, const T (&b)[NZ], T (&rh)[NZ]) {
+#pragma clang fp contract(off)
+    constexpr int HALF = (NZ - 1) / 2;   // of the NZ - 2 rows
+    T XG[3], YG[3], xm[HALF + 2], xp[HALF + 2], ym[HALF + 2], yp[HALF + 2], r[HALF];
+    R.ghost_level(R.X1, R.XW, i, L.nxg, XG);
+    if constexpr (D3) R.ghost_level(R.Y1, R.YW, j, L.nyg, YG);
+#pragma unroll
+    for (int m = 0; m < 3; m++) {   // the upper half has no sigma ghost level among its rows
+        XG[m] = pick(hi, R.X1[m], XG[m]);
+        if constexpr (D3) YG[m] = pick(hi, R.Y1[m], YG[m]);
+    }
+#pragma unroll
+    for (int q = 0; q < HALF + 2; q++) {
+        const int k = hi ? cmin(HALF + q, NZ - 1) : q;
+        xm[q] = c[k - SXS]; xp[q] = c[k + SXS];
+        if constexpr (D3) { ym[q] = c[k - SYS]; yp[q] = c[k + SYS]; }
+    }
+    {   // bottom row (used by the lower lanes)
+        T off = bw[0] * xm[1];
+        off = off + bw[1] * xp[1];
+        if constexpr (D3) {
+            off = off + bw[2] * ym[1];
+            off = off + bw[3] * yp[1];
+        }
+        rh[0] = b[0] - off;
+    }
+#pragma unroll
+    for (int q = 0; q < HALF; q++) {
+        constexpr int TOP = NZ - 2;
+        const int kl = 1 + q, kh = cmin(1 + q + HALF, TOP);
+        const T om = T(1) - pick(hi, L.zs[kh], L.zs[kl]);
+        const T s2 = om * c3, s4 = om * c4;
+        T Z1[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) Z1[m] = pick(hi, L.sz[kh * 6 + m], L.sz[kl * 6 + m]);
+        T off = R.X2[0] * xm[q + 1];
+        off = off + R.X2[2] * xp[q + 1];
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            const T w = T(2) * s2 * Z1[m];
+            off = off + (w * (q + m == 0 ? XG[0] : R.X1[0])) * xm[q + m];
+            off = off + (w * (q + m == 0 ? XG[2] : R.X1[2])) * xp[q + m];
+        }
+        if constexpr (D3) {
+            off = off + R.Y2[0] * ym[q + 1];
+            off = off + R.Y2[2] * yp[q + 1];
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                const T w = T(2) * s4 * Z1[m];
+                off = off + (w * (q + m == 0 ? YG[0] : R.Y1[0])) * ym[q + m];
+                off = off + (w * (q + m == 0 ? YG[2] : R.Y1[2])) * yp[q + m];
+            }
+        }
+        r[q] = pick(hi, b[kh], b[kl]) - off;
+    }
+#pragma unroll
+    for (int q = 0; q < HALF; q++) {
+        const T up = __shfl_xor(r[q], 32);
+        rh[1 + q] = r[q];
+        if (1 + q + HALF <= NZ - 2) rh[1 + q + HALF] = up;
+    }
+    rh[NZ - 1] = b[NZ - 1];
+}
+
+// What the sweeps of a level need of a column that depends on the bottom and the grid only (LvArgs::fac), one record
+// per column: the factors of its line matrix f[0 .. NZ-2], up[0 .. NZ-2], inv[0 .. NZ-2], then h_x / h, h_y / h and
+// the bottom row's weights of the four neighbours.  A colour's records are contiguous, so that the lanes of a wave
+// read neighbouring ones with 16-byte loads (as 3 NZ planes with coalesced 4-byte loads a 257^2 sweep took
+// 15.2 us, and 4 us of a small level's sweep were address arithmetic and load issue).
+template <typename T, int NZ>
+struct LineRecord {
+    static constexpr int W = 16 / sizeof(T), N = (3 * NZ - 3 + 6 + W - 1) / W * W;
+    static constexpr int C3 = 3 * NZ - 3, C4 = C3 + 1, BW = C3 + 2;
+    __host__ __device__ static size_t index(int nxg, int nyg, int i, int j) {   // of column (i, j), in records
+        return ((size_t)((i + j) & 1) * nyg + j) * ((nxg + 1) / 2) + (i >> 1);
+    }
+    __host__ __device__ static size_t count(int nxg, int nyg) { return (size_t)2 * nyg * ((nxg + 1) / 2); }
+};
+template <typename T, int NZ, bool D3>
+__global__ __launch_bounds__(256) void k_mg_factor(LvArgs<T> L, T *__restrict__ fac) {
+#pragma clang fp contract(off)
+    using Rec = LineRecord<T, NZ>;
+    const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (p >= L.nxy) return;
+    const int j = p / L.nxg, i = p - j * L.nxg;
+    if (i < 1 || i > L.nxg - 2 || (D3 && (j < 1 || j > L.nyg - 2))) return;
+    T cp[6], lo[NZ], di[NZ], up[NZ], f[NZ], inv[NZ], e2;
+#pragma unroll
+    for (int q = 0; q < 6; q++) cp[q] = L.col[(size_t)q * L.nxy + p];
+    LineRows<T, D3> R;
+    R.load(L, i, j);
+    const bool edge = i < 2 || i > L.nxg - 3 || (D3 && (j < 2 || j > L.nyg - 3));
+    if (edge || !L.uni) line_matrix_general<T, NZ, D3>(L, i, j, R, cp, lo, di, up, e2);
+    else line_matrix_uniform<T, NZ, D3>(L, cp, R.X1, R.Y1, lo, di, up, e2);
+    line_factor<T, NZ>(lo, di, up, e2, f, inv);
+    T *d = fac + Rec::index(L.nxg, L.nyg, i, j) * Rec::N;
+#pragma unroll
+    for (int k = 0; k < NZ - 1; k++) { d[k] = f[k]; d[NZ - 1 + k] = up[k]; d[2 * NZ - 2 + k] = inv[k]; }
+    d[Rec::C3] = cp[3]; d[Rec::C4] = cp[4];
+    d[Rec::BW] = cp[1] * R.X1[0]; d[Rec::BW + 1] = cp[1] * R.X1[2];
+    d[Rec::BW + 2] = D3 ? cp[2] * R.Y1[0] : T(0); d[Rec::BW + 3] = D3 ? cp[2] * R.Y1[2] : T(0);
+}
+
 // Prolongation fused into the first post-smoothing sweep of a level with interpolation tables
 // (k_mg_prolong_tab's tables and arithmetic; the coarse level is coarsened in x and y, not in sigma).
 template <typename T>
 struct ProArgs {
     const T *ec;              // coarse correction
-    const int2 *pxi, *pyi;    // per fine column / row: left and right coarse index (-1: none)
     const T *pxw, *pyw;       // per fine column / row: left weight, right weight, 1 / sum
     int nxgc;                 // coarse row length
-};
-// Coarse window of a fine window WX x WY: fine interior column i >= 1 interpolates from coarse columns
-// 1 + (i - 1) / 2 and 1 + i / 2.
-template <int WX, int WY>
-struct ProWindow {
-    static constexpr int CWX = WX / 2 + 2, CWY = WY / 2 + 2;
+    int ghosts;               // 0: nothing reads the wall ghost points of the sweep's result before they are set anew
 };
 
-template <typename T, int NZ, int TX, int TY, int NT, int MODE = 0>
-__global__ __launch_bounds__(NT) void k_mg_zebra_rb(LvArgs<T> L, const T *__restrict__ xin, T *__restrict__ xout, const T *__restrict__ b,
-                                                    const double *__restrict__ r0, T *__restrict__ bout, double *__restrict__ uout,
-                                                    ProArgs<T> P) {
-    // MODE 1: x = 0, b from r0; MODE 2: result to uout in FP64; MODE 3: the coarse correction P is added to
-    // x first (prolongation); MODE 4: MODE 3 with the result to uout
-    constexpr bool ZX = MODE == 1, ZO = MODE == 2 || MODE == 4, PRO = MODE == 3 || MODE == 4;
-    if (!L.spec && solve_done(L.skip)) return;
-    constexpr int H = 2, WX = TX + 2 * H, WY = TY + 2 * H, NZP = NZ | 1;
-    constexpr int PR = (TX + 2) / 2, NS = PR * (TY + 2);   // red slots: ring-extended tile
-    constexpr int CWX = ProWindow<WX, WY>::CWX, CWY = ProWindow<WX, WY>::CWY;
+// First interior column (from 1) of tile t of nt over n columns: tiles of equal width but for one column.  The
+// grids have 2^p m + 1 columns, so tiles of a fixed width of 2^q leave a last one with a single column; here every
+// tile has two or more, as its wall ghost values need.
+__host__ __device__ inline int tile_begin(int n, int t, int nt) { return 1 + (int)((long)n * t / nt); }
+
+// Tile of the zebra sweep: at most TX x TY interior columns (TY = 1: x-z problems), one thread per column of a colour
+// of the tile and its one-column ring, and one more wave for the columns next to a wall.
+template <int NZ, int TX, int TY>
+struct SweepTile {
+    static constexpr bool D3 = TY > 1;
+    static constexpr int H = 2, WX = TX + 2 * H, WY = D3 ? TY + 2 * H : 1, NZP = NZ | 1;
+    static constexpr int RX = TX / 2 + 1, RY = D3 ? TY + 2 : 1;     // columns of a colour per row, rows (with the ring)
+    static constexpr int NR = (RX * RY + 63) / 64 * 64, NT = NR + 64;
+    static constexpr int BX = D3 ? TX / 2 + 1 : 0, BY = D3 ? TY / 2 + 1 : 1;   // wall columns of a colour per side
+    static constexpr int GX = D3 ? TX + 2 : 0, GY = D3 ? TY + 2 : 1;           // wall ghost columns beside the ring per side
+    static_assert(TX % 2 == 0 && (TY % 2 == 0 || TY == 1), "even tiles");
+    static_assert(2 * (BX + BY) <= 64, "wall columns of a colour fit one wave");
+    static_assert(2 * (GX + GY) <= NT, "one thread per wall ghost column");
+    static_assert((WX / 2) * WY <= NT, "one thread per window column of a colour");
+};
+
+// One full zebra sweep (red columns, then black columns) in one launch, out of place (xin -> xout: a block's
+// staged neighbours must not change while other blocks write their results).  A block owns a tile of
+// at most TX x TY interior columns.  The red half-sweep covers the tile and its one-column ring (a red column reads only black
+// neighbours, which do not change in the red half-sweep, so the ring gets exactly the values the owning blocks
+// compute), the black half-sweep the tile.  The wall ghost pass before the sweep is done on the staged window
+// and the one after it for the ghost points next to the tile, so one launch does (ghost pass, red, black, ghost
+// pass) with x read once and written once.
+//
+// One thread per column: right-hand side, coefficients and the tridiagonal system live in its registers, and
+// LDS holds only what columns read of each other.  A red column reads black ones and no column reads its own
+// old value, so only black columns are staged (and, in tiles at a wall, red ones for the ghost pass).
+// Columns next to a wall take a longer path; they have a wave of their own, so that no other wave runs both.
+//
+// MODE 1: the first sweep of a preconditioner application, from x = 0 with the right-hand side given as
+// the FP64 residual r0: x is not read, b = (T) r0 is written to bout (unless NULL) for the points the tile owns (its
+// columns and the ghost points the post-sweep ghost pass gives it), which together cover the level.
+// MODE 2: the last sweep of an application: the owned points of the result go to uout as FP64 instead of to
+// xout.  MODE 3: the coarse correction P is added to x first (prolongation); MODE 4: MODE 3 with the result to
+// uout.  MODE 5: the first sweep of a coarse level: x = 0 (not read) and b is zero on the wall ghost columns, as
+// the restrictions leave it, so that the ghost values are zero too and the red columns' rows are b alone.
+// For levels whose columns' records are kept (L.fac): small levels, where a sweep is a chain of latencies, so every
+// load is issued before the first wait and the red columns' loads before the black ones'.  What such a launch takes
+// hardly depends on the level's size (FP32 / FP64, 33^2 to 129^2 columns of 10 values): from zero 5.8 / 6.8 us, with
+// the correction 7.1-9.4 / 9.6-11.6 us, where a row of the line systems per thread, the systems passed through LDS and
+// the Thomas solves on a few threads took 12.5 / 15-17 and 13.3-14.4 / 16-19 us.
+template <typename T, int NZ, int TX, int TY, int MODE>
+__global__ __launch_bounds__((SweepTile<NZ, TX, TY>::NT)) void k_mg_sweep(LvArgs<T> L, const T *__restrict__ xin, T *__restrict__ xout,
+                                                                          const T *__restrict__ b, const double *__restrict__ r0,
+                                                                          T *__restrict__ bout, double *__restrict__ uout, ProArgs<T> P) {
+#pragma clang fp contract(off)
+    constexpr bool ZX = MODE == 1, ZB = MODE == 5, ZO = MODE == 2 || MODE == 4, PRO = MODE == 3 || MODE == 4;
+    using G = SweepTile<NZ, TX, TY>;
+    constexpr bool D3 = G::D3, PAIR = 2 * (G::BX + G::BY) <= 32;   // PAIR: two lanes per wall column
+    constexpr int H = G::H, WX = G::WX, WY = G::WY, NZP = G::NZP, SXS = NZP, SYS = WX * NZP;
+    using Rec = LineRecord<T, NZ>;
     __shared__ T sX[WX * WY * NZP];
-    __shared__ T sC[CoefLds<WX, WY, NZ>::TOTAL];
-    __shared__ T sR[4 * NS * NZ];
-    __shared__ T sE[NS];
-    __shared__ T sB[(TX + 2) * (TY + 2) * NZ];   // right-hand sides of the ring-extended tile
-    __shared__ T sP[PRO ? CWX * CWY * NZP : 1];              // coarse correction window
-    __shared__ int2 sPi[PRO ? WX + WY : 1];                  // interpolation tables of the window's columns, rows
-    __shared__ T sPw[PRO ? 3 * (WX + WY) : 1];
-    const int nxg = L.nxg, nyg = L.nyg, d3 = L.dim3;
-    // tiles of TX x TY interior columns; when a direction's count leaves a one-column remainder the first
-    // tile is one column short instead, so every tile next to a wall has the two columns its ghost
-    // values are computed from
-    const int nxi = nxg - 2 * L.gx, nyi = d3 ? nyg - 2 * L.gy : 1;
-    const int offx = (nxi % TX == 1) ? 1 : 0, offy = (d3 && nyi % TY == 1) ? 1 : 0;
-    // (tiles in launch order: the XCD-aware order of k_mg_residual_restrict halves the sweep's HBM fetch at
-    // 513^2, 55 -> 29 MB, but the sweep then takes 49.4 instead of 46.0 us)
-    const int i0 = L.gx + cmax(0, (int)blockIdx.x * TX - offx), ie = L.gx + cmin(nxi, ((int)blockIdx.x + 1) * TX - offx);
-    const int j0 = d3 ? L.gy + cmax(0, (int)blockIdx.y * TY - offy) : 0;
-    const int je = d3 ? L.gy + cmin(nyi, ((int)blockIdx.y + 1) * TY - offy) : 1;
-    const int lox = cmax(i0 - H, 0), loy = d3 ? cmax(j0 - H, 0) : 0;
-    const int wcols = cmin(ie + H, nxg) - lox, wrows = d3 ? cmin(je + H, nyg) - loy : 1;
-    // b over the ring-extended tile [i0-1, ie] x [j0-1, je] (clipped to the grid)
-    const int blox = i0 - 1, bloy = d3 ? j0 - 1 : 0;
-    const int bcols = cmin(ie + 1, nxg) - blox, brows = d3 ? cmin(je + 1, nyg) - bloy : 1;
-    // every HBM load of the block (coefficients, x window, b ring) is in flight before the first wait
-    CoefRegs<T, NZ, WX, WY, NT> cr;
-    WindowRegs<T, NZ, WY, ZX ? 1 : WX, NT> xr;   // unused when ZX
-    WindowRegs<typename std::conditional<ZX, double, T>::type, NZ, TY + 2, TX + 2, NT> br;
-    WindowRegs<T, NZ, PRO ? CWY : 1, PRO ? CWX : 1, NT> pr;   // unused unless PRO
-    cr.load(L, lox, loy, wcols, wrows);
-    if constexpr (ZX) br.load(r0 + ((size_t)bloy * nxg + blox) * NZ, (size_t)nxg * NZ, brows, bcols);
-    else {
-        xr.load(xin + ((size_t)loy * nxg + lox) * NZ, (size_t)nxg * NZ, wrows, wcols);
-        br.load(b + ((size_t)bloy * nxg + blox) * NZ, (size_t)nxg * NZ, brows, bcols);
-    }
-    // coarse columns [cxo, cxo + ccols) x rows [cyo, cyo + crows) reach the window's interior columns
-    const int cxo = ((cmax(lox, 1) - 1) >> 1) + 1, cyo = ((cmax(loy, 1) - 1) >> 1) + 1;
-    const int ccols = (cmin(lox + wcols - 1, nxg - 2) >> 1) + 2 - cxo, crows = (cmin(loy + wrows - 1, nyg - 2) >> 1) + 2 - cyo;
-    int2 pti = make_int2(-1, -1);
-    T ptw0 = T(0), ptw1 = T(0), ptw2 = T(0);
-    if constexpr (PRO) {
-        const int t = (int)threadIdx.x;
-        if (t < wcols) {
-            pti = P.pxi[lox + t];
-            ptw0 = P.pxw[3 * (lox + t)]; ptw1 = P.pxw[3 * (lox + t) + 1]; ptw2 = P.pxw[3 * (lox + t) + 2];
-        } else if (t >= WX && t < WX + wrows) {
-            pti = P.pyi[loy + t - WX];
-            ptw0 = P.pyw[3 * (loy + t - WX)]; ptw1 = P.pyw[3 * (loy + t - WX) + 1]; ptw2 = P.pyw[3 * (loy + t - WX) + 2];
-        }
-        pr.load(P.ec + ((size_t)cyo * P.nxgc + cxo) * NZ, (size_t)P.nxgc * NZ, crows, ccols);
-    }
-    if (L.spec && solve_done(L.skip)) return;
-    const CoefS<T> C = cr.store(sC);
-    if constexpr (ZX) {
-        for (int e = threadIdx.x; e < WX * WY * NZP; e += NT) sX[e] = T(0);
-    } else {
-        xr.template store<NZP, WX>(sX, wrows, wcols);
-    }
-    br.template store<NZ, TX + 2>(sB, brows, bcols);
-    if constexpr (PRO) {
-        const int t = (int)threadIdx.x;
-        if (t < WX + WY) {
-            sPi[t] = pti;
-            sPw[3 * t] = ptw0; sPw[3 * t + 1] = ptw1; sPw[3 * t + 2] = ptw2;
-        }
-        pr.template store<NZP, CWX>(sP, crows, ccols);
-    }
-    __syncthreads();
-    if constexpr (PRO) {
-        // x += interpolated coarse correction on the window's interior columns, sigma levels 1 .. NZ - 2
-        // (k_mg_prolong_tab's arithmetic), before the ghost pass reads them
-        for (int q = threadIdx.x; q < WX * WY; q += NT) {
-            const int r = q / WX, c = q - r * WX;
-            if (r >= wrows || c >= wcols) continue;
-            const int2 xi = sPi[c], yi = sPi[WX + r];
-            if (xi.x < 0 || yi.x < 0) continue;
-            const T wxl = sPw[3 * c], wxr = sPw[3 * c + 1], sxw = sPw[3 * c + 2];
-            const T wyl = sPw[3 * (WX + r)], wyr = sPw[3 * (WX + r) + 1], syw = sPw[3 * (WX + r) + 2];
-            const T *ea = sP + ((yi.x - cyo) * CWX + (xi.x - cxo)) * NZP, *eb = sP + ((yi.x - cyo) * CWX + (xi.y - cxo)) * NZP;
-            const T *ec = sP + ((yi.y - cyo) * CWX + (xi.x - cxo)) * NZP, *ed = sP + ((yi.y - cyo) * CWX + (xi.y - cxo)) * NZP;
-            T *xc = sX + (r * WX + c) * NZP;
-#pragma unroll
-            for (int k = 1; k < NZ - 1; k++) {
-                const T el = (wxl * ea[k] + wxr * eb[k]) * sxw, er = (wxl * ec[k] + wxr * ed[k]) * sxw;
-                const T e = (wyl * el + wyr * er) * syw;
-                xc[k] = xc[k] + e;
-            }
-        }
-        __syncthreads();
-    }
-    // owned points [gi0, gi1) x [gj0, gj1): the tile's columns and the ghost points beside them
-    const int gi0 = (i0 == L.gx) ? 0 : i0, gi1 = (ie == nxg - L.gx) ? nxg : ie;
-    const int gj0 = d3 ? ((j0 == L.gy) ? 0 : j0) : 0, gj1 = d3 ? ((je == nyg - L.gy) ? nyg : je) : 1;
-    if constexpr (ZX) {
-        const int w = (gi1 - gi0) * NZ;
-        for (int r = gj0; r < gj1; r++) {
-            T *dst = bout + ((size_t)r * nxg + gi0) * NZ;
-            const T *src = sB + ((r - bloy) * (TX + 2) + (gi0 - blox)) * NZ;
-            for (int e = threadIdx.x; e < w; e += NT) dst[e] = src[e];
-        }
-    }
-    auto X = [&](int k, int ii, int jj) -> T { return sX[((jj - loy) * WX + (ii - lox)) * NZP + k]; };
-    const int jlo = d3 ? L.gy : 0, jhi = d3 ? nyg - L.gy : 1;
-    // value of wall ghost point (ii, jj, k) of the ring-extended tile from the staged interior values
-    // (GaussSeidelSpecialPoints.f90 rows: identity on the sigma ghost level and at corners, the Neumann row
-    // relaxed pointwise elsewhere)
-    auto ghost_value = [&](int ii, int jj, int k) -> T {
-        const bool wxg = L.gx && (ii == 0 || ii == nxg - 1), wyg = L.gy && (jj == 0 || jj == nyg - 1);
-        const T bq = sB[((jj - bloy) * (TX + 2) + (ii - blox)) * NZ + k];
-        if ((wxg && wyg) || k == 0) return bq;
-        T sum = T(0), dg = T(1);
-        if (wxg) {
-            const int ib = ii == 0 ? 1 : nxg - 2, ws = cclamp(ib - 1, 0, nxg - 3);
-            const T *S = C.sx(ib);
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                if (ws + m == ii) dg = S[m];
-                else sum += S[m] * X(k, ws + m, jj);
-            }
-        } else {
-            const int jb = jj == 0 ? 1 : nyg - 2, ws = cclamp(jb - 1, 0, nyg - 3);
-            const T *S = C.sy(jb);
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                if (ws + m == jj) dg = S[m];
-                else sum += S[m] * X(k, ii, ws + m);
-            }
-        }
-        return (bq - sum) / dg;
-    };
-    auto is_ghost = [&](int ii, int jj) -> bool {
-        return (L.gx && (ii == 0 || ii == nxg - 1)) || (L.gy && (jj == 0 || jj == nyg - 1));
-    };
-    // the ghost pass before the sweep, on the ring-extended tile (ghost values depend on interior values
-    // only; the sweep reads no ghost point outside that ring: a relaxed ring column's outer neighbour is
-    // interior, since no tile is one column or row wide)
-    if (blox == 0 || blox + bcols == nxg || (d3 && (bloy == 0 || bloy + brows == nyg))) {
-        for (int e = threadIdx.x; e < brows * bcols * NZ; e += NT) {
-            const int r = e / (bcols * NZ), rem = e - r * bcols * NZ, c = rem / NZ, k = rem - c * NZ;
-            const int ii = blox + c, jj = bloy + r;
-            if (is_ghost(ii, jj)) {
-                const T v = ghost_value(ii, jj, k);
-                sX[((jj - loy) * WX + (ii - lox)) * NZP + k] = v;
-            }
-        }
-        __syncthreads();
-    }
-    // one half-sweep over the columns of colour COL: red (0) over the ring-extended tile, black (1) over
-    // the tile; slot s of row rr is the t-th column of that colour in the row
-    auto half = [&](auto colour_tag) {
-        constexpr int COL = decltype(colour_tag)::value;
-        constexpr int PER = COL == 0 ? PR : TX / 2;
-        const int r0 = COL == 0 ? (d3 ? j0 - 1 : 0) : j0;
-        const int nr = COL == 0 ? (d3 ? (je - j0) + 2 : 1) : je - j0;
-        const int ib = COL == 0 ? i0 - 1 : i0, iend = COL == 0 ? ie : ie - 1;
-        const int ns = PER * nr;
-        auto slot = [&](int sl, int &i, int &j) -> bool {
-            const int rr = sl / PER, t = sl - rr * PER;
-            j = r0 + rr;
-            i = ib + (((ib + j) & 1) != COL ? 1 : 0) + 2 * t;
-            return i <= iend && j >= jlo && j < jhi && i >= L.gx && i < nxg - L.gx;
-        };
-        // rows in level-major order (task = k * NSM + slot): the lanes of a wave share the level, so
-        // bottom, interior and surface rows do not diverge inside a wave; row arrays are slot-fastest
-        // (sR[(m * NZ + k) * NS + slot]), conflict-free for both phases
-        constexpr int NSM = PER * (COL == 0 ? TY + 2 : TY);
-        for (int task = threadIdx.x; task < NSM * NZ; task += NT) {
-            const int k = task / NSM, sl = task - k * NSM;
-            int i, j;
-            if (sl >= ns || !slot(sl, i, j)) continue;
-            T lo, di, up, rh, e2;
-            const T bk = sB[((j - bloy) * (TX + 2) + (i - blox)) * NZ + k];
-            if (i >= 2 && i <= nxg - 3 && (!d3 || (j >= 2 && j <= nyg - 3))) {
-                const T *cc = sX + ((j - loy) * WX + (i - lox)) * NZP;
-                if (L.uni && k >= 1 && k <= NZ - 2) {
-                    zebra_row_uniform<T, NZP, WX * NZP>(L, C, d3, i, j, k, cc, bk, lo, di, up, rh);
-                    e2 = T(0);
-                } else {
-                    zebra_row_interior<T, NZP, WX * NZP>(C, d3, i, j, k, NZ, cc, bk, lo, di, up, rh, e2);
-                }
-            } else
-                zebra_row<T>(L, C, i, j, k, NZ, X, bk, lo, di, up, rh, e2);
-            sR[(0 * NZ + k) * NS + sl] = lo; sR[(1 * NZ + k) * NS + sl] = di;
-            sR[(2 * NZ + k) * NS + sl] = up; sR[(3 * NZ + k) * NS + sl] = rh;
-            if (k == 0) sE[sl] = e2;
-        }
-        __syncthreads();
-        for (int sl = threadIdx.x; sl < ns; sl += NT) {
-            int i, j;
-            if (!slot(sl, i, j)) continue;
-            T lo[NZ], di[NZ], up[NZ], rh[NZ];
-#pragma unroll
-            for (int k = 0; k < NZ; k++) {
-                lo[k] = sR[(0 * NZ + k) * NS + sl]; di[k] = sR[(1 * NZ + k) * NS + sl];
-                up[k] = sR[(2 * NZ + k) * NS + sl]; rh[k] = sR[(3 * NZ + k) * NS + sl];
-            }
-            zebra_thomas<T, NZ>(lo, di, up, rh, sE[sl], sX + ((j - loy) * WX + (i - lox)) * NZP);
-        }
-        __syncthreads();
-    };
-    half(std::integral_constant<int, 0>{});
-    half(std::integral_constant<int, 1>{});
+    const int nxg = L.nxg, nyg = L.nyg, th = (int)threadIdx.x;
+    const int i0 = tile_begin(nxg - 2, (int)blockIdx.x, (int)gridDim.x), ie = tile_begin(nxg - 2, (int)blockIdx.x + 1, (int)gridDim.x);
+    const int j0 = D3 ? tile_begin(nyg - 2, (int)blockIdx.y, (int)gridDim.y) : 0;
+    const int je = D3 ? tile_begin(nyg - 2, (int)blockIdx.y + 1, (int)gridDim.y) : 1;
+    const int lox = cmax(i0 - H, 0), loy = D3 ? cmax(j0 - H, 0) : 0;
+    const int wcols = cmin(ie + H, nxg) - lox, wrows = D3 ? cmin(je + H, nyg) - loy : 1;
+    const bool ww = i0 == 1, we = ie == nxg - 1, ws = D3 && j0 == 1, wn = D3 && je == nyg - 1;
+    const bool wall = ww || we || ws || wn;
+    const bool edge = th >= G::NR;   // the wave of the columns next to a wall
+    const bool upper = PAIR && th >= G::NR + 32;
     using O = typename std::conditional<ZO, double, T>::type;
     O *const out = ZO ? (O *)uout : (O *)xout;
-    for (int r = 0; r < je - j0; r++)
-        store_row<NZ, NZP, NT>(out + ((size_t)(j0 + r) * nxg + i0) * NZ, sX + ((j0 + r - loy) * WX + (i0 - lox)) * NZP, ie - i0);
-    // the ghost pass after the sweep for the ghost points this tile owns: wall columns beside its rows,
-    // wall rows beside its columns, and the corners of the tiles at the corners of the domain
-    {
-        if (gi0 != i0 || gi1 != ie || gj0 != j0 || gj1 != je) {
-            const int w = gi1 - gi0;
-            for (int e = threadIdx.x; e < (gj1 - gj0) * w * NZ; e += NT) {
-                const int r = e / (w * NZ), rem = e - r * w * NZ, c = rem / NZ, k = rem - c * NZ;
-                const int ii = gi0 + c, jj = gj0 + r;
-                if (is_ghost(ii, jj)) out[((size_t)jj * nxg + ii) * NZ + k] = (O)ghost_value(ii, jj, k);
+    auto lds = [&](int i, int j) -> T * { return sX + ((j - loy) * WX + (i - lox)) * NZP; };
+
+    // a thread's column of a colour, and what its solve needs besides its neighbours
+    struct Column {
+        int i, j;
+        bool on;
+        T b[NZ], rec[Rec::N];
+        LineRows<T, D3> R;
+    };
+    auto load = [&](Column &c, auto colour_tag) {
+        constexpr int COL = decltype(colour_tag)::value;
+        const int ilo = COL == 0 ? cmax(i0 - 1, 1) : i0, ihi = COL == 0 ? cmin(ie, nxg - 2) : ie - 1;
+        const int jlo = !D3 ? 0 : (COL == 0 ? cmax(j0 - 1, 1) : j0), jhi = !D3 ? 0 : (COL == 0 ? cmin(je, nyg - 2) : je - 1);
+        if (!edge) {   // away from the walls
+            const int r = th / G::RX, t = th - r * G::RX;
+            c.j = jlo + r;
+            c.i = ilo + (((ilo + c.j) & 1) != COL ? 1 : 0) + 2 * t;
+            c.on = c.i <= ihi && c.j <= jhi && c.i >= 2 && c.i <= nxg - 3 && (!D3 || (c.j >= 2 && c.j <= nyg - 3));
+        } else {       // south row, north row, then west and east column
+            const int l = PAIR ? (th - G::NR) & 31 : th - G::NR;
+            if (D3 && l < 2 * G::BX) {
+                const bool first = l < G::BX;
+                const int t = first ? l : l - G::BX;
+                c.j = first ? 1 : nyg - 2;
+                c.i = ilo + (((ilo + c.j) & 1) != COL ? 1 : 0) + 2 * t;
+                c.on = c.i <= ihi && c.j >= jlo && c.j <= jhi && (first || nyg > 3);
+            } else {
+                const int q = l - 2 * G::BX;
+                const bool first = q < G::BY;
+                const int t = first ? q : q - G::BY;
+                c.i = first ? 1 : nxg - 2;
+                c.j = jlo + (((c.i + jlo) & 1) != COL ? 1 : 0) + 2 * t;
+                c.on = t < G::BY && c.i >= ilo && c.i <= ihi && c.j <= jhi && (first || nxg > 3) && !(D3 && (c.j == 1 || c.j == nyg - 2));
             }
+        }
+        const int i = c.on ? c.i : 1, j = c.on ? c.j : (D3 ? 1 : 0);   // (idle lanes load a valid column)
+        const size_t p = (size_t)j * nxg + i;
+        if constexpr (ZX) load_column<NZ>(r0 + p * NZ, c.b);
+        else load_column<NZ>(b + p * NZ, c.b);
+        load_record(L.fac + Rec::index(nxg, nyg, i, j) * Rec::N, c.rec);
+        if (edge) c.R.load(L, i, j);
+    };
+    // a window column of one colour per thread: x, with the prolongated correction added
+    struct Staged {
+        int i, j;
+        bool on;
+        T x[NZ];
+    };
+    auto stage_load = [&](Staged &c, int col) {
+        const int r = th / (WX / 2), t = th - r * (WX / 2);
+        c.j = loy + r;
+        c.i = lox + (((lox + c.j) & 1) != col ? 1 : 0) + 2 * t;
+        c.on = r < wrows && c.i < lox + wcols;
+        if (!c.on) return;
+        if constexpr (ZX || ZB) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) c.x[k] = T(0);
+        } else {
+            load_column<NZ>(xin + ((size_t)c.j * nxg + c.i) * NZ, c.x);
+        }
+        if constexpr (PRO) {
+            // interior columns, sigma levels 1 .. NZ - 2; column i lies on coarse column 1 + (i - 1) / 2 or between it
+            // and the next
+            if (c.i >= 1 && c.i <= nxg - 2 && c.j >= 1 && c.j <= nyg - 2) {
+                const int2 xi = make_int2(1 + ((c.i - 1) >> 1), 1 + (c.i >> 1)), yi = make_int2(1 + ((c.j - 1) >> 1), 1 + (c.j >> 1));
+                const T wxl = P.pxw[3 * c.i], wxr = P.pxw[3 * c.i + 1], sxw = P.pxw[3 * c.i + 2];
+                const T wyl = P.pyw[3 * c.j], wyr = P.pyw[3 * c.j + 1], syw = P.pyw[3 * c.j + 2];
+                T ea[NZ], eb[NZ], ec[NZ], ed[NZ];
+                load_column<NZ>(P.ec + ((size_t)yi.x * P.nxgc + xi.x) * NZ, ea);
+                load_column<NZ>(P.ec + ((size_t)yi.x * P.nxgc + xi.y) * NZ, eb);
+                load_column<NZ>(P.ec + ((size_t)yi.y * P.nxgc + xi.x) * NZ, ec);
+                load_column<NZ>(P.ec + ((size_t)yi.y * P.nxgc + xi.y) * NZ, ed);
+#pragma unroll
+                for (int k = 1; k < NZ - 1; k++) {
+                    const T el = fma1(wxl, ea[k], wxr * eb[k]) * sxw, er = fma1(wxl, ec[k], wxr * ed[k]) * sxw;
+                    c.x[k] = fma1(fma1(wyl, el, wyr * er), syw, c.x[k]);
+                }
+            }
+        }
+    };
+    auto stage_store = [&](const Staged &c) {
+        if (!c.on) return;
+        T *d = lds(c.i, c.j);
+#pragma unroll
+        for (int k = 0; k < NZ; k++) d[k] = c.x[k];
+    };
+    // the thread's wall ghost column of the ring-extended tile (west, east, south, north; corners with west and east):
+    // right-hand side and Neumann row (weight of the ghost, of the two columns beside it)
+    int gi = -1, gj = 0;
+    T gb[NZ], dg = T(1), wa = T(0), wb = T(0);
+    if (wall) {
+        if (th < 2 * G::GY) {
+            const bool first = th < G::GY;
+            const int r = (D3 ? j0 - 1 : 0) + (first ? th : th - G::GY);
+            if ((first ? ww : we) && r <= (D3 ? je : 0)) { gi = first ? 0 : nxg - 1; gj = r; }
+        } else if (th < 2 * (G::GX + G::GY)) {
+            const int q = th - 2 * G::GY;
+            const bool first = q < G::GX;
+            const int c = i0 - 1 + (first ? q : q - G::GX);
+            if ((first ? ws : wn) && c <= ie && !(ww && c == 0) && !(we && c == nxg - 1)) { gi = c; gj = first ? 0 : nyg - 1; }
+        }
+        if (gi >= 0) {
+            const size_t p = (size_t)gj * nxg + gi;
+            if constexpr (ZX) load_column<NZ>(r0 + p * NZ, gb);
+            else load_column<NZ>(b + p * NZ, gb);
+            const bool gx = gi == 0 || gi == nxg - 1, low = gx ? gi == 0 : gj == 0;
+            const T *S = gx ? L.sx + (low ? 1 : nxg - 2) * 6 : L.sy + (low ? 1 : nyg - 2) * 6;
+            const T w0 = S[0], w1 = S[1], w2 = S[2];
+            dg = low ? w0 : w2; wa = low ? w1 : w0; wb = low ? w2 : w1;
+        }
+    }
+    // its value from the staged interior values (GaussSeidelSpecialPoints.f90 rows: identity on the sigma ghost
+    // level and at corners, the Neumann row relaxed pointwise elsewhere)
+    auto ghost = [&](T (&v)[NZ]) {
+        const bool gx = gi == 0 || gi == nxg - 1, gy = D3 && (gj == 0 || gj == nyg - 1);
+        if (gx && gy) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) v[k] = gb[k];
+            return;
+        }
+        const bool low = gx ? gi == 0 : gj == 0;
+        const T *xa = gx ? lds(low ? 1 : nxg - 3, gj) : lds(gi, low ? 1 : nyg - 3);
+        const T *xb = gx ? lds(low ? 2 : nxg - 2, gj) : lds(gi, low ? 2 : nyg - 2);
+        v[0] = gb[0];
+#pragma unroll
+        for (int k = 1; k < NZ; k++) {
+            const T sum = fma1(wb, xb[k], wa * xa[k]);
+            v[k] = (gb[k] - sum) / dg;
+        }
+    };
+    auto half = [&](const Column &c, auto x0) {
+        constexpr bool X0 = decltype(x0)::value;   // all neighbours are zero
+        if (c.on) {
+            T *d = lds(c.i, c.j);
+            T f[NZ], up[NZ], inv[NZ], rh[NZ], x[NZ], bw[4];
+            const T c3 = c.rec[Rec::C3], c4 = c.rec[Rec::C4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) bw[q] = c.rec[Rec::BW + q];
+#pragma unroll
+            for (int k = 0; k < NZ - 1; k++) { f[k] = c.rec[k]; up[k] = c.rec[NZ - 1 + k]; inv[k] = c.rec[2 * NZ - 2 + k]; }
+            if constexpr (X0) {
+#pragma unroll
+                for (int k = 0; k < NZ; k++) rh[k] = c.b[k];
+            } else if (!edge && L.uni) {
+                line_rhs_uniform<T, NZ, D3, SXS, SYS>(L, c3, c4, bw, d, c.b, rh);
+            } else if (PAIR && edge) {
+                line_rhs_pair<T, NZ, D3, SXS, SYS>(L, c.i, c.j, upper, c.R, c3, c4, bw, d, c.b, rh);
+            } else {
+                LineRows<T, D3> R = c.R;
+                if (!edge) R.load(L, c.i, c.j);
+                line_rhs_general<T, NZ, D3, SXS, SYS>(L, c.i, c.j, R, c3, c4, bw, d, c.b, rh);
+            }
+            line_solve<T, NZ>(f, up, inv, rh, x);
+            if (!upper) {
+#pragma unroll
+                for (int k = 0; k < NZ; k++) d[k] = x[k];
+                if (c.i >= i0 && c.i < ie && c.j >= j0 && c.j < je) {
+                    const size_t q = ((size_t)c.j * nxg + c.i) * NZ;
+                    store_column<NZ>(out + q, x);
+                    if constexpr (ZX) { if (bout) store_column<NZ>(bout + q, c.b); }
+                }
+            }
+        }
+    };
+    Column red, black;
+    load(red, std::integral_constant<int, 0>{});
+    if constexpr (!ZB) {
+        Staged s1, s0;
+        if (!ZX || wall) {
+            stage_load(s1, 1);
+            if (wall) stage_load(s0, 0);
+        }
+        if (solve_done(L.skip)) return;
+        if (!ZX || wall) {
+            stage_store(s1);
+            if (wall) stage_store(s0);
+        }
+        load(black, std::integral_constant<int, 1>{});
+        if (!ZX || wall) lds_barrier();
+        // the ghost pass before the sweep, on the ring-extended tile (the sweep reads no ghost point outside it)
+        if (wall) {
+            if (gi >= 0) {
+                T v[NZ];
+                ghost(v);
+                T *d = lds(gi, gj);
+#pragma unroll
+                for (int k = 0; k < NZ; k++) d[k] = v[k];
+            }
+            lds_barrier();
+        }
+    } else {
+        load(black, std::integral_constant<int, 1>{});
+        if (solve_done(L.skip)) return;
+        if (gi >= 0) {
+            T *d = lds(gi, gj);
+#pragma unroll
+            for (int k = 0; k < NZ; k++) d[k] = T(0);
+        }
+    }
+    if (ZB || (ZX && !wall && L.uni)) half(red, std::integral_constant<bool, ZX || ZB>{});
+    else half(red, std::false_type{});
+    lds_barrier();
+    half(black, std::false_type{});
+    // the ghost points this tile owns: wall columns beside its rows, wall rows beside its columns, and the corners of the
+    // tiles at the corners of the domain
+    const bool own = gi >= 0 && gi >= (ww ? 0 : i0) && gi < (we ? nxg : ie) && gj >= (ws ? 0 : j0) && gj < (wn ? nyg : je);
+    const size_t gq = ((size_t)gj * nxg + gi) * NZ;
+    if constexpr (ZX) {
+        if (own && bout) store_column<NZ>(bout + gq, gb);
+    }
+    if (!wall || !P.ghosts) return;
+    lds_barrier();
+    if (own) {   // the ghost pass after the sweep
+        T v[NZ];
+        ghost(v);
+        store_column<NZ>(out + gq, v);
+    }
+}
+
+
+// A window of ROWS x COLS columns between HBM and LDS by rows: a thread takes the same piece (two values of a column
+// where NZ is even) of every row, so that its addresses differ by a constant and each row is one contiguous segment.
+template <typename S, int NZ, int ROWS, int COLS, int NT>
+struct RowWindow {
+    static constexpr int E = NZ % 2 == 0 ? 2 : 1, CH = COLS * NZ / E, PER = (CH + NT - 1) / NT;
+    S v[ROWS][PER][E];
+    __device__ __forceinline__ void load(const S *__restrict__ src, size_t pitch, int rows, int cols) {
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+            const int e = ((int)threadIdx.x + p * NT) * E;
+            const bool in = e < cols * NZ;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                if (!in || r >= rows) continue;
+                if constexpr (E == 2) {
+                    const ColPair<S> w = *reinterpret_cast<const ColPair<S> *>(src + (size_t)r * pitch + e);
+                    v[r][p][0] = w.a; v[r][p][1] = w.b;
+                } else {
+                    v[r][p][0] = src[(size_t)r * pitch + e];
+                }
+            }
+        }
+    }
+    template <int NZP, int RS, typename T>
+    __device__ __forceinline__ void store(T *lds, int rows, int cols) const {
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+            const int e = ((int)threadIdx.x + p * NT) * E, c = e / NZ, k = e - c * NZ;
+            if (e >= cols * NZ) continue;
+            T *d = lds + c * NZP + k;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                if (r >= rows) continue;
+#pragma unroll
+                for (int q = 0; q < E; q++) d[r * RS * NZP + q] = (T)v[r][p][q];
+            }
+        }
+    }
+};
+// rows x cols columns from LDS to HBM the same way.
+template <int NZ, int ROWS, int COLS, int NT, int NZP, int RS, typename T, typename O>
+__device__ __forceinline__ void store_rows(O *__restrict__ dst, size_t pitch, const T *lds, int rows, int cols) {
+    constexpr int E = NZ % 2 == 0 ? 2 : 1, CH = COLS * NZ / E, PER = (CH + NT - 1) / NT;
+#pragma unroll
+    for (int p = 0; p < PER; p++) {
+        const int e = ((int)threadIdx.x + p * NT) * E, c = e / NZ, k = e - c * NZ;
+        if (e >= cols * NZ) continue;
+        const T *s = lds + c * NZP + k;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            if (r >= rows) continue;
+            if constexpr (E == 2) *reinterpret_cast<ColPair<O> *>(dst + (size_t)r * pitch + e) = ColPair<O>{(O)s[r * RS * NZP], (O)s[r * RS * NZP + 1]};
+            else dst[(size_t)r * pitch + e] = (O)s[r * RS * NZP];
+        }
+    }
+}
+
+// k_mg_sweep for large 3D levels (same modes, same arithmetic): there the sweep is bound by the throughput of its
+// HBM accesses and by its arithmetic, not by latency (513^2 x 10, FP32: 28 us, of which 12 are the loads, 12 the line
+// solves and 2 the stores; 46 us with the row-per-thread form; FP64 39-42 us against 71-73).  All fields move through LDS in whole rows (column by column,
+// each lane's 40 bytes apart, the address units were busy 60% of a 513^2 sweep's 26 us), the line matrices are
+// formed in registers (reading the records costs more bytes than the arithmetic costs time), the coarse window and
+// then the right-hand sides share one LDS region, and the columns next to a wall are a second pass of the tiles
+// that have some.
+template <int NZ, int TX, int TY>
+struct TiledSweep {
+    static constexpr int H = 2, WX = TX + 2 * H, WY = TY + 2 * H, NZP = NZ | 1, BXC = TX + 2, BYC = TY + 2;
+    static constexpr int RX = TX / 2 + 1, RY = TY + 2, NT = (RX * RY + 63) / 64 * 64;
+    static constexpr int BX = TX / 2 + 1, BY = TY / 2 + 1;              // wall columns of a colour per side
+    static constexpr int CWX = WX / 2 + 2, CWY = WY / 2 + 2;            // coarse window
+    static constexpr int X = WX * WY * NZP, B = cmax(BXC * BYC, CWX * CWY) * NZP, TOTAL = X + B;
+    static_assert(TX % 2 == 0 && TY % 2 == 0, "even tiles");
+    static_assert(2 * (BX + BY) <= NT && 2 * (BXC + BYC) <= NT && (WX / 2) * WY <= 2 * NT, "threads cover the tile's lists");
+};
+template <typename T, int NZ, int TX, int TY, int MODE>
+__global__ __launch_bounds__((TiledSweep<NZ, TX, TY>::NT)) void k_mg_sweep_tiled(
+    LvArgs<T> L, const T *__restrict__ xin, T *__restrict__ xout, const T *__restrict__ b, const double *__restrict__ r0, T *__restrict__ bout,
+    double *__restrict__ uout, ProArgs<T> P) {
+#pragma clang fp contract(off)
+    constexpr bool ZX = MODE == 1, ZB = MODE == 5, ZO = MODE == 2 || MODE == 4, PRO = MODE == 3 || MODE == 4;
+    using G = TiledSweep<NZ, TX, TY>;
+    constexpr int H = G::H, WX = G::WX, WY = G::WY, NZP = G::NZP, NT = G::NT, BXC = G::BXC, BYC = G::BYC, SXS = NZP, SYS = WX * NZP;
+    if (solve_done(L.skip)) return;
+    __shared__ T sX[G::X];
+    __shared__ T sB[G::B];   // the coarse window, then the right-hand sides of the ring-extended tile
+    const int nxg = L.nxg, nyg = L.nyg, nxy = L.nxy, th = (int)threadIdx.x;
+    const int i0 = tile_begin(nxg - 2, (int)blockIdx.x, (int)gridDim.x), ie = tile_begin(nxg - 2, (int)blockIdx.x + 1, (int)gridDim.x);
+    const int j0 = tile_begin(nyg - 2, (int)blockIdx.y, (int)gridDim.y), je = tile_begin(nyg - 2, (int)blockIdx.y + 1, (int)gridDim.y);
+    const int lox = cmax(i0 - H, 0), loy = cmax(j0 - H, 0), wcols = cmin(ie + H, nxg) - lox, wrows = cmin(je + H, nyg) - loy;
+    const int blox = i0 - 1, bloy = j0 - 1, bcols = ie + 1 - blox, brows = je + 1 - bloy;
+    const bool ww = i0 == 1, we = ie == nxg - 1, ws = j0 == 1, wn = je == nyg - 1, wall = ww || we || ws || wn;
+    using O = typename std::conditional<ZO, double, T>::type;
+    O *const out = ZO ? (O *)uout : (O *)xout;
+    auto lds = [&](int i, int j) -> T * { return sX + ((j - loy) * WX + (i - lox)) * NZP; };
+    auto ldb = [&](int i, int j) -> T * { return sB + ((j - bloy) * BXC + (i - blox)) * NZP; };
+    const size_t pitch = (size_t)nxg * NZ;
+    // a thread's column of a colour away from the walls, its planes and first-derivative rows (loaded before the
+    // window's wait; a column's solve would wait for them otherwise)
+    struct Column {
+        int i, j;
+        bool on;
+        T cp[6], s1x[3], s1y[3];
+    };
+    auto column = [&](Column &c, int col) {
+        const int ilo = col == 0 ? cmax(i0 - 1, 1) : i0, ihi = col == 0 ? cmin(ie, nxg - 2) : ie - 1;
+        const int jlo = col == 0 ? cmax(j0 - 1, 1) : j0, jhi = col == 0 ? cmin(je, nyg - 2) : je - 1;
+        const int r = th / G::RX;
+        c.j = jlo + r;
+        c.i = ilo + (((ilo + c.j) & 1) != col ? 1 : 0) + 2 * (th - r * G::RX);
+        c.on = c.i <= ihi && c.j <= jhi && c.i >= 2 && c.i <= nxg - 3 && c.j >= 2 && c.j <= nyg - 3;
+        const int i = c.on ? c.i : 1, j = c.on ? c.j : 1;
+#pragma unroll
+        for (int q = 0; q < 6; q++) c.cp[q] = L.col[(size_t)q * nxy + (size_t)j * nxg + i];
+#pragma unroll
+        for (int m = 0; m < 3; m++) { c.s1x[m] = L.sx[i * 6 + m]; c.s1y[m] = L.sy[j * 6 + m]; }
+    };
+    Column red, black;
+    {
+        RowWindow<T, NZ, WY, WX, NT> xr;
+        RowWindow<typename std::conditional<ZX, double, T>::type, NZ, BYC, BXC, NT> br;
+        const int cxo = ((cmax(lox, 1) - 1) >> 1) + 1, cyo = ((cmax(loy, 1) - 1) >> 1) + 1;   // coarse window's first column, row
+        if constexpr (PRO) {
+            RowWindow<T, NZ, G::CWY, G::CWX, NT> pr;
+            const int ccols = (cmin(lox + wcols - 1, nxg - 2) >> 1) + 2 - cxo, crows = (cmin(loy + wrows - 1, nyg - 2) >> 1) + 2 - cyo;
+            pr.load(P.ec + ((size_t)cyo * P.nxgc + cxo) * NZ, (size_t)P.nxgc * NZ, crows, ccols);
+            xr.load(xin + loy * pitch + (size_t)lox * NZ, pitch, wrows, wcols);
+            br.load(b + bloy * pitch + (size_t)blox * NZ, pitch, brows, bcols);
+            pr.template store<NZP, G::CWX>(sB, crows, ccols);
+            xr.template store<NZP, WX>(sX, wrows, wcols);
+            lds_barrier();
+            // black columns take the correction (no column reads its own old value); in tiles at a wall red ones too,
+            // for the ghost pass
+            for (int q = th; q < (WX / 2) * WY * (wall ? 2 : 1); q += NT) {
+                const int col = q < (WX / 2) * WY ? 1 : 0, e = col ? q : q - (WX / 2) * WY, r = e / (WX / 2);
+                const int j = loy + r, i = lox + (((lox + j) & 1) != col ? 1 : 0) + 2 * (e - r * (WX / 2));
+                if (r >= wrows || i >= lox + wcols || i < 1 || i > nxg - 2 || j < 1 || j > nyg - 2) continue;
+                const T wxl = P.pxw[3 * i], wxr = P.pxw[3 * i + 1], sxw = P.pxw[3 * i + 2];
+                const T wyl = P.pyw[3 * j], wyr = P.pyw[3 * j + 1], syw = P.pyw[3 * j + 2];
+                const int xa = 1 + ((i - 1) >> 1) - cxo, xb = 1 + (i >> 1) - cxo, ya = 1 + ((j - 1) >> 1) - cyo, yb = 1 + (j >> 1) - cyo;
+                const T *ea = sB + (ya * G::CWX + xa) * NZP, *eb = sB + (ya * G::CWX + xb) * NZP;
+                const T *ec = sB + (yb * G::CWX + xa) * NZP, *ed = sB + (yb * G::CWX + xb) * NZP;
+                T *x = lds(i, j);
+#pragma unroll
+                for (int k = 1; k < NZ - 1; k++) {
+                    const T el = fma1(wxl, ea[k], wxr * eb[k]) * sxw, er = fma1(wxl, ec[k], wxr * ed[k]) * sxw;
+                    x[k] = fma1(fma1(wyl, el, wyr * er), syw, x[k]);
+                }
+            }
+            lds_barrier();
+        } else {
+            if constexpr (ZX) {
+                br.load(r0 + bloy * pitch + (size_t)blox * NZ, pitch, brows, bcols);
+            } else {
+                if constexpr (!ZB) xr.load(xin + loy * pitch + (size_t)lox * NZ, pitch, wrows, wcols);
+                br.load(b + bloy * pitch + (size_t)blox * NZ, pitch, brows, bcols);
+            }
+            if constexpr (ZX || ZB) {
+                if (wall) for (int e = th; e < G::X; e += NT) sX[e] = T(0);
+            } else {
+                xr.template store<NZP, WX>(sX, wrows, wcols);
+            }
+        }
+        column(red, 0);
+        br.template store<NZP, BXC>(sB, brows, bcols);
+        lds_barrier();
+    }
+    if (ZX && bout) store_rows<NZ, TY, TX, NT, NZP, BXC>(bout + j0 * pitch + (size_t)i0 * NZ, pitch, ldb(i0, j0), je - j0, ie - i0);
+    // wall ghost column of thread th of the ring-extended tile (west, east, south, north; corners with west and east)
+    int gi = -1, gj = 0;
+    if (wall) {
+        if (th < 2 * BYC) {
+            const bool first = th < BYC;
+            const int r = j0 - 1 + (first ? th : th - BYC);
+            if ((first ? ww : we) && r <= je) { gi = first ? 0 : nxg - 1; gj = r; }
+        } else if (th < 2 * (BXC + BYC)) {
+            const int q = th - 2 * BYC;
+            const bool first = q < BXC;
+            const int c = i0 - 1 + (first ? q : q - BXC);
+            if ((first ? ws : wn) && c <= ie && !(ww && c == 0) && !(we && c == nxg - 1)) { gi = c; gj = first ? 0 : nyg - 1; }
+        }
+    }
+    auto ghost = [&](T (&v)[NZ]) {   // its value, as in k_mg_sweep
+        const bool gx = gi == 0 || gi == nxg - 1, gy = gj == 0 || gj == nyg - 1;
+        const T *gb = ldb(gi, gj);
+        if (gx && gy) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) v[k] = gb[k];
+            return;
+        }
+        const bool low = gx ? gi == 0 : gj == 0;
+        const T *S = gx ? L.sx + (low ? 1 : nxg - 2) * 6 : L.sy + (low ? 1 : nyg - 2) * 6;
+        const T w0 = S[0], w1 = S[1], w2 = S[2];
+        const T dg = low ? w0 : w2, wa = low ? w1 : w0, wb = low ? w2 : w1;
+        const T *xa = gx ? lds(low ? 1 : nxg - 3, gj) : lds(gi, low ? 1 : nyg - 3);
+        const T *xb = gx ? lds(low ? 2 : nxg - 2, gj) : lds(gi, low ? 2 : nyg - 2);
+        v[0] = gb[0];
+#pragma unroll
+        for (int k = 1; k < NZ; k++) {
+            const T sum = fma1(wb, xb[k], wa * xa[k]);
+            v[k] = (gb[k] - sum) / dg;
+        }
+    };
+    if (wall && !ZB) {
+        if (gi >= 0) {
+            T v[NZ];
+            ghost(v);
+            T *d = lds(gi, gj);
+#pragma unroll
+            for (int k = 0; k < NZ; k++) d[k] = v[k];
+        }
+        lds_barrier();
+    }
+    // one column's line solve; x0: all neighbours are zero
+    auto solve = [&](int i, int j, const T (&cp)[6], const T (&s1x)[3], const T (&s1y)[3], auto edge_tag, auto x0) {
+        constexpr bool EDGE = decltype(edge_tag)::value, X0 = decltype(x0)::value;
+        T bc[NZ], lo[NZ], di[NZ], up[NZ], f[NZ], inv[NZ], rh[NZ], x[NZ], e2;
+        T *d = lds(i, j);
+        const T *bl = ldb(i, j);
+        LineRows<T, true> R;
+        if (EDGE || !L.uni) {
+            R.load(L, i, j);
+            line_matrix_general<T, NZ, true>(L, i, j, R, cp, lo, di, up, e2);
+        } else {
+            line_matrix_uniform<T, NZ, true>(L, cp, s1x, s1y, lo, di, up, e2);
+        }
+        const T bw[4] = {cp[1] * s1x[0], cp[1] * s1x[2], cp[2] * s1y[0], cp[2] * s1y[2]};
+        line_factor<T, NZ>(lo, di, up, e2, f, inv);   // before the right-hand side is formed: fewer live values
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < NZ; k++) bc[k] = bl[k];
+        if constexpr (X0) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) rh[k] = bc[k];
+        } else if (EDGE || !L.uni) {
+            line_rhs_general<T, NZ, true, SXS, SYS>(L, i, j, R, cp[3], cp[4], bw, d, bc, rh);
+        } else {
+            line_rhs_uniform<T, NZ, true, SXS, SYS>(L, cp[3], cp[4], bw, d, bc, rh);
+        }
+        line_solve<T, NZ>(f, up, inv, rh, x);
+#pragma unroll
+        for (int k = 0; k < NZ; k++) d[k] = x[k];
+    };
+    auto half = [&](const Column &c, int col, auto x0) {
+        if (c.on) solve(c.i, c.j, c.cp, c.s1x, c.s1y, std::false_type{}, x0);
+        if (wall && th < 2 * (G::BX + G::BY)) {   // beside the walls: south row, north row, then west and east column
+            const int ilo = col == 0 ? cmax(i0 - 1, 1) : i0, ihi = col == 0 ? cmin(ie, nxg - 2) : ie - 1;
+            const int jlo = col == 0 ? cmax(j0 - 1, 1) : j0, jhi = col == 0 ? cmin(je, nyg - 2) : je - 1;
+            int i, j;
+            bool on;
+            if (th < 2 * G::BX) {
+                const bool first = th < G::BX;
+                j = first ? 1 : nyg - 2;
+                i = ilo + (((ilo + j) & 1) != col ? 1 : 0) + 2 * (first ? th : th - G::BX);
+                on = i <= ihi && j >= jlo && j <= jhi && (first || nyg > 3);
+            } else {
+                const int q = th - 2 * G::BX;
+                const bool first = q < G::BY;
+                i = first ? 1 : nxg - 2;
+                j = jlo + (((i + jlo) & 1) != col ? 1 : 0) + 2 * (first ? q : q - G::BY);
+                on = i >= ilo && i <= ihi && j <= jhi && (first || nxg > 3) && j != 1 && j != nyg - 2;
+            }
+            if (on) {
+                T cp[6], s1x[3], s1y[3];
+#pragma unroll
+                for (int q = 0; q < 6; q++) cp[q] = L.col[(size_t)q * nxy + (size_t)j * nxg + i];
+#pragma unroll
+                for (int m = 0; m < 3; m++) { s1x[m] = L.sx[i * 6 + m]; s1y[m] = L.sy[j * 6 + m]; }
+                solve(i, j, cp, s1x, s1y, std::true_type{}, x0);
+            }
+        }
+        lds_barrier();
+    };
+    column(black, 1);
+    if (ZB || (ZX && !wall)) half(red, 0, std::integral_constant<bool, ZX || ZB>{});
+    else half(red, 0, std::false_type{});
+    half(black, 1, std::false_type{});
+    store_rows<NZ, TY, TX, NT, NZP, WX>(out + j0 * pitch + (size_t)i0 * NZ, pitch, lds(i0, j0), je - j0, ie - i0);
+    if (gi >= 0 && gi >= (ww ? 0 : i0) && gi < (we ? nxg : ie) && gj >= (ws ? 0 : j0) && gj < (wn ? nyg : je)) {
+        const size_t q = gj * pitch + (size_t)gi * NZ;
+        T v[NZ];
+        if (ZX && bout) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) v[k] = ldb(gi, gj)[k];
+            store_column<NZ>(bout + q, v);
+        }
+        if (P.ghosts) {
+            ghost(v);
+            store_column<NZ>(out + q, v);
         }
     }
 }
@@ -2667,12 +3169,12 @@ __device__ __forceinline__ T restrict_value(const RestrictGeo &G, size_t q, cons
     const size_t col = q / G.nzgc;
     return restrict_at(G, kc, (int)(col % G.nxgc), (int)(col / G.nxgc), rf);
 }
-// Coarse point q; also clears the coarse iterate xz (the coarse V cycle starts from zero).
+// Coarse point q; also clears the coarse iterate xz where the coarse level's sweep reads it (nullptr otherwise).
 template <typename T>
 __device__ __forceinline__ void restrict_point(const RestrictGeo &G, size_t q, const T *__restrict__ rf, T *__restrict__ rc, T *__restrict__ xz) {
     const size_t nc = (size_t)G.nxgc * G.nygc * G.nzgc;
     if (q >= nc) return;
-    xz[q] = T(0);
+    if (xz) xz[q] = T(0);
     rc[q] = restrict_value(G, q, rf);
 }
 template <typename T>
@@ -2682,7 +3184,7 @@ __global__ void k_mg_restrict(RestrictGeo G, const T *__restrict__ rf, T *__rest
     if (q >= (size_t)G.nxgc * G.nygc * G.nzgc) return;
     const T v = restrict_value(G, q, rf);
     if (G.spec && solve_done(G.skip)) return;
-    xz[q] = T(0);
+    if (xz) xz[q] = T(0);
     rc[q] = v;
 }
 // The same with one grid row of coarse columns per blockIdx.y and the coarse level count NZC known at
@@ -2696,7 +3198,7 @@ __global__ void k_mg_restrict_t(RestrictGeo G, const T *__restrict__ rf, T *__re
     const T v = restrict_at(G, kc, ic, jc, rf);
     if (G.spec && solve_done(G.skip)) return;
     const size_t q = (size_t)jc * G.nxgc * NZC + t;
-    xz[q] = T(0);
+    if (xz) xz[q] = T(0);
     rc[q] = v;
 }
 
@@ -2813,7 +3315,7 @@ __global__ void k_mg_restrict_tab(RestrictGeo G, const T *__restrict__ rxw, cons
     }
     if (G.spec && solve_done(G.skip)) return;
     const size_t q = (size_t)jc * G.nxgc * NZC + t;
-    xz[q] = T(0);
+    if (xz) xz[q] = T(0);
     rc[q] = v;
 }
 
@@ -2914,7 +3416,7 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(LvArgs<T> L, Restri
             }
         }
         const size_t q = ((size_t)jc * G.nxgc + ic) * NZ + k;
-        xz[q] = T(0);
+        if (xz) xz[q] = T(0);
         rc[q] = v;
     }
 }

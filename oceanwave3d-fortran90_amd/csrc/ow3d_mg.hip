@@ -5,6 +5,20 @@
 
 namespace ow3d_host {
 
+namespace {
+bool plane_coarsened(const Grid &f, const Grid &c) { return c.xc && c.yc && !c.zc && f.ny > 1; }   // MgLevel::ptab
+}  // namespace
+
+bool needs_b(const ow3d_tank *t, int k) {
+    const int top = (int)t->levels.size() - 1;
+    return !(k == top && top >= 1 && t->cfg.mg_precision == 0 && t->fused_rb && t->cfg.nu1 >= 1 && t->bot_lim == 0);
+}
+bool needs_r(const ow3d_tank *t, int k) {
+    // (the one-launch residual and restriction of 14 FP64 values a column exceeds 64 KiB of LDS)
+    const bool fits = t->cfg.mg_precision != 0 || t->levels[k].nzg < 14;
+    return t->bot_lim > 0 || (k > 0 && !(fits && plane_coarsened(t->levels[k], t->levels[k - 1])));
+}
+
 // Multigrid hierarchy of the tank (MGPreProcess.f90:6-460 with coarsening strategy 0), level operators in
 // the precision the configuration asks for, and the levels handed to the one-workgroup bottom kernel.
 int mg_setup(ow3d_tank *t) {
@@ -14,17 +28,15 @@ int mg_setup(ow3d_tank *t) {
     for (auto &L : t->levels)
         if (L.nzg < 3 || L.nzg > 14) { err() = "multigrid level depth outside 3..14"; return -1; }
     if (t->levels[0].n > 4096) { err() = "coarsest multigrid level too large for the dense solve"; return -1; }
-    int rc = c.mg_precision == 0 ? mg_build64(t) : mg_build32(t);
-    if (rc) return -1;
     // levels small enough for the one-workgroup bottom kernel (OW3D_MG_BOTTOM: point limit, 0 = off)
     // The group must share one column depth on levels 1 .. bot_top (level 0 is solved densely).
-    long lim = 0;
-    if (const char *e = std::getenv("OW3D_MG_BOTTOM")) lim = std::atol(e);
-    if (c.mg_precision == 2) lim = 0;   // the bottom kernel reads the FP32 inverse
+    if (const char *e = std::getenv("OW3D_MG_BOTTOM")) t->bot_lim = std::atol(e);
+    if (c.mg_precision == 2) t->bot_lim = 0;   // the bottom kernel reads the FP32 inverse
     if (const char *e = std::getenv("OW3D_MG_FUSED_RB")) t->fused_rb = e[0] != '0';
+    if (c.mg_precision == 0 ? mg_build64(t) : mg_build32(t)) return -1;
     t->bot_top = -1;
     for (int k = 1; k < t->nlev && k < MG_BOTTOM_MAX; k++) {
-        if ((long)t->levels[k].n > lim) break;
+        if ((long)t->levels[k].n > t->bot_lim) break;
         bool same = true;
         for (int q = 1; q < k; q++) same &= t->levels[q].nzg == t->levels[k].nzg;
         if (same) t->bot_top = k;

@@ -14,19 +14,6 @@ constexpr size_t residual_lds() {
     constexpr int C3 = CoefLds<WX, WY, NZ>::TOTAL, C2 = CoefLds<RS2, 1, NZ>::TOTAL;
     return ((size_t)LX * (NZ | 1) + (C3 > C2 ? C3 : C2)) * sizeof(T);
 }
-template <typename T, int NZ, int TX, int TY>
-constexpr size_t rb_lds() {
-    constexpr int NS = ((TX + 2) / 2) * (TY + 2);
-    return ((size_t)(TX + 4) * (TY + 4) * (NZ | 1) + CoefLds<TX + 4, TY + 4, NZ>::TOTAL + 4 * NS * NZ + NS +
-            (size_t)(TX + 2) * (TY + 2) * NZ) * sizeof(T);
-}
-// The same with the prolongation's coarse window and tables (MODE 3 and 4).
-template <typename T, int NZ, int TX, int TY>
-constexpr size_t rb_lds_pro() {
-    using W = ProWindow<TX + 4, TY + 4>;
-    return rb_lds<T, NZ, TX, TY>() + (size_t)W::CWX * W::CWY * (NZ | 1) * sizeof(T) + (size_t)(TX + TY + 8) * (sizeof(int2) + 3 * sizeof(T));
-}
-
 template <typename T, int NZ>
 void mg_launch_nz(const LvArgs<T> &L, int what, int colour, T *x, const T *b, T *r, hipStream_t s) {
     if (what == 0) {
@@ -205,6 +192,20 @@ inline bool uniform_rows(const std::vector<double> &S, int N, double *c) {
     return true;
 }
 
+// Factors of a level's line matrices (k_mg_factor).
+template <typename T>
+int factor_launch(const LvArgs<T> &L, T *fac, hipStream_t s) {
+    const dim3 grid((L.nxy + 255) / 256);
+    switch (L.nzg) {
+#define OW3D_NZF(N) case N: if (L.dim3) hipLaunchKernelGGL((k_mg_factor<T, N, true>), grid, dim3(256), 0, s, L, fac); \
+                            else hipLaunchKernelGGL((k_mg_factor<T, N, false>), grid, dim3(256), 0, s, L, fac); return 0;
+        OW3D_NZF(3) OW3D_NZF(4) OW3D_NZF(5) OW3D_NZF(6) OW3D_NZF(7) OW3D_NZF(8) OW3D_NZF(9) OW3D_NZF(10)
+        OW3D_NZF(11) OW3D_NZF(12) OW3D_NZF(13) OW3D_NZF(14)
+#undef OW3D_NZF
+    }
+    return -1;
+}
+
 template <typename T>
 int mg_build(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg) {
     hipStream_t s = t->s;
@@ -234,7 +235,9 @@ int mg_build(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg) {
         HIPCHK(up(L->sx, g.sx)); HIPCHK(up(L->sy, sy)); HIPCHK(up(L->sz, g.sz)); HIPCHK(up(L->zs, zs)); HIPCHK(up(L->col, col));
         // the coarsest level's b is padded with zeros to the inverse's row pitch (whole 16-byte loads)
         const size_t nb = k == 0 ? (size_t)minv_pitch((int)g.n) : g.n;
-        HIPCHK(L->x.alloc(g.n)); HIPCHK(L->x2.alloc(g.n)); HIPCHK(L->b.alloc(nb)); HIPCHK(L->r.alloc(g.n));
+        HIPCHK(L->x.alloc(g.n)); HIPCHK(L->x2.alloc(g.n));
+        if (needs_b(t, k)) HIPCHK(L->b.alloc(nb));
+        if (needs_r(t, k)) HIPCHK(L->r.alloc(g.n));
         if (k == 0) HIPCHK(hipMemset(L->b.p, 0, nb * sizeof(T)));
         HIPCHK(L->xf.alloc(g.nxg)); HIPCHK(L->yf.alloc(g.nyg)); HIPCHK(L->zf.alloc(g.nzg));
         HIPCHK(hipMemcpy(L->xf.p, g.x.data(), g.nxg * 8, hipMemcpyHostToDevice));
@@ -283,6 +286,13 @@ int mg_build(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg) {
             L->args.uni = ux && uy;
             L->args.cx1 = (T)c[0]; L->args.cx2 = (T)c[1]; L->args.cxc = (T)c[2];
             L->args.cy1 = (T)c[3]; L->args.cy2 = (T)c[4]; L->args.cyc = (T)c[5];
+        }
+        L->args.fac = nullptr;
+        if (k > 0 && has_records(g)) {
+            HIPCHK(L->fac.alloc(line_records<T>(g.nxg, g.nyg, g.nzg)));
+            if (factor_launch<T>(L->args, L->fac.p, s)) { err() = "multigrid level depth outside 3..14"; return -1; }
+            HIPCHK(hipGetLastError());
+            L->args.fac = L->fac.p;
         }
         mg.push_back(std::move(L));
     }
@@ -375,10 +385,10 @@ int fill_bottom(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, Bott
 }
 
 template <typename T>
-void ghost_pass(MgLevel<T> &L, T *x, hipStream_t s) {
+void ghost_pass(MgLevel<T> &L, T *x, const T *b, hipStream_t s) {
     const Grid &g = L.g;
     const int nb = (g.ny > 1 ? 2 * g.nxg + 2 * (g.nyg - 2) : 2) * g.nzg;
-    hipLaunchKernelGGL((k_mg_ghost_p<T>), dim3((nb + 255) / 256), dim3(256), 0, s, L.args, x, (const T *)L.b.p);
+    hipLaunchKernelGGL((k_mg_ghost_p<T>), dim3((nb + 255) / 256), dim3(256), 0, s, L.args, x, b);
 }
 
 // Restriction and prolongation: one grid row of columns per blockIdx.y with the level count a template
@@ -409,20 +419,20 @@ void restrict_tab_launch(const RestrictGeo &G, const MgLevel<T> &F, const T *rf,
 // column depths whose tile fits 64 KiB of LDS; false otherwise (the caller then launches the two).  Coarse
 // tiles of 8 x 7 columns: 17 x 15 fine columns, one per thread of 256.
 template <typename T, int NZ>
-bool resrestrict_nz(const MgLevel<T> &F, const RestrictGeo &G, const T *x, T *rc, T *xz, hipStream_t s) {
+bool resrestrict_nz(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
     constexpr int CX = 8, CY = 7;
     if constexpr (ResRestrictLds<NZ, CX, CY>::TOTAL * sizeof(T) <= 65536) {
         hipLaunchKernelGGL((k_mg_residual_restrict<T, NZ, CX, CY, 256>), dim3((G.nxgc + CX - 1) / CX, (G.nygc + CY - 1) / CY), dim3(256), 0, s,
-                           F.args, G, (const T *)F.rxw.p, (const T *)F.ryw.p, x, (const T *)F.b.p, rc, xz);
+                           F.args, G, (const T *)F.rxw.p, (const T *)F.ryw.p, x, b, rc, xz);
         return true;
     }
     return false;
 }
 template <typename T>
-bool resrestrict_launch(const MgLevel<T> &F, const RestrictGeo &G, const T *x, T *rc, T *xz, hipStream_t s) {
+bool resrestrict_launch(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
     if (!F.ptab || !F.args.dim3 || G.gx != 1 || G.gy != 1 || G.nzgc != F.g.nzg) return false;
     switch (F.g.nzg) {
-#define OW3D_NZ(N) case N: return resrestrict_nz<T, N>(F, G, x, rc, xz, s);
+#define OW3D_NZ(N) case N: return resrestrict_nz<T, N>(F, G, x, b, rc, xz, s);
         OW3D_NZ(3) OW3D_NZ(4) OW3D_NZ(5) OW3D_NZ(6) OW3D_NZ(7) OW3D_NZ(8) OW3D_NZ(9) OW3D_NZ(10)
         OW3D_NZ(11) OW3D_NZ(12) OW3D_NZ(13) OW3D_NZ(14)
 #undef OW3D_NZ
@@ -452,65 +462,62 @@ void prolong_launch(const RestrictGeo &G, const T *ec, T *xf, hipStream_t s) {
     hipLaunchKernelGGL((k_mg_prolong_add<T>), dim3(grid_blocks((size_t)G.nxgf * G.nygf * G.nzgf)), dim3(256), 0, s, G, ec, xf);
 }
 
-// Fused sweep on TX x TY tiles with NT threads (the launch grid the kernel's tile arithmetic assumes).
-// With pro (not NULL) the sweep first adds the prolongated coarse correction; false (nothing launched)
-// when that tile does not fit 64 KiB of LDS.
-template <typename T, int NZ, int TX, int TY, int NT>
-bool rb_tiles(const LvArgs<T> &L, const T *xin, T *xout, const T *b, hipStream_t s, const double *r0, T *bout, double *uout,
-              const ProArgs<T> *pro) {
-    static_assert(rb_lds<T, NZ, TX, TY>() <= 65536, "zebra sweep tile exceeds 64 KiB of LDS");
-    const int nxi = L.nxg - 2 * L.gx, nyi = L.dim3 ? L.nyg - 2 * L.gy : 1;
-    const int offx = (nxi % TX == 1) ? 1 : 0, offy = (L.dim3 && nyi % TY == 1) ? 1 : 0;
-    const dim3 grid((nxi + offx + TX - 1) / TX, L.dim3 ? (nyi + offy + TY - 1) / TY : 1);
-    const ProArgs<T> P = pro ? *pro : ProArgs<T>{};
-    if (pro) {
-        if constexpr (rb_lds_pro<T, NZ, TX, TY>() <= 65536) {
-            if (uout) hipLaunchKernelGGL((k_mg_zebra_rb<T, NZ, TX, TY, NT, 4>), grid, dim3(NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
-            else hipLaunchKernelGGL((k_mg_zebra_rb<T, NZ, TX, TY, NT, 3>), grid, dim3(NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
-            return true;
-        }
-        return false;
-    }
-    if (r0) hipLaunchKernelGGL((k_mg_zebra_rb<T, NZ, TX, TY, NT, 1>), grid, dim3(NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
-    else if (uout) hipLaunchKernelGGL((k_mg_zebra_rb<T, NZ, TX, TY, NT, 2>), grid, dim3(NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
-    else hipLaunchKernelGGL((k_mg_zebra_rb<T, NZ, TX, TY, NT>), grid, dim3(NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
-    return true;
-}
-
 // Fused red-black sweep from xin into xout (out of place: a block's staged neighbours must not change
 // under it while other blocks write their results).
-template <typename T, int NZ>
-bool rb_launch_nz(const LvArgs<T> &L, const T *xin, T *xout, const T *b, int threads, hipStream_t s,
-                  const double *r0, T *bout, double *uout, const ProArgs<T> *pro) {
-    // the widest tile (32, 16 or 8 columns, 4 rows) whose staged data fits in 56 KiB of LDS
-    constexpr int TY = 4, TX = rb_lds<T, NZ, 32, TY>() <= 57344 ? 32 : (rb_lds<T, NZ, 16, TY>() <= 57344 ? 16 : 8);
-    const int nxi = L.nxg - 2 * L.gx, nyi = L.dim3 ? L.nyg - 2 * L.gy : 1;
-    const long tiles = (long)((nxi + TX - 1) / TX) * (L.dim3 ? (nyi + TY - 1) / TY : 1);
-    // FP32 3D levels with many tiles (measured at 513^2 x 10 and 257^2 x 10, kernel medians per sweep):
-    // 16 x 8 tiles of 512 threads on the largest (42.7 us against 49.0 us for 32 x 4 tiles of 1024
-    // threads: with twice the blocks per CU one block's loads overlap another's rows), 32 x 4 tiles of
-    // 512 threads on the next (20.4 against 22.2 us); smaller levels keep one 1024-thread block per tile
-    if constexpr (sizeof(T) == 4 && TX == 32 && rb_lds<T, NZ, 16, 8>() <= 65536) {
-        if (L.dim3 && threads != 256 && tiles >= 1500) return rb_tiles<T, NZ, 16, 8, 512>(L, xin, xout, b, s, r0, bout, uout, pro);
-        if (L.dim3 && threads != 256 && tiles >= 400) return rb_tiles<T, NZ, 32, 4, 512>(L, xin, xout, b, s, r0, bout, uout, pro);
+template <typename T, int NZ, int TX, int TY, bool TILED>
+void sweep_tiles(const LvArgs<T> &L, const T *xin, T *xout, const T *b, hipStream_t s, const double *r0, T *bout, double *uout,
+                 const ProArgs<T> *pro, bool zero, bool ghosts) {
+    constexpr bool D3 = TY > 1;
+    const dim3 grid((L.nxg - 2 + TX - 1) / TX, D3 ? (L.nyg - 2 + TY - 1) / TY : 1);
+    ProArgs<T> P = pro ? *pro : ProArgs<T>{};
+    P.ghosts = ghosts;
+    auto go = [&](auto mode) {
+        constexpr int M = decltype(mode)::value;
+        if constexpr (TILED) {
+            using G = TiledSweep<NZ, TX, TY>;
+            static_assert(G::TOTAL * sizeof(T) <= 65536, "zebra sweep tile exceeds 64 KiB of LDS");
+            hipLaunchKernelGGL((k_mg_sweep_tiled<T, NZ, TX, TY, M>), grid, dim3(G::NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
+        } else {
+            using G = SweepTile<NZ, TX, TY>;
+            static_assert((size_t)G::WX * G::WY * G::NZP * sizeof(T) <= 65536, "zebra sweep tile exceeds 64 KiB of LDS");
+            hipLaunchKernelGGL((k_mg_sweep<T, NZ, TX, TY, M>), grid, dim3(G::NT), 0, s, L, xin, xout, b, r0, bout, uout, P);
+        }
+    };
+    if constexpr (D3) {
+        if (pro) {
+            if (uout) go(std::integral_constant<int, 4>{});
+            else go(std::integral_constant<int, 3>{});
+            return;
+        }
     }
-    // levels with fewer tiles than CUs are latency-bound: give each tile 1024 threads (about one row of
-    // the line systems per thread); larger levels use 256-thread blocks for occupancy
-    const bool big = threads == 1024 || (threads == 0 && tiles < 256);
-    if (big) return rb_tiles<T, NZ, TX, TY, 1024>(L, xin, xout, b, s, r0, bout, uout, pro);
-    return rb_tiles<T, NZ, TX, TY, 256>(L, xin, xout, b, s, r0, bout, uout, pro);
+    if (zero) go(std::integral_constant<int, 5>{});
+    else if (r0) go(std::integral_constant<int, 1>{});
+    else if (uout) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 0>{});
+}
+// Levels whose column records are kept (up to SWEEP_RECORD_POINTS points, and all x-z levels) take the latency-bound
+// kernel, larger ones the tiled one.  At 257^2 x 10 the first takes 8.4 / 9.4 us (from zero / with the correction; FP64
+// 12.3 / 18.5) and the second 13 / 18 (18 / 23); at 513^2 x 10 both take 27-28 us in FP32, and in FP64 45-49 us and
+// 39-42, the records' 76 MB being the difference.
+template <typename T, int NZ>
+void sweep_nz(const LvArgs<T> &L, const T *xin, T *xout, const T *b, hipStream_t s, const double *r0, T *bout, double *uout,
+              const ProArgs<T> *pro, bool zero, bool ghosts) {
+    if (!L.dim3) sweep_tiles<T, NZ, 66, 1, false>(L, xin, xout, b, s, r0, bout, uout, nullptr, zero, ghosts);
+    else if (L.fac) sweep_tiles<T, NZ, 18, 8, false>(L, xin, xout, b, s, r0, bout, uout, pro, zero, ghosts);
+    // 36 x 8 columns fill 190 of 192 threads of the red half; in FP64 such a tile would exceed 64 KiB
+    else sweep_tiles<T, NZ, sizeof(T) == 4 ? 36 : 18, 8, true>(L, xin, xout, b, s, r0, bout, uout, pro, zero, ghosts);
 }
 
 // Fused sweep xin -> xout; with r0 (not NULL) the first sweep of an application: x = 0 and b = (T) r0,
 // written to bout (the level's b); with uout (not NULL) the last: the result goes to uout in FP64 and
-// xout is not written; with pro (not NULL) the prolongated coarse correction is added to xin's values
-// first.  Returns 0 when launched, 1 when the prolongating form does not fit (nothing launched), -1 for
-// a column depth outside 3..14.
+// xout is not written; with pro (not NULL; 3D levels) the prolongated coarse correction is added to xin's
+// values first; with zero the first sweep of a coarse level: x = 0 (xin is not read).  ghosts: the wall ghost
+// points of the result are set too.  Returns 0 when launched, -1 for a column depth outside 3..14.
 template <typename T>
-int rb_launch(const LvArgs<T> &L, const T *xin, T *xout, const T *b, int threads, hipStream_t s,
-              const double *r0 = nullptr, T *bout = nullptr, double *uout = nullptr, const ProArgs<T> *pro = nullptr) {
+int sweep_launch(const LvArgs<T> &L, const T *xin, T *xout, const T *b, hipStream_t s, const double *r0, T *bout, double *uout,
+                 const ProArgs<T> *pro, bool zero, bool ghosts) {
     switch (L.nzg) {
-#define OW3D_NZ(N) case N: return rb_launch_nz<T, N>(L, xin, xout, b, threads, s, r0, bout, uout, pro) ? 0 : 1;
+#define OW3D_NZ(N) case N: sweep_nz<T, N>(L, xin, xout, b, s, r0, bout, uout, pro, zero, ghosts); return 0;
         OW3D_NZ(3) OW3D_NZ(4) OW3D_NZ(5) OW3D_NZ(6) OW3D_NZ(7) OW3D_NZ(8) OW3D_NZ(9) OW3D_NZ(10)
         OW3D_NZ(11) OW3D_NZ(12) OW3D_NZ(13) OW3D_NZ(14)
 #undef OW3D_NZ
@@ -523,27 +530,29 @@ int rb_launch(const LvArgs<T> &L, const T *xin, T *xout, const T *b, int threads
 // r0 (fused sweeps, nu >= 1 only): the level's x is zero and its b is (T) r0, both still to be set; the
 // first sweep does it.  uout (fused sweeps, nu >= 1 only): the last sweep writes its result there in FP64
 // (cur is then stale).
-// pro (fused sweeps, nu >= 1 only): the first sweep adds the prolongated coarse correction to cur's values;
-// returns 1 with nothing launched when that sweep form does not fit.
+// pro (fused sweeps, nu >= 1 only): the first sweep adds the prolongated coarse correction to cur's values.
+// zero (fused sweeps, nu >= 1 only): cur is zero and not read.  ghosts: the wall ghost points of the last sweep's
+// result are read (those of the others are set anew by the next sweep).
+// b: the level's right-hand side (with r0 and an FP64 level it may be r0 itself: b = r0 is then not written).
 template <typename T>
-int smooth(ow3d_tank *t, MgLevel<T> &L, int nu, T *&cur, hipStream_t s, const double *r0 = nullptr,
-           double *uout = nullptr, const ProArgs<T> *pro = nullptr) {
+int smooth(ow3d_tank *t, MgLevel<T> &L, const T *b, int nu, T *&cur, hipStream_t s, const double *r0, double *uout, const ProArgs<T> *pro,
+           bool zero, bool ghosts) {
     if (t->fused_rb) {   // each launch is (ghost pass, red, black, ghost pass)
-        if (nu == 0) ghost_pass(L, cur, s);
+        if (nu == 0) ghost_pass(L, cur, b, s);
         for (int it = 0; it < nu; it++) {
             T *nxt = (cur == L.x.p) ? L.x2.p : L.x.p;
-            const int rc = rb_launch<T>(L.args, cur, nxt, L.b.p, t->rb_threads, s, it == 0 ? r0 : nullptr, L.b.p,
-                                        it == nu - 1 ? uout : nullptr, it == 0 ? pro : nullptr);
+            const int rc = sweep_launch<T>(L.args, cur, nxt, b, s, it == 0 ? r0 : nullptr, (const void *)b == r0 ? nullptr : L.b.p,
+                                           it == nu - 1 ? uout : nullptr, it == 0 ? pro : nullptr, zero && it == 0, ghosts && it == nu - 1);
             if (rc) return rc;
             cur = nxt;
         }
         return 0;
     }
-    ghost_pass(L, cur, s);
+    ghost_pass(L, cur, b, s);
     for (int it = 0; it < nu; it++) {
-        if (mg_launch<T>(L.args, 1, 0, cur, L.b.p, nullptr, s)) return -1;
-        if (mg_launch<T>(L.args, 1, 1, cur, L.b.p, nullptr, s)) return -1;
-        ghost_pass(L, cur, s);
+        if (mg_launch<T>(L.args, 1, 0, cur, b, nullptr, s)) return -1;
+        if (mg_launch<T>(L.args, 1, 1, cur, b, nullptr, s)) return -1;
+        ghost_pass(L, cur, b, s);
     }
     return 0;
 }
@@ -552,10 +561,10 @@ template <typename T> const BottomArgs<T> *bottom_args(const ow3d_tank *t);
 template <> inline const BottomArgs<double> *bottom_args<double>(const ow3d_tank *t) { return t->bot64d.p; }
 template <> inline const BottomArgs<float> *bottom_args<float>(const ow3d_tank *t) { return t->bot32d.p; }
 
-// V cycle on level k from its current iterate `cur` (on entry L.x for every level below the finest);
+// V cycle on level k with right-hand side b from its current iterate `cur` (on entry L.x for every level below the finest);
 // on return `cur` points at the buffer holding the result.
 template <typename T>
-int vcycle(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, int k, T *&cur, hipStream_t s,
+int vcycle(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, int k, const T *b, T *&cur, hipStream_t s,
            const double *r0 = nullptr, double *uout = nullptr) {
     MgLevel<T> &L = *mg[k];
     if (k == t->bot_top) {   // in place on L.x
@@ -572,35 +581,36 @@ int vcycle(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, int k, T 
     if (k == 0) {
         if (L.minv16.p)
             hipLaunchKernelGGL((k_mg_coarse<T, __half>), dim3(((int)L.g.n + 3) / 4), dim3(256), 0, s, (int)L.g.n, L.minv_pitch,
-                               (const __half *)L.minv16.p, (const T *)L.b.p, L.x.p, t->done());
+                               (const __half *)L.minv16.p, b, L.x.p, t->done());
         else
             hipLaunchKernelGGL((k_mg_coarse<T, T>), dim3(((int)L.g.n + 3) / 4), dim3(256), 0, s, (int)L.g.n, L.minv_pitch,
-                               (const T *)L.minv.p, (const T *)L.b.p, L.x.p, t->done());
+                               (const T *)L.minv.p, b, L.x.p, t->done());
         cur = L.x.p;
         return 0;
     }
     MgLevel<T> &C = *mg[k - 1];
-    if (smooth(t, L, t->cfg.nu1, cur, s, r0)) return -1;
+    const bool top = k == t->nlev - 1, zero = !top && t->fused_rb && t->cfg.nu1 >= 1;
+    if (smooth<T>(t, L, b, t->cfg.nu1, cur, s, r0, nullptr, nullptr, zero, true)) return -1;
     RestrictGeo G = geo(L.g, C.g, L.xf.p, L.yf.p, L.zf.p, t->done());
     G.spec = L.args.spec;
-    if (!resrestrict_launch<T>(L, G, cur, C.b.p, C.x.p, s)) {
-        if (mg_launch<T>(L.args, 0, 0, cur, L.b.p, L.r.p, s)) return -1;
-        if (L.ptab) restrict_tab_launch<T>(G, L, (const T *)L.r.p, C.b.p, C.x.p, s);
-        else restrict_launch<T>(G, (const T *)L.r.p, C.b.p, C.x.p, s);
+    // the coarse iterate is cleared where something reads it: not by the dense solve, nor by a first sweep from zero
+    T *xz = t->bot_top < 0 && (k == 1 || (t->fused_rb && t->cfg.nu1 >= 1)) ? nullptr : C.x.p;
+    if (!resrestrict_launch<T>(L, G, cur, b, C.b.p, xz, s)) {
+        if (!L.r.p) { err() = "multigrid level has no residual buffer"; return -1; }   // needs_r says otherwise
+        if (mg_launch<T>(L.args, 0, 0, cur, b, L.r.p, s)) return -1;
+        if (L.ptab) restrict_tab_launch<T>(G, L, (const T *)L.r.p, C.b.p, xz, s);
+        else restrict_launch<T>(G, (const T *)L.r.p, C.b.p, xz, s);
     }
     T *ccur = C.x.p;
-    if (vcycle(t, mg, k - 1, ccur, s)) return -1;
-    // with fused sweeps the first post-smoothing sweep adds the prolongated correction itself; FP64 levels
-    // above 2^20 points keep the separate prolongation (at 515^2 x 10 the coarse window takes the FP64
-    // sweep tile from 50 to 57 KiB of LDS, two blocks per CU instead of three: 0.55 ms per RK4 step slower)
-    if (L.ptab && t->fused_rb && t->cfg.nu2 >= 1 && L.args.dim3 && (sizeof(T) == 4 || L.args.spec)) {
-        const ProArgs<T> P{(const T *)ccur, L.pxi.p, L.pyi.p, L.pxw.p, L.pyw.p, C.g.nxg};
-        const int rc = smooth(t, L, t->cfg.nu2, cur, s, nullptr, uout, &P);
-        if (rc <= 0) return rc;
+    if (vcycle<T>(t, mg, k - 1, C.b.p, ccur, s)) return -1;
+    // with fused sweeps the first post-smoothing sweep adds the prolongated correction itself
+    if (L.ptab && t->fused_rb && t->cfg.nu2 >= 1 && L.args.dim3) {
+        const ProArgs<T> P{(const T *)ccur, L.pxw.p, L.pyw.p, C.g.nxg, 0};
+        return smooth<T>(t, L, b, t->cfg.nu2, cur, s, nullptr, uout, &P, false, top);
     }
     if (L.ptab) prolong_tab_launch<T>(G, L, (const T *)ccur, cur, s);
     else prolong_launch<T>(G, (const T *)ccur, cur, s);
-    if (smooth(t, L, t->cfg.nu2, cur, s, nullptr, uout)) return -1;
+    if (smooth<T>(t, L, b, t->cfg.nu2, cur, s, nullptr, uout, nullptr, false, top)) return -1;
     return 0;
 }
 
@@ -619,12 +629,16 @@ int precond_body(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, con
     // x = 0 itself; otherwise one pass does it first
     const bool fused = t->fused_rb && top >= 1 && top != t->bot_top;
     const bool fuse_in = fused && t->cfg.nu1 >= 1, fuse_out = fused && u && t->cfg.nu2 >= 1;
+    // FP64: r itself is the finest level's right-hand side (needs_b; r stays unchanged through the application)
+    const T *b = F.b.p;
+    if constexpr (std::is_same<T, double>::value) { if (!b && fuse_in) b = r; }
+    if (!b) { err() = "multigrid level has no right-hand side"; return -1; }
     if (!fuse_in)
         hipLaunchKernelGGL((k_precond_in<T>), dim3(grid_blocks(n)), dim3(256), 0, s, n, r, F.b.p, F.x.p, t->done());
     T *cur = F.x.p;
     const int cycles = t->nlev == 1 ? 1 : std::max(1, t->cfg.maxit);
     for (int it = 0; it < cycles; it++) {
-        if (vcycle<T>(t, mg, top, cur, s, (fuse_in && it == 0) ? r : nullptr, (fuse_out && it == cycles - 1) ? u : nullptr)) return -1;
+        if (vcycle<T>(t, mg, top, b, cur, s, (fuse_in && it == 0) ? r : nullptr, (fuse_out && it == cycles - 1) ? u : nullptr)) return -1;
     }
     *out = fuse_out ? nullptr : cur;
     return 0;
