@@ -2166,6 +2166,51 @@ __device__ __forceinline__ void store_column(O *__restrict__ p, const T (&v)[NZ]
     }
 }
 
+// A window of ROWS x COLS columns between HBM and LDS by rows: a thread takes the same piece (two values of a column
+// where NZ is even) of every row (of every GR-th row with GR row groups), so that its addresses differ by a constant
+// and each row is one contiguous segment.
+template <typename S, int NZ, int ROWS, int COLS, int NT, int GR = 1>
+struct RowWindow {
+    static constexpr int E = NZ % 2 == 0 ? 2 : 1, CH = COLS * NZ / E, NG = NT / GR, PER = (CH + NG - 1) / NG, RG = (ROWS + GR - 1) / GR;
+    S v[RG][PER][E];
+    __device__ __forceinline__ void load(const S *__restrict__ src, size_t pitch, int rows, int cols) {
+        const int t = GR == 1 ? (int)threadIdx.x : (int)threadIdx.x % NG, g = GR == 1 ? 0 : (int)threadIdx.x / NG;
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+            const int e = (t + p * NG) * E;
+            const bool in = e < cols * NZ;
+#pragma unroll
+            for (int q = 0; q < RG; q++) {
+                const int r = q * GR + g;
+                if (!in || r >= rows) continue;
+                if constexpr (E == 2) {
+                    const ColPair<S> w = *reinterpret_cast<const ColPair<S> *>(src + (size_t)r * pitch + e);
+                    v[q][p][0] = w.a; v[q][p][1] = w.b;
+                } else {
+                    v[q][p][0] = src[(size_t)r * pitch + e];
+                }
+            }
+        }
+    }
+    template <int NZP, int RS, typename T>
+    __device__ __forceinline__ void store(T *lds, int rows, int cols) const {
+        const int t = GR == 1 ? (int)threadIdx.x : (int)threadIdx.x % NG, g = GR == 1 ? 0 : (int)threadIdx.x / NG;
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+            const int e = (t + p * NG) * E, c = e / NZ, k = e - c * NZ;
+            if (e >= cols * NZ) continue;
+            T *d = lds + c * NZP + k;
+#pragma unroll
+            for (int q = 0; q < RG; q++) {
+                const int r = q * GR + g;
+                if (r >= rows) continue;
+#pragma unroll
+                for (int m = 0; m < E; m++) d[r * RS * NZP + m] = (T)v[q][p][m];
+            }
+        }
+    }
+};
+
 // Line system of an interior column (two columns or more from every wall) on a uniform horizontal grid: the
 // matrix rows, and the right-hand side with the neighbours' terms.  Each mixed-derivative coupling is
 // 2 s2 cx1 sum_m Z1[m] (x[i+1] - x[i-1]) on the three sigma levels around k (the centre weight of the first
@@ -2761,45 +2806,6 @@ __global__ __launch_bounds__((SweepTile<NZ, TX, TY>::NT)) void k_mg_sweep(LvArgs
 }
 
 
-// A window of ROWS x COLS columns between HBM and LDS by rows: a thread takes the same piece (two values of a column
-// where NZ is even) of every row, so that its addresses differ by a constant and each row is one contiguous segment.
-template <typename S, int NZ, int ROWS, int COLS, int NT>
-struct RowWindow {
-    static constexpr int E = NZ % 2 == 0 ? 2 : 1, CH = COLS * NZ / E, PER = (CH + NT - 1) / NT;
-    S v[ROWS][PER][E];
-    __device__ __forceinline__ void load(const S *__restrict__ src, size_t pitch, int rows, int cols) {
-#pragma unroll
-        for (int p = 0; p < PER; p++) {
-            const int e = ((int)threadIdx.x + p * NT) * E;
-            const bool in = e < cols * NZ;
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                if (!in || r >= rows) continue;
-                if constexpr (E == 2) {
-                    const ColPair<S> w = *reinterpret_cast<const ColPair<S> *>(src + (size_t)r * pitch + e);
-                    v[r][p][0] = w.a; v[r][p][1] = w.b;
-                } else {
-                    v[r][p][0] = src[(size_t)r * pitch + e];
-                }
-            }
-        }
-    }
-    template <int NZP, int RS, typename T>
-    __device__ __forceinline__ void store(T *lds, int rows, int cols) const {
-#pragma unroll
-        for (int p = 0; p < PER; p++) {
-            const int e = ((int)threadIdx.x + p * NT) * E, c = e / NZ, k = e - c * NZ;
-            if (e >= cols * NZ) continue;
-            T *d = lds + c * NZP + k;
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                if (r >= rows) continue;
-#pragma unroll
-                for (int q = 0; q < E; q++) d[r * RS * NZP + q] = (T)v[r][p][q];
-            }
-        }
-    }
-};
 // rows x cols columns from LDS to HBM the same way.
 template <int NZ, int ROWS, int COLS, int NT, int NZP, int RS, typename T, typename O>
 __device__ __forceinline__ void store_rows(O *__restrict__ dst, size_t pitch, const T *lds, int rows, int cols) {
@@ -3319,33 +3325,100 @@ __global__ void k_mg_restrict_tab(RestrictGeo G, const T *__restrict__ rxw, cons
     rc[q] = v;
 }
 
-// LDS elements of k_mg_residual_restrict's window (x, then the residual tile over it), coefficients and
-// restriction weights.
+// Residual of a column of a 3D level from its rows (residual_column's arithmetic, its roundings written out): c its
+// level 0 in LDS, x- and y-neighbours at +- SXS and +- SYS; i, j the column (wall columns take the rows of the
+// column beside them).
+template <typename T, int NZ, int SXS, int SYS>
+__device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, const LineRows<T, true> &R, const T (&cp)[6], const T *c,
+                                              const T (&b)[NZ], T (&o)[NZ]) {
+#pragma clang fp contract(off)
+    auto dot3 = [](const T (&S)[3], T a, T m, T z) -> T {
+#pragma clang fp contract(off)
+        return fma1(S[2], z, fma1(S[0], a, S[1] * m));
+    };
+    const int nxg = L.nxg, nyg = L.nyg;
+    const bool wx = i == 0 || i == nxg - 1, wy = j == 0 || j == nyg - 1;
+    if (wx || wy) {
+        // identity at corners and on the sigma ghost level, else the Neumann row of the column beside the wall
+        const int st = wx ? SXS : SYS, c0 = wx ? (i == 0 ? 0 : -2) : (j == 0 ? 0 : -2);
+        T S[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) S[m] = pick(wx, R.X1[m], R.Y1[m]);
+#pragma unroll
+        for (int k = 0; k < NZ; k++) {
+            const T *q = c + c0 * st + k;
+            o[k] = (wx && wy) || k == 0 ? b[k] - c[k] : b[k] - dot3(S, q[0], q[st], q[2 * st]);
+        }
+        return;
+    }
+    T xc[NZ], dxl[NZ], dyl[NZ], xx[NZ];
+#pragma unroll
+    for (int k = 0; k < NZ; k++) {
+        const T xm = c[k - SXS], xp = c[k + SXS], ym = c[k - SYS], yp = c[k + SYS];
+        xc[k] = c[k];
+        dxl[k] = dot3(R.X1, xm, xc[k], xp);
+        dyl[k] = dot3(R.Y1, ym, xc[k], yp);
+        if (k > 0 && k < NZ - 1) xx[k] = dot3(R.X2, xm, xc[k], xp) + dot3(R.Y2, ym, xc[k], yp);
+    }
+    // beside a wall the first derivative on the sigma ghost level takes the window shifted one column inwards
+    if (i == 1 || i == nxg - 2) {
+        const T *q = c + (i == 1 ? 0 : -2) * SXS;
+        dxl[0] = dot3(R.XW, q[0], q[SXS], q[2 * SXS]);
+    }
+    if (j == 1 || j == nyg - 2) {
+        const T *q = c + (j == 1 ? 0 : -2) * SYS;
+        dyl[0] = dot3(R.YW, q[0], q[SYS], q[2 * SYS]);
+    }
+    o[NZ - 1] = b[NZ - 1] - xc[NZ - 1];
+#pragma unroll
+    for (int k = 1; k < NZ - 1; k++) {
+        const T *Z = L.sz + k * 6;
+        const T Z1[3] = {Z[0], Z[1], Z[2]}, Z2[3] = {Z[3], Z[4], Z[5]};
+        const T om = T(1) - L.zs[k];
+        const T s2 = om * cp[3], s4 = om * cp[4], s3 = om * cp[5], s5 = cp[0];
+        const T dz = dot3(Z1, xc[k - 1], xc[k], xc[k + 1]), dzz = dot3(Z2, xc[k - 1], xc[k], xc[k + 1]);
+        const T dxz = dot3(Z1, dxl[k - 1], dxl[k], dxl[k + 1]), dyz = dot3(Z1, dyl[k - 1], dyl[k], dyl[k + 1]);
+        const T mixed = fma1(s2, dxz, s4 * dyz), czz = fma1(s5, s5, fma1(s2, s2, s4 * s4));
+        o[k] = b[k] - fma1(czz, dzz, fma1(T(2), mixed, fma1(s3, dz, xx[k])));
+    }
+    {
+        const T *Z = L.sz + 6;
+        const T Z1[3] = {Z[0], Z[1], Z[2]};
+        const T om = T(1) - L.zs[1];
+        const T s2 = om * cp[3], s4 = om * cp[4], s5 = cp[0], hx = cp[1], hy = cp[2];
+        const T dz = dot3(Z1, xc[0], xc[1], xc[2]), cz = fma1(hy, s4, fma1(hx, s2, s5));
+        o[0] = b[0] - fma1(hy, dyl[1], fma1(cz, dz, hx * dxl[1]));
+    }
+}
+
+// LDS elements of k_mg_residual_restrict: the x window, then the residual tile over it.
 template <int NZ, int CX, int CY>
 struct ResRestrictLds {
     static constexpr int FW = 2 * CX + 1, FH = 2 * CY + 1, WX = FW + 4, WY = FH + 4, NZP = NZ | 1;
-    static constexpr int X = WX * WY * NZP, C = CoefLds<WX, WY, NZ>::TOTAL, W = 4 * (CX + CY);
-    static constexpr int TOTAL = X + C + W;
+    static constexpr int TOTAL = WX * WY * NZP;
 };
 // Residual of a level and its restriction onto a coarse level coarsened in x and y but not in sigma, in one
 // launch (k_mg_residual_t followed by k_mg_restrict_tab, same arithmetic).  A block owns CX x CY coarse
-// columns (ghost columns included); it computes the fine residual (residual_column) on the (2 CX + 1) x
-// (2 CY + 1) fine columns their restriction stencils reach, one thread per column (the fine column between
-// two tiles is computed by both), keeps it in LDS over the staged x window and restricts from there, so the
-// fine residual never goes to HBM.  Also clears the coarse iterate.  Requires wall ghost layers in x and y
-// (gx = gy = 1), as every level with restriction tables has.
+// columns (ghost columns included); it computes the fine residual on the (2 CX + 1) x (2 CY + 1) fine columns
+// their restriction stencils reach, one thread per column (the fine column between two tiles is computed by
+// both), keeps it in LDS over the staged x window and restricts from there, so the fine residual never goes
+// to HBM.  Requires wall ghost layers in x and y (gx = gy = 1), as every level with restriction tables has.
+// A thread's right-hand side, planes and stencil rows go straight to its registers: staging them in LDS by
+// element took more instructions than the residual itself.  The barriers wait for LDS only, not for the loads in
+// flight.  With 10 sigma levels, everything staged in LDS and then as here: FP32 at 513 x 513 columns 19.9 us
+// before, 13.8 us after (bound by the instructions of the residual); at 257 x 257 10.2 and 7.4 us; on a level of
+// one or two tiles 8.9 and 6.3 us (the chain load, residual, barrier, restriction, store).  FP64: 43.8 and
+// 21.9 us, 17.9 and 10.0 us, 9.8 and 7.5 us.
 template <typename T, int NZ, int CX, int CY, int NT>
 __global__ __launch_bounds__(NT) void k_mg_residual_restrict(LvArgs<T> L, RestrictGeo G, const T *__restrict__ rxw, const T *__restrict__ ryw,
                                                              const T *__restrict__ x, const T *__restrict__ b, T *__restrict__ rc,
                                                              T *__restrict__ xz) {
+#pragma clang fp contract(off)
     if (!L.spec && solve_done(L.skip)) return;
     using S = ResRestrictLds<NZ, CX, CY>;
-    constexpr int FW = S::FW, FH = S::FH, WX = S::WX, WY = S::WY, NZP = S::NZP, R = 2;
+    constexpr int FW = S::FW, FH = S::FH, WX = S::WX, WY = S::WY, NZP = S::NZP, R = 2, RES = (CY * CX * NZ + NT - 1) / NT;
     static_assert(FW * FH <= NT, "one thread per fine column of the tile");
-    static_assert(4 * (CX + CY) <= NT, "one weight per thread");
-    __shared__ T sX[S::X];
-    __shared__ T sC[S::C];
-    __shared__ T sW[S::W];
+    __shared__ T sX[S::TOTAL];
     const int nxg = L.nxg, nyg = L.nyg, t = (int)threadIdx.x;
     // XCD-aware tile order (xcd_tile over the row-major tile index): each XCD takes one contiguous band of
     // tile rows, so the halos neighbouring tiles share are re-read from that XCD's L2 (at 513^2: HBM fetch
@@ -3359,65 +3432,68 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(LvArgs<T> L, Restri
     const int tx = t % FW, ty = t / FW;
     const int i = fi0 + tx, j = fj0 + ty;
     const bool active = t < FW * FH && i >= 0 && i < nxg && j >= 0 && j < nyg;
-    // every HBM load of the block (coefficients, x window, the thread's column of b, the tile's restriction
-    // weights) is in flight before the first wait
-    T bc[NZ];
-    const T *bp = b + (active ? (size_t)i + (size_t)nxg * j : (size_t)0) * NZ;
-#pragma unroll
-    for (int k = 0; k < NZ; k++) bc[k] = active ? bp[k] : T(0);
-    T w = T(0);
-    if (t < 4 * CX) {
-        if (ic0 + t / 4 < G.nxgc) w = rxw[4 * ic0 + t];
-    } else if (t < 4 * (CX + CY)) {
-        if (jc0 + (t - 4 * CX) / 4 < G.nygc) w = ryw[4 * jc0 + t - 4 * CX];
-    }
-    CoefRegs<T, NZ, WX, WY, NT> cr;
-    WindowRegs<T, NZ, WY, WX, NT> xr;
-    cr.load(L, lox, loy, wcols, wrows);
+    // every HBM load of the block is in flight before the first wait
+    RowWindow<T, NZ, WY, WX, NT, (WX * NZ / 2 <= NT / 2) ? 2 : 1> xr;
     xr.load(x + ((size_t)loy * nxg + lox) * NZ, (size_t)nxg * NZ, wrows, wcols);
+    T bc[NZ], cp[6];
+    LineRows<T, true> rows;
+    {
+        const int ii = active ? i : 0, jj = active ? j : 0;   // (idle threads load a valid column)
+        const size_t p = (size_t)jj * nxg + ii;
+        load_column<NZ>(b + p * NZ, bc);
+#pragma unroll
+        for (int q = 0; q < 6; q++) cp[q] = L.col[(size_t)q * L.nxy + p];
+        rows.load(L, cclamp(ii, 1, nxg - 2), cclamp(jj, 1, nyg - 2));
+    }
+    // the thread's coarse points (CX * NZ contiguous values per coarse row) and their weights
+    struct Point { int cc, rr, k; T x[4], y[4]; } pt[RES];
+#pragma unroll
+    for (int q = 0; q < RES; q++) {
+        const int e = t + q * NT, c = e % (CX * NZ);
+        pt[q].rr = e / (CX * NZ); pt[q].cc = c / NZ; pt[q].k = c - pt[q].cc * NZ;
+        const int ic = cmin(ic0 + pt[q].cc, G.nxgc - 1), jc = cmin(jc0 + pt[q].rr, G.nygc - 1);
+#pragma unroll
+        for (int m = 0; m < 4; m++) { pt[q].x[m] = rxw[4 * ic + m]; pt[q].y[m] = ryw[4 * jc + m]; }
+    }
     if (L.spec && solve_done(L.skip)) return;
-    const CoefS<T> C = cr.store(sC);
     xr.template store<NZP, WX>(sX, wrows, wcols);
-    if (t < 4 * (CX + CY)) sW[t] = w;
-    __syncthreads();
-    auto X = [&](int k, int ii, int jj) -> T { return sX[((jj - loy) * WX + (ii - lox)) * NZP + k]; };
+    lds_barrier();
     T o[NZ];
-    if (active) residual_column<T, NZ>(L, C, i, j, X, bc, o);
-    __syncthreads();
+    if (active) residual_rows<T, NZ, NZP, WX * NZP>(L, i, j, rows, cp, sX + ((j - loy) * WX + (i - lox)) * NZP, bc, o);
+    lds_barrier();
     if (active) {
         T *dst = sX + (ty * FW + tx) * NZP;
 #pragma unroll
         for (int k = 0; k < NZ; k++) dst[k] = o[k];
     }
-    __syncthreads();
-    // restriction (k_mg_restrict_tab's arithmetic) of the tile's coarse points, CX * NZ contiguous values
-    // per coarse row
-    for (int e = t; e < CY * CX * NZ; e += NT) {
-        const int rr = e / (CX * NZ), c = e - rr * (CX * NZ), cc = c / NZ, k = c - cc * NZ;
-        const int ic = ic0 + cc, jc = jc0 + rr;
-        if (ic >= G.nxgc || jc >= G.nygc) continue;
-        const int icn = ic - 1, jcn = jc - 1;
+    lds_barrier();
+    // restriction (k_mg_restrict_tab's arithmetic)
+#pragma unroll
+    for (int q = 0; q < RES; q++) {
+        const Point &p = pt[q];
+        const int ic = ic0 + p.cc, jc = jc0 + p.rr;
+        if (t + q * NT >= CY * CX * NZ || ic >= G.nxgc || jc >= G.nygc) continue;
         T v = T(0);
-        if (k >= 1 && icn >= 0 && icn < G.nxc && jcn >= 0 && jcn < G.nyc) {
-            const int ti = 2 * cc + 1, tj = 2 * rr + 1;   // tile position of fine column (2 ic - 1, 2 jc - 1)
-            auto Rt = [&](int a, int bb) -> T { return sX[(bb * FW + a) * NZP + k]; };
-            if (k <= G.nzf - 1) {
-                const T x0 = sW[4 * cc], x1 = sW[4 * cc + 1], x2 = sW[4 * cc + 2], ax = sW[4 * cc + 3];
+        if (p.k >= 1 && ic >= 1 && ic <= G.nxc && jc >= 1 && jc <= G.nyc) {
+            const int ti = 2 * p.cc + 1, tj = 2 * p.rr + 1;   // tile position of fine column (2 ic - 1, 2 jc - 1)
+            auto Rt = [&](int a, int bb) -> T { return sX[(bb * FW + a) * NZP + p.k]; };
+            if (p.k <= G.nzf - 1) {
                 const int jf = 2 * jc - 1;
                 auto Xv = [&](int dj) -> T {
+#pragma clang fp contract(off)
                     const int jj = jf + dj;
-                    if (jj < 1 || jj > G.nyf) return Rt(ti, tj + dj);
-                    return ax * ((x0 * Rt(ti - 1, tj + dj) + x1 * Rt(ti, tj + dj)) + x2 * Rt(ti + 1, tj + dj));
+                    const T r1 = Rt(ti, tj + dj);
+                    const T s = p.x[3] * fma1(p.x[2], Rt(ti + 1, tj + dj), fma1(p.x[0], Rt(ti - 1, tj + dj), p.x[1] * r1));
+                    return jj < 1 || jj > G.nyf ? r1 : s;
                 };
-                const T *Y = sW + 4 * CX + 4 * rr;
-                v = Y[3] * ((Y[0] * Xv(-1) + Y[1] * Xv(0)) + Y[2] * Xv(1));
+                v = p.y[3] * fma1(p.y[2], Xv(1), fma1(p.y[0], Xv(-1), p.y[1] * Xv(0)));
             } else {
                 v = Rt(ti, tj);
             }
         }
-        const size_t q = ((size_t)jc * G.nxgc + ic) * NZ + k;
-        if (xz) xz[q] = T(0);
-        rc[q] = v;
+        const size_t d = ((size_t)jc * G.nxgc + ic) * NZ + p.k;
+        if (xz) xz[d] = T(0);
+        rc[d] = v;
     }
 }
 

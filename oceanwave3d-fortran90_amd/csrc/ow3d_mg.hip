@@ -14,9 +14,7 @@ bool needs_b(const ow3d_tank *t, int k) {
     return !(k == top && top >= 1 && t->cfg.mg_precision == 0 && t->fused_rb && t->cfg.nu1 >= 1 && t->bot_lim == 0);
 }
 bool needs_r(const ow3d_tank *t, int k) {
-    // (the one-launch residual and restriction of 14 FP64 values a column exceeds 64 KiB of LDS)
-    const bool fits = t->cfg.mg_precision != 0 || t->levels[k].nzg < 14;
-    return t->bot_lim > 0 || (k > 0 && !(fits && plane_coarsened(t->levels[k], t->levels[k - 1])));
+    return t->bot_lim > 0 || (k > 0 && !plane_coarsened(t->levels[k], t->levels[k - 1]));
 }
 
 // Multigrid hierarchy of the tank (MGPreProcess.f90:6-460 with coarsening strategy 0), level operators in

@@ -415,18 +415,15 @@ void restrict_tab_launch(const RestrictGeo &G, const MgLevel<T> &F, const T *rf,
     }
     hipLaunchKernelGGL((k_mg_restrict<T>), dim3(grid_blocks((size_t)G.nxgc * G.nygc * G.nzgc)), dim3(256), 0, s, G, rf, rc, xz);
 }
-// Residual of level F and its restriction in one launch (k_mg_residual_restrict, F.ptab levels), for the
-// column depths whose tile fits 64 KiB of LDS; false otherwise (the caller then launches the two).  Coarse
-// tiles of 8 x 7 columns: 17 x 15 fine columns, one per thread of 256.
+// Residual of level F and its restriction in one launch (k_mg_residual_restrict, F.ptab levels); false where it does not
+// apply (the caller then launches the two).  Coarse tiles of 8 x 7 columns: 17 x 15 fine columns, one per thread of 256.
 template <typename T, int NZ>
 bool resrestrict_nz(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
     constexpr int CX = 8, CY = 7;
-    if constexpr (ResRestrictLds<NZ, CX, CY>::TOTAL * sizeof(T) <= 65536) {
-        hipLaunchKernelGGL((k_mg_residual_restrict<T, NZ, CX, CY, 256>), dim3((G.nxgc + CX - 1) / CX, (G.nygc + CY - 1) / CY), dim3(256), 0, s,
-                           F.args, G, (const T *)F.rxw.p, (const T *)F.ryw.p, x, b, rc, xz);
-        return true;
-    }
-    return false;
+    static_assert(ResRestrictLds<NZ, CX, CY>::TOTAL * sizeof(T) <= 65536, "residual tile exceeds 64 KiB of LDS");
+    hipLaunchKernelGGL((k_mg_residual_restrict<T, NZ, CX, CY, 256>), dim3((G.nxgc + CX - 1) / CX, (G.nygc + CY - 1) / CY), dim3(256), 0, s,
+                       F.args, G, (const T *)F.rxw.p, (const T *)F.ryw.p, x, b, rc, xz);
+    return true;
 }
 template <typename T>
 bool resrestrict_launch(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
