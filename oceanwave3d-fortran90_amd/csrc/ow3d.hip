@@ -1060,6 +1060,7 @@ extern "C" long long ow3d_estimate_bytes(const ow3d_config *cfg) {
         ow3d_tank probe;   // the hierarchy and the settings that needs_b and needs_r read
         probe.cfg = *cfg;
         probe.levels = lev;
+        probe.bot_top = bottom_top(&probe);
         for (size_t k = 0; k < lev.size(); k++) {
             const Grid &L = lev[k];
             b += p * ((long long)L.n * (2 + needs_b(&probe, (int)k) + needs_r(&probe, (int)k)) + 6LL * L.nxy + 12LL * (L.nxg + L.nyg + L.nzg)) + 8LL * (L.nxg + L.nyg + L.nzg);

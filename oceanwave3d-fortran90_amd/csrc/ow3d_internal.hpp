@@ -111,6 +111,31 @@ size_t line_records(int nxg, int nyg, int nzg) {
     return n * LineRecord<T, 3>::count(nxg, nyg);
 }
 
+// k_mg_bottom on levels 0 .. top: values of its tables at most, and LDS elements of the iterate and right-hand side of each
+// level (columns padded to an odd stride above level 0), the finest one's residual and the tables, whose offsets go to
+// A (unless NULL).
+inline size_t bottom_tables(const std::vector<Grid> &lv, int top) {
+    size_t n = 0;
+    for (int k = 1; k <= top; k++)   // rows 6, prolongation 3, restriction 4 (coarse) per column and row; 3 and 3 per level
+        n += (size_t)9 * (lv[k].nxg + lv[k].nyg) + 4 * (lv[k - 1].nxg + lv[k - 1].nyg) + 3 * (lv[k].nzg + lv[k - 1].nzg);
+    return n;
+}
+template <typename T>
+size_t bottom_layout(const std::vector<Grid> &lv, int top, BottomArgs<T> *A) {
+    size_t off = 0;
+    auto take = [&](size_t n) { const size_t o = off; off += (n + 3) / 4 * 4; return (int)o; };
+    size_t ntop = 0;
+    for (int k = top; k >= 0; k--) {
+        const size_t xy = (size_t)lv[k].nxg * lv[k].nyg, n = k ? xy * (lv[k].nzg | 1) : (lv[0].n + 7) / 8 * 8;
+        if (k == top) ntop = n;
+        const int x = take(n), b = take(n);
+        if (A) { A->lev[k].x = x; A->lev[k].b = b; }
+    }
+    const int image = (int)off, r = take(ntop), tab = take(bottom_tables(lv, top));
+    if (A) { A->image = image; A->r = r; A->tab = tab; }
+    return off;
+}
+
 inline int grid_blocks(size_t n, int bs = 256) {
     size_t b = (n + bs - 1) / bs;
     return (int)std::min<size_t>(std::max<size_t>(b, 1), 65535 * 16);
@@ -146,7 +171,10 @@ struct ow3d_tank {
     std::vector<Grid> levels;
     std::vector<std::unique_ptr<MgLevel<double>>> mg64;
     std::vector<std::unique_ptr<MgLevel<float>>> mg32;
-    long bot_lim = 0;                 // points a level handed to the one-workgroup bottom kernel may have (0: off)
+    long bot_lim = 1 << 20;           // points a level handed to the one-workgroup bottom kernel may have (0: off)
+    size_t bot_lds = 0;               // LDS bytes of that kernel
+    bool bot_split = false;           // the dense solve is a launch of its own between its two parts
+    DevBuf<double> bot_tab, bot_img;  // its tables, and its LDS image between the parts
     int bot_top = -1;                 // finest level handled by the one-workgroup bottom kernel (-1: none)
     bool fused_rb = true;             // one launch per zebra sweep (red and black halves) on the upper levels
     // launch choices (ow3d_tune): matvec variant 0 column kernel, widest tile / 1 column kernel, 8-row
@@ -209,7 +237,9 @@ int launch_matvec(const ow3d_tank *t, const double *phi, double *y, hipStream_t 
 bool matvec_supported(int nzg, int A);
 // multigrid (ow3d_mg.hip): hierarchy set-up for t->cfg and u = M^-1 r on device vectors
 int mg_setup(ow3d_tank *t);
-// Buffers of level k that some path uses (t->levels, t->fused_rb and t->bot_lim are set): the right-hand side, except
+int bottom_top(const ow3d_tank *t);   // t->bot_top from t->levels and the settings
+bool bottom_split(const ow3d_tank *t);   // t->bot_split
+// Buffers of level k that some path uses (t->levels, t->fused_rb and t->bot_top are set): the right-hand side, except
 // on an FP64 finest level whose first sweep reads the residual itself, and the residual, except where it goes into its
 // restriction in one launch.
 bool needs_b(const ow3d_tank *t, int k);

@@ -1635,6 +1635,7 @@ struct LvArgs {
     int uni;
     T cx1, cx2, cxc, cy1, cy2, cyc;
     const T *fac;           // records of the columns (LineRecord); nullptr: the sweep forms their line matrices
+    int facq;               // 0: a record's values are contiguous; else its 16-byte chunk q is chunk q * facq + r of fac
 };
 
 // Level coefficients as the column kernels read them: 3-point stencil rows sx(i), sy(j), sz(k) (first then
@@ -2063,10 +2064,6 @@ __device__ __forceinline__ void ghost_point(const LvArgs<T> &L, int t, T *__rest
     }
     x[q] = (b[q] - s) / dg;
 }
-template <typename T>
-__device__ __forceinline__ int ghost_count(const LvArgs<T> &L) {
-    return (L.dim3 ? 2 * L.nxg + 2 * (L.nyg - 2) : 2) * L.nzg;
-}
 
 // Column index c of the sweep colour -> (i, j); false past the last column of that colour.
 template <typename T>
@@ -2248,8 +2245,9 @@ __device__ __forceinline__ void line_matrix_uniform(const LvArgs<T> &L, const T 
     }
 }
 // bw: the bottom row's weights of the west, east, south and north neighbour; c3, c4: h_x / h, h_y / h.
-template <typename T, int NZ, bool D3, int SXS, int SYS>
-__device__ __forceinline__ void line_rhs_uniform(const LvArgs<T> &L, T c3, T c4, const T (&bw)[4], const T *c, const T (&b)[NZ], T (&rh)[NZ]) {
+template <typename T, int NZ, bool D3, int SXS>
+__device__ __forceinline__ void line_rhs_uniform(const LvArgs<T> &L, T c3, T c4, const T (&bw)[4], const T *c, int SYS, const T (&b)[NZ],
+                                                 T (&rh)[NZ]) {
 #pragma clang fp contract(off)
     T sx[NZ], gx[NZ], sy[NZ], gy[NZ];   // sums and differences of the x- and y-neighbours
 #pragma unroll
@@ -2348,9 +2346,9 @@ __device__ __forceinline__ void line_matrix_general(const LvArgs<T> &L, int i, i
         lo[k] = a[0]; di[k] = a[1]; up[k] = a[2];
     }
 }
-template <typename T, int NZ, bool D3, int SXS, int SYS>
+template <typename T, int NZ, bool D3, int SXS>
 __device__ __forceinline__ void line_rhs_general(const LvArgs<T> &L, int i, int j, const LineRows<T, D3> &R, T c3, T c4, const T (&bw)[4],
-                                                 const T *c, const T (&b)[NZ], T (&rh)[NZ]) {
+                                                 const T *c, int SYS, const T (&b)[NZ], T (&rh)[NZ]) {
 #pragma clang fp contract(off)
     T XG[3], YG[3], xm[NZ], xp[NZ], ym[NZ], yp[NZ];
     R.ghost_level(R.X1, R.XW, i, L.nxg, XG);
@@ -2402,9 +2400,9 @@ __device__ __forceinline__ void line_rhs_general(const LvArgs<T> &L, int i, int 
 // line_rhs_general by two lanes per column, 32 apart: `hi` of them forms the upper half of the rows (half the time of
 // the longest path of a small level's sweep; the rows of a wall column are about three times an interior
 // column's).  The lower lanes receive all rows.
-template <typename T, int NZ, bool D3, int SXS, int SYS>
+template <typename T, int NZ, bool D3, int SXS>
 __device__ __forceinline__ void line_rhs_pair(const LvArgs<T> &L, int i, int j, bool hi, const LineRows<T, D3> &R, T c3, T c4, const T (&bw)[4],
-                                              const T *c, const T (&b)[NZ], T (&rh)[NZ]) {
+                                              const T *c, int SYS, const T (&b)[NZ], T (&rh)[NZ]) {
 #pragma clang fp contract(off)
     constexpr int HALF = (NZ - 1) / 2;   // of the NZ - 2 rows
     T XG[3], YG[3], xm[HALF + 2], xp[HALF + 2], ym[HALF + 2], yp[HALF + 2], r[HALF];
@@ -2499,12 +2497,13 @@ __global__ __launch_bounds__(256) void k_mg_factor(LvArgs<T> L, T *__restrict__ 
     if (edge || !L.uni) line_matrix_general<T, NZ, D3>(L, i, j, R, cp, lo, di, up, e2);
     else line_matrix_uniform<T, NZ, D3>(L, cp, R.X1, R.Y1, lo, di, up, e2);
     line_factor<T, NZ>(lo, di, up, e2, f, inv);
-    T *d = fac + Rec::index(L.nxg, L.nyg, i, j) * Rec::N;
+    const size_t r = Rec::index(L.nxg, L.nyg, i, j);
+    auto put = [&](int q, T v) { fac[L.facq ? ((size_t)(q / Rec::W) * L.facq + r) * Rec::W + q % Rec::W : r * Rec::N + q] = v; };
 #pragma unroll
-    for (int k = 0; k < NZ - 1; k++) { d[k] = f[k]; d[NZ - 1 + k] = up[k]; d[2 * NZ - 2 + k] = inv[k]; }
-    d[Rec::C3] = cp[3]; d[Rec::C4] = cp[4];
-    d[Rec::BW] = cp[1] * R.X1[0]; d[Rec::BW + 1] = cp[1] * R.X1[2];
-    d[Rec::BW + 2] = D3 ? cp[2] * R.Y1[0] : T(0); d[Rec::BW + 3] = D3 ? cp[2] * R.Y1[2] : T(0);
+    for (int k = 0; k < NZ - 1; k++) { put(k, f[k]); put(NZ - 1 + k, up[k]); put(2 * NZ - 2 + k, inv[k]); }
+    put(Rec::C3, cp[3]); put(Rec::C4, cp[4]);
+    put(Rec::BW, cp[1] * R.X1[0]); put(Rec::BW + 1, cp[1] * R.X1[2]);
+    put(Rec::BW + 2, D3 ? cp[2] * R.Y1[0] : T(0)); put(Rec::BW + 3, D3 ? cp[2] * R.Y1[2] : T(0));
 }
 
 // Prolongation fused into the first post-smoothing sweep of a level with interpolation tables
@@ -2730,13 +2729,13 @@ __global__ __launch_bounds__((SweepTile<NZ, TX, TY>::NT)) void k_mg_sweep(LvArgs
 #pragma unroll
                 for (int k = 0; k < NZ; k++) rh[k] = c.b[k];
             } else if (!edge && L.uni) {
-                line_rhs_uniform<T, NZ, D3, SXS, SYS>(L, c3, c4, bw, d, c.b, rh);
+                line_rhs_uniform<T, NZ, D3, SXS>(L, c3, c4, bw, d, SYS, c.b, rh);
             } else if (PAIR && edge) {
-                line_rhs_pair<T, NZ, D3, SXS, SYS>(L, c.i, c.j, upper, c.R, c3, c4, bw, d, c.b, rh);
+                line_rhs_pair<T, NZ, D3, SXS>(L, c.i, c.j, upper, c.R, c3, c4, bw, d, SYS, c.b, rh);
             } else {
                 LineRows<T, D3> R = c.R;
                 if (!edge) R.load(L, c.i, c.j);
-                line_rhs_general<T, NZ, D3, SXS, SYS>(L, c.i, c.j, R, c3, c4, bw, d, c.b, rh);
+                line_rhs_general<T, NZ, D3, SXS>(L, c.i, c.j, R, c3, c4, bw, d, SYS, c.b, rh);
             }
             line_solve<T, NZ>(f, up, inv, rh, x);
             if (!upper) {
@@ -3001,9 +3000,9 @@ __global__ __launch_bounds__((TiledSweep<NZ, TX, TY>::NT)) void k_mg_sweep_tiled
 #pragma unroll
             for (int k = 0; k < NZ; k++) rh[k] = bc[k];
         } else if (EDGE || !L.uni) {
-            line_rhs_general<T, NZ, true, SXS, SYS>(L, i, j, R, cp[3], cp[4], bw, d, bc, rh);
+            line_rhs_general<T, NZ, true, SXS>(L, i, j, R, cp[3], cp[4], bw, d, SYS, bc, rh);
         } else {
-            line_rhs_uniform<T, NZ, true, SXS, SYS>(L, cp[3], cp[4], bw, d, bc, rh);
+            line_rhs_uniform<T, NZ, true, SXS>(L, cp[3], cp[4], bw, d, SYS, bc, rh);
         }
         line_solve<T, NZ>(f, up, inv, rh, x);
 #pragma unroll
@@ -3135,13 +3134,12 @@ struct RestrictGeo {
     const int *skip;                                 // solve_done flag (nullptr: always run)
     int spec;                                        // 1: loads are issued before skip is tested
 };
-// Restricted residual at coarse point (kc, ic, jc) (0 on ghost points).
-template <typename T>
-__device__ __forceinline__ T restrict_at(const RestrictGeo &G, int kc, int ic, int jc, const T *__restrict__ rf) {
+// Restricted residual at coarse point (kc, ic, jc) (0 on ghost points), the residual read through R(k, i, j).
+template <typename T, class RA>
+__device__ __forceinline__ T restrict_at(const RestrictGeo &G, int kc, int ic, int jc, const RA &R) {
     const int icn = ic - G.gx, jcn = jc - G.gy;
     if (kc < 1 || icn < 0 || icn >= G.nxc || jcn < 0 || jcn >= G.nyc) return T(0);
     const int kf = 1 + (kc - 1) * (1 + G.zc), ifn = G.gx + icn * (1 + G.xc), jfn = G.gy + jcn * (1 + G.yc);
-    auto R = [&](int k, int i, int j) -> T { return rf[(size_t)(j * G.nxgf + i) * G.nzgf + k]; };
     // x pass value at (k,i,j)
     auto Xv = [&](int k, int i, int j) -> T {
         if (G.xc && k >= 1 && k <= G.nzf - 1 && j >= G.gy && j <= G.nyf + G.gy - 1 && ((i - G.gx) % 2 == 0) && i >= G.gx && i <= G.nxf + G.gx - 1) {
@@ -3173,15 +3171,8 @@ template <typename T>
 __device__ __forceinline__ T restrict_value(const RestrictGeo &G, size_t q, const T *__restrict__ rf) {
     const int kc = (int)(q % G.nzgc);
     const size_t col = q / G.nzgc;
-    return restrict_at(G, kc, (int)(col % G.nxgc), (int)(col / G.nxgc), rf);
-}
-// Coarse point q; also clears the coarse iterate xz where the coarse level's sweep reads it (nullptr otherwise).
-template <typename T>
-__device__ __forceinline__ void restrict_point(const RestrictGeo &G, size_t q, const T *__restrict__ rf, T *__restrict__ rc, T *__restrict__ xz) {
-    const size_t nc = (size_t)G.nxgc * G.nygc * G.nzgc;
-    if (q >= nc) return;
-    if (xz) xz[q] = T(0);
-    rc[q] = restrict_value(G, q, rf);
+    auto R = [&](int k, int i, int j) -> T { return rf[(size_t)(j * G.nxgf + i) * G.nzgf + k]; };
+    return restrict_at<T>(G, kc, (int)(col % G.nxgc), (int)(col / G.nxgc), R);
 }
 template <typename T>
 __global__ void k_mg_restrict(RestrictGeo G, const T *__restrict__ rf, T *__restrict__ rc, T *__restrict__ xz) {
@@ -3201,7 +3192,8 @@ __global__ void k_mg_restrict_t(RestrictGeo G, const T *__restrict__ rf, T *__re
     const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (t >= G.nxgc * NZC) return;
     const int ic = t / NZC, kc = t - ic * NZC, jc = (int)blockIdx.y;
-    const T v = restrict_at(G, kc, ic, jc, rf);
+    auto R = [&](int k, int i, int j) -> T { return rf[(size_t)(j * G.nxgf + i) * G.nzgf + k]; };
+    const T v = restrict_at<T>(G, kc, ic, jc, R);
     if (G.spec && solve_done(G.skip)) return;
     const size_t q = (size_t)jc * G.nxgc * NZC + t;
     if (xz) xz[q] = T(0);
@@ -3211,11 +3203,11 @@ __global__ void k_mg_restrict_t(RestrictGeo G, const T *__restrict__ rf, T *__re
 // Prolongation (MGProlongation3DExplicit.f90) of the coarse correction, added to x on interior
 // columns below the free surface.
 // Interpolated correction at fine point q < nxgf * nygf * nzgf; false where q takes none (ghost points,
-// the sigma ghost level and the surface).
+// the sigma ghost level and the surface).  The coarse correction is read through E(kc, ic, jc).
 // (The factors XF, YF, ZF are 1 or 2: x % F is x & (F - 1) and x / F is x >> (F - 1) on the
 // non-negative offsets they are applied to.)
-template <typename T>
-__device__ __forceinline__ bool prolong_at(const RestrictGeo &G, int k, int i, int j, const T *__restrict__ ec, T &out) {
+template <typename T, class EA>
+__device__ __forceinline__ bool prolong_at(const RestrictGeo &G, int k, int i, int j, const EA &E, T &out) {
     if (k < 1 || k > G.nzf - 1 || i < G.gx || i > G.nxf + G.gx - 1 || j < G.gy || j > G.nyf + G.gy - 1) return false;
     const int XF = G.xc ? 2 : 1, YF = G.yc ? 2 : 1, ZF = G.zc ? 2 : 1;
     const int xs = G.xc ? 1 : 0, ys = G.yc ? 1 : 0, zs = G.zc ? 1 : 0;
@@ -3224,7 +3216,7 @@ __device__ __forceinline__ bool prolong_at(const RestrictGeo &G, int k, int i, i
         if (((ii - G.gx) & xs) != 0 || ((jj - G.gy) & ys) != 0) return T(0);
         const int kc = 1 + ((kk - 1) >> zs), ic = G.gx + ((ii - G.gx) >> xs), jc = G.gy + ((jj - G.gy) >> ys);
         if (kc > G.nzc - 1) return T(0);
-        return ec[(size_t)(jc * G.nxgc + ic) * G.nzgc + kc];
+        return E(kc, ic, jc);
     };
     auto EX = [&](int kk, int ii, int jj) -> T {
         if (XF == 2 && ((jj - G.gy) & ys) == 0 && ((ii - G.gx) % 2) == 1 && kk >= 1 && kk <= G.nzf - 1 && ((kk - 1) & zs) == 0) {
@@ -3256,13 +3248,8 @@ template <typename T>
 __device__ __forceinline__ bool prolong_value(const RestrictGeo &G, size_t q, const T *__restrict__ ec, T &out) {
     const int k = (int)(q % G.nzgf);
     const size_t col = q / G.nzgf;
-    return prolong_at(G, k, (int)(col % G.nxgf), (int)(col / G.nxgf), ec, out);
-}
-template <typename T>
-__device__ __forceinline__ void prolong_point(const RestrictGeo &G, size_t q, const T *__restrict__ ec, T *__restrict__ xf) {
-    if (q >= (size_t)G.nxgf * G.nygf * G.nzgf) return;
-    T e;
-    if (prolong_value(G, q, ec, e)) xf[q] = xf[q] + e;
+    auto E = [&](int kc, int ic, int jc) -> T { return ec[(size_t)(jc * G.nxgc + ic) * G.nzgc + kc]; };
+    return prolong_at<T>(G, k, (int)(col % G.nxgf), (int)(col / G.nxgf), E, out);
 }
 template <typename T>
 __global__ void k_mg_prolong_add(RestrictGeo G, const T *__restrict__ ec, T *__restrict__ xf) {
@@ -3284,7 +3271,8 @@ __global__ void k_mg_prolong_add_t(RestrictGeo G, const T *__restrict__ ec, T *_
     if (t >= G.nxgf * NZF) return;
     const int i = t / NZF, k = t - i * NZF, j = (int)blockIdx.y;
     T e;
-    if (!prolong_at(G, k, i, j, ec, e)) return;
+    auto E = [&](int kc, int ic, int jc) -> T { return ec[(size_t)(jc * G.nxgc + ic) * G.nzgc + kc]; };
+    if (!prolong_at<T>(G, k, i, j, E, e)) return;
     const size_t q = (size_t)j * G.nxgf * NZF + t;
     const T x0 = xf[q];
     if (G.spec && solve_done(G.skip)) return;
@@ -3325,11 +3313,11 @@ __global__ void k_mg_restrict_tab(RestrictGeo G, const T *__restrict__ rxw, cons
     rc[q] = v;
 }
 
-// Residual of a column of a 3D level from its rows (residual_column's arithmetic, its roundings written out): c its
-// level 0 in LDS, x- and y-neighbours at +- SXS and +- SYS; i, j the column (wall columns take the rows of the
+// Residual of a column from its rows (residual_column's arithmetic, its roundings written out): c its level 0 in
+// LDS, x- and y-neighbours at +- SXS and +- SYS; i, j the column (wall columns take the rows of the
 // column beside them).
-template <typename T, int NZ, int SXS, int SYS>
-__device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, const LineRows<T, true> &R, const T (&cp)[6], const T *c,
+template <typename T, int NZ, bool D3, int SXS>
+__device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, const LineRows<T, D3> &R, const T (&cp)[6], const T *c, int SYS,
                                               const T (&b)[NZ], T (&o)[NZ]) {
 #pragma clang fp contract(off)
     auto dot3 = [](const T (&S)[3], T a, T m, T z) -> T {
@@ -3337,13 +3325,16 @@ __device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, 
         return fma1(S[2], z, fma1(S[0], a, S[1] * m));
     };
     const int nxg = L.nxg, nyg = L.nyg;
-    const bool wx = i == 0 || i == nxg - 1, wy = j == 0 || j == nyg - 1;
+    const bool wx = i == 0 || i == nxg - 1, wy = D3 && (j == 0 || j == nyg - 1);
     if (wx || wy) {
         // identity at corners and on the sigma ghost level, else the Neumann row of the column beside the wall
         const int st = wx ? SXS : SYS, c0 = wx ? (i == 0 ? 0 : -2) : (j == 0 ? 0 : -2);
         T S[3];
 #pragma unroll
-        for (int m = 0; m < 3; m++) S[m] = pick(wx, R.X1[m], R.Y1[m]);
+        for (int m = 0; m < 3; m++) {
+            if constexpr (D3) S[m] = pick(wx, R.X1[m], R.Y1[m]);
+            else S[m] = R.X1[m];
+        }
 #pragma unroll
         for (int k = 0; k < NZ; k++) {
             const T *q = c + c0 * st + k;
@@ -3354,20 +3345,27 @@ __device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, 
     T xc[NZ], dxl[NZ], dyl[NZ], xx[NZ];
 #pragma unroll
     for (int k = 0; k < NZ; k++) {
-        const T xm = c[k - SXS], xp = c[k + SXS], ym = c[k - SYS], yp = c[k + SYS];
+        const T xm = c[k - SXS], xp = c[k + SXS];
         xc[k] = c[k];
         dxl[k] = dot3(R.X1, xm, xc[k], xp);
-        dyl[k] = dot3(R.Y1, ym, xc[k], yp);
-        if (k > 0 && k < NZ - 1) xx[k] = dot3(R.X2, xm, xc[k], xp) + dot3(R.Y2, ym, xc[k], yp);
+        dyl[k] = T(0);
+        if (k > 0 && k < NZ - 1) xx[k] = dot3(R.X2, xm, xc[k], xp);
+        if constexpr (D3) {
+            const T ym = c[k - SYS], yp = c[k + SYS];
+            dyl[k] = dot3(R.Y1, ym, xc[k], yp);
+            if (k > 0 && k < NZ - 1) xx[k] = xx[k] + dot3(R.Y2, ym, xc[k], yp);
+        }
     }
     // beside a wall the first derivative on the sigma ghost level takes the window shifted one column inwards
     if (i == 1 || i == nxg - 2) {
         const T *q = c + (i == 1 ? 0 : -2) * SXS;
         dxl[0] = dot3(R.XW, q[0], q[SXS], q[2 * SXS]);
     }
-    if (j == 1 || j == nyg - 2) {
-        const T *q = c + (j == 1 ? 0 : -2) * SYS;
-        dyl[0] = dot3(R.YW, q[0], q[SYS], q[2 * SYS]);
+    if constexpr (D3) {
+        if (j == 1 || j == nyg - 2) {
+            const T *q = c + (j == 1 ? 0 : -2) * SYS;
+            dyl[0] = dot3(R.YW, q[0], q[SYS], q[2 * SYS]);
+        }
     }
     o[NZ - 1] = b[NZ - 1] - xc[NZ - 1];
 #pragma unroll
@@ -3385,7 +3383,7 @@ __device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, 
         const T *Z = L.sz + 6;
         const T Z1[3] = {Z[0], Z[1], Z[2]};
         const T om = T(1) - L.zs[1];
-        const T s2 = om * cp[3], s4 = om * cp[4], s5 = cp[0], hx = cp[1], hy = cp[2];
+        const T s2 = om * cp[3], s4 = om * cp[4], s5 = cp[0], hx = cp[1], hy = D3 ? cp[2] : T(0);
         const T dz = dot3(Z1, xc[0], xc[1], xc[2]), cz = fma1(hy, s4, fma1(hx, s2, s5));
         o[0] = b[0] - fma1(hy, dyl[1], fma1(cz, dz, hx * dxl[1]));
     }
@@ -3459,7 +3457,7 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(LvArgs<T> L, Restri
     xr.template store<NZP, WX>(sX, wrows, wcols);
     lds_barrier();
     T o[NZ];
-    if (active) residual_rows<T, NZ, NZP, WX * NZP>(L, i, j, rows, cp, sX + ((j - loy) * WX + (i - lox)) * NZP, bc, o);
+    if (active) residual_rows<T, NZ, true, NZP>(L, i, j, rows, cp, sX + ((j - loy) * WX + (i - lox)) * NZP, WX * NZP, bc, o);
     lds_barrier();
     if (active) {
         T *dst = sX + (ty * FW + tx) * NZP;
@@ -3523,6 +3521,21 @@ __global__ void k_mg_prolong_tab(RestrictGeo G, const int2 *__restrict__ pxi, co
     xf[q] = x0 + e;
 }
 
+// Row r's partial sums of x = Minv b for one wave: every lane's products of 16-byte chunks of the row and the matching
+// values of b, in order (k_mg_coarse, and the dense solve of k_mg_bottom).
+template <typename T, typename M>
+__device__ __forceinline__ T coarse_chunk(const M *__restrict__ row, const T *b, int c0) {
+    constexpr int V = 16 / (int)sizeof(M);
+    const uint4 q = *reinterpret_cast<const uint4 *>(row + c0);
+    M m[V];
+    __builtin_memcpy(m, &q, 16);
+    T bv[V];
+    __builtin_memcpy(bv, __builtin_assume_aligned(b + c0, 16), V * sizeof(T));
+    T p = T(0);
+#pragma unroll
+    for (int v = 0; v < V; v++) p += (T)m[v] * bv[v];
+    return p;
+}
 // Coarsest level: x = Minv b with the dense inverse computed at set-up, stored as M (T, or FP16 with
 // sums in T) in rows of `pitch` elements (a multiple of 8; zeros past n); b holds pitch elements (zeros
 // past n).  One 64-lane wave per row: each lane reads 16 bytes of the row and the matching b values per
@@ -3537,129 +3550,500 @@ __global__ __launch_bounds__(256) void k_mg_coarse(int n, int pitch, const M *__
     const M *row = Minv + (size_t)r * pitch;
     T s = T(0);
 #pragma unroll 4
-    for (int c0 = lane * V; c0 < n; c0 += 64 * V) {
-        const uint4 q = *reinterpret_cast<const uint4 *>(row + c0);
-        M m[V];
-        __builtin_memcpy(m, &q, 16);
-        T bv[V];
-        __builtin_memcpy(bv, __builtin_assume_aligned(b + c0, 16), V * sizeof(T));
-        T p = T(0);
-#pragma unroll
-        for (int v = 0; v < V; v++) p += (T)m[v] * bv[v];
-        s += p;
-    }
+    for (int c0 = lane * V; c0 < n; c0 += 64 * V) s += coarse_chunk<T, M>(row, b, c0);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if (lane == 0) x[r] = s;
 }
 
-
-// The bottom of the V cycle in one workgroup: levels 0 .. nlev-1 of a hierarchy (0 = coarsest) whose
-// finest member `top` = nlev-1 arrives with its right-hand side set and x = 0.  Runs the same sequence
-// as the multi-kernel V cycle (ghost pass, nu1 x (red, black, ghost), residual, restriction, ..., dense
-// coarse solve, ..., prolongation, ghost pass, nu2 x (red, black, ghost)), with the level vectors in HBM /
-// L2 and a workgroup barrier between the steps.  Small levels cost one barrier per step instead of one
-// kernel launch.
-constexpr int MG_BOTTOM_MAX = 10;
+// The V cycle on the small levels in one workgroup: levels 0 .. top of the hierarchy (0 = coarsest, solved densely), whose
+// finest member's right-hand side arrives in HBM and whose iterate starts from zero.  Same steps as the launches it
+// replaces (per level: sweeps with their ghost passes, residual, restriction; dense solve; prolongation, sweeps).
+// Each of those launches is a chain of latencies with a few hundred columns of work: its start, its loads, its stores
+// and the drain before the next one take 5-10 us for 1-2 us of arithmetic.  Here the level vectors stay in LDS from the
+// first restriction to the last prolongation and a step ends with an LDS barrier.  What bounds it is the instruction
+// chain of a step on at most four waves per SIMD-quad, so columns keep everything in registers, stores come after all
+// loads of a step, and the tables of a level (stencil rows, transfer weights) are copied to LDS once.
+// One thread per column of a colour in a sweep, 256 threads: a wave per SIMD, so that a thread can hold the records
+// of its red and its black column at once (up to 350 registers in FP64).  The records of these levels are stored by
+// 16-byte chunk (LvArgs::facq): one compute unit serves a line per cycle and about one load instruction per 16, and
+// the 64 lanes of a wave read 64 lines with a column's contiguous record per lane (4000-5500 cycles a step), 37
+// instructions with a value per lane (4000-6500), 16 lines and a fourth or half of the instructions with a chunk.
+constexpr int MG_BOTTOM_MAX = 10, MG_BOTTOM_NT = 256;
+// A level handed to the kernel has at most one column of a colour per thread: columns away from the walls, and (in waves
+// of their own, two lanes per column) those beside a wall.
+__host__ __device__ inline int bottom_inner(int nxg, int nyg, bool d3) {   // columns of a colour, two or more from every wall
+    return (nxg > 4 && (!d3 || nyg > 4)) ? (nxg - 3) / 2 * (d3 ? nyg - 4 : 1) : 0;
+}
+__host__ __device__ inline int bottom_edge(int nxg, int nyg, bool d3) { return d3 ? 2 * ((nxg - 1) / 2) + 2 * ((nyg - 1) / 2) : 2; }
+__host__ __device__ inline int bottom_ghosts(int nxg, int nyg, bool d3) { return d3 ? 2 * nxg + 2 * (nyg - 2) : 2; }
+inline bool bottom_fits(int nxg, int nyg, bool d3) {
+    return (bottom_inner(nxg, nyg, d3) + 63) / 64 * 64 + (bottom_edge(nxg, nyg, d3) + 31) / 32 * 64 <= MG_BOTTOM_NT &&
+           bottom_ghosts(nxg, nyg, d3) <= MG_BOTTOM_NT / 2 && nxg * nyg <= 2 * MG_BOTTOM_NT;
+}
+template <typename T>
+struct BottomLevel {
+    LvArgs<T> L;
+    int xc, yc, zc, tab;                  // coarsening of the next coarser level; its transfers have weight tables (MgLevel::ptab)
+    int nxgc, nygc, nzgc, pad;
+    int x, b;                             // LDS offsets (elements) of iterate and right-hand side
+    // offsets in the tables: stencil rows; restriction weights per coarse column and row (d_lo, d_lo + d_hi, d_hi,
+    // 1 / (2 (d_lo + d_hi))) and level (d_lo, d_hi, 1 / (2 (d_lo + d_hi))); prolongation weights per fine column, row and
+    // level (left, right, 1 / sum)
+    int sx, sy, rx, ry, rz, px, py, pz;
+};
 template <typename T>
 struct BottomArgs {
-    int nlev, nu1, nu2, n0, pitch0;   // pitch0: row pitch (elements) of minv
-    const T *minv;
-    LvArgs<T> L[MG_BOTTOM_MAX];
-    T *x[MG_BOTTOM_MAX];
-    T *b[MG_BOTTOM_MAX];
-    T *r[MG_BOTTOM_MAX];
-    RestrictGeo G[MG_BOTTOM_MAX];   // G[l]: level l (fine) -> level l-1 (coarse), l >= 1
-    const int *skip;                // solve_done flag (nullptr: always run)
+    int nlev, nu1, nu2, n0, pitch0, half0;   // pitch0: row pitch (elements) of minv; half0: it is FP16
+    int r, tab, ntab, image;                 // LDS offsets of the residual and of the tables; elements of tables and of all x and b
+    const void *minv;
+    const T *tables;
+    T *b, *x;                                // right-hand side of level nlev - 1; its result
+    T *b0, *x0;                              // the same of level 0, and
+    T *img;                                  // the LDS image, where the dense solve is a launch of its own
+    BottomLevel<T> lev[MG_BOTTOM_MAX];
 };
+// Read-only device data behind a pointer that was itself loaded from memory: as constant address space, so that
+// uniform reads are scalar loads and the others global (not flat) ones.
+template <typename P>
+__device__ __forceinline__ const P *ro(const P *p) {
+    return (const P *)(const __attribute__((address_space(4))) P *)(unsigned long long)p;
+}
 
-template <typename T, int NZ>
-__device__ void bottom_sweep(const LvArgs<T> &L, int colour, T *__restrict__ x, const T *__restrict__ b) {
-    const int nxi = L.nxg - 2 * L.gx, half = (nxi + 1) / 2, nyi = L.dim3 ? L.nyg - 2 * L.gy : 1;
-    const int nxg = L.nxg;
-    auto X = [&](int k, int ii, int jj) -> T { return x[((size_t)jj * nxg + ii) * NZ + k]; };
-    for (int c = threadIdx.x; c < half * nyi; c += blockDim.x) {
+template <typename T, int NZ, bool D3>
+struct BottomStep {
+    using Rec = LineRecord<T, NZ>;
+    static constexpr int NZP = NZ | 1, NT = MG_BOTTOM_NT, NZH = (NZ - 2) / 2 + 2;   // NZH: depth of a sigma-coarsened level
+    // The steps other than the sweeps' halves take two threads per column, NT / 2 apart: f(0) the levels below HALF, f(1)
+    // the others (each thread's chain is half as long, and which half it is is known per wave).
+    static constexpr int HALF = NZ / 2, NC = NT / 2;
+    template <class F>
+    __device__ __forceinline__ static void halves(const F &f) {
+        if ((int)threadIdx.x < NC) f(std::integral_constant<int, 0>{});
+        else f(std::integral_constant<int, 1>{});
+    }
+    struct Column {
         int i, j;
-        if (!colour_column(L, colour, c, i, j)) continue;
-        const size_t p = (size_t)i + (size_t)nxg * j;
-        zebra_column<T, NZ>(L, CoefG<T>{L}, i, j, X, b + p * NZ, x + p * NZ);
-    }
-}
+        bool on;
+        T rec[Rec::N];
+    };
+    LvArgs<T> L;
+    const T *tab;                // the tables in LDS
+    T *X, *B;
+    Column cur, nxt;             // the thread's red and black column
+    T cp[6];                     // planes of the thread's next column in the residual
+    bool edge, upper;
+    int gi, gj;                  // the thread's wall ghost column (gi < 0: none)
 
-template <typename T, int NZ>
-__device__ void bottom_residual(const LvArgs<T> &L, const T *__restrict__ x, const T *__restrict__ b, T *__restrict__ r) {
-    const int nxg = L.nxg;
-    auto X = [&](int k, int ii, int jj) -> T { return x[((size_t)jj * nxg + ii) * NZ + k]; };
-    for (int c = threadIdx.x; c < L.nxy; c += blockDim.x) {
-        const int i = c % nxg, j = c / nxg;
-        T o[NZ];
-        residual_column<T, NZ>(L, CoefG<T>{L}, i, j, X, b + (size_t)c * NZ, o);
-#pragma unroll
-        for (int k = 0; k < NZ; k++) r[(size_t)c * NZ + k] = o[k];
-    }
-}
-
-template <typename T>
-__device__ void bottom_ghost(const LvArgs<T> &L, T *x, const T *b) {
-    const int nb = ghost_count(L);
-    for (int t = threadIdx.x; t < nb; t += blockDim.x) ghost_point(L, t, x, b);
-}
-
-template <typename T, int NZ>
-__device__ void bottom_smooth(const LvArgs<T> &L, int nu, T *x, const T *b) {
-    bottom_ghost(L, x, b);
-    __syncthreads();
-    for (int it = 0; it < nu; it++) {
-        bottom_sweep<T, NZ>(L, 0, x, b);
-        __syncthreads();
-        bottom_sweep<T, NZ>(L, 1, x, b);
-        __syncthreads();
-        bottom_ghost(L, x, b);
-        __syncthreads();
-    }
-}
-
-// The V cycle on the small levels in one workgroup (a workgroup barrier between steps instead of a
-// kernel boundary).  All levels 1 .. nlev-1 of the group have NZ sigma levels; level 0 is solved
-// densely.  The level table lives in device memory: each level's arguments are copied out of it once
-// (no run-time indexing of a kernel-argument array, which would go through scratch).
-template <typename T, int NZ>
-__global__ __launch_bounds__(512) void k_mg_bottom(const BottomArgs<T> *__restrict__ A) {
-    if (solve_done(A->skip)) return;
-    const int top = A->nlev - 1, nu1 = A->nu1, nu2 = A->nu2;
-    for (int l = top; l >= 1; l--) {
-        const LvArgs<T> L = A->L[l];
-        T *x = A->x[l], *r = A->r[l];
-        const T *b = A->b[l];
-        bottom_smooth<T, NZ>(L, nu1, x, b);
-        bottom_residual<T, NZ>(L, x, b, r);
-        __syncthreads();
-        const RestrictGeo G = A->G[l];
-        T *bc = A->b[l - 1], *xc = A->x[l - 1];
-        const size_t nc = (size_t)G.nxgc * G.nygc * G.nzgc;
-        for (size_t q = threadIdx.x; q < nc; q += blockDim.x) restrict_point(G, q, (const T *)r, bc, xc);
-        __syncthreads();
-    }
-    {
-        const int n0 = A->n0;
-        const T *minv = A->minv, *b0 = A->b[0];
-        T *x0 = A->x[0];
-        for (int rr = threadIdx.x; rr < n0; rr += blockDim.x) {
-            T s = T(0);
-            for (int c = 0; c < n0; c++) s += minv[(size_t)rr * A->pitch0 + c] * b0[c];
-            x0[rr] = s;
+    // Step l of the cycle: what does not depend on the step before is loaded here.
+    __device__ __forceinline__ void load(const BottomLevel<T> &V, T *lds, const T *ltab, bool down) {
+        L = V.L;
+        L.sx = ltab + V.sx; L.sy = ltab + V.sy;
+        L.sz = ro(L.sz); L.zs = ro(L.zs); L.col = ro(L.col); L.fac = ro(L.fac);
+        tab = ltab;
+        X = lds + V.x; B = lds + V.b;
+        const int nxg = L.nxg, nyg = L.nyg, th = (int)threadIdx.x;
+        const int nip = (bottom_inner(nxg, nyg, D3) + 63) / 64 * 64;
+        edge = th >= nip;
+        upper = edge && ((th - nip) & 32);
+        column(cur, 0); column(nxt, 1);
+        const int tc = th & (NC - 1);
+        if (down) planes(cmin(tc, L.nxy - 1));
+        gi = -1; gj = 0;
+        if (tc < bottom_ghosts(nxg, nyg, D3)) {
+            if (!D3) gi = tc == 0 ? 0 : nxg - 1;
+            else if (tc < nxg) gi = tc;
+            else if (tc < 2 * nxg) { gi = tc - nxg; gj = nyg - 1; }
+            else if (tc < 2 * nxg + nyg - 2) { gi = 0; gj = 1 + tc - 2 * nxg; }
+            else { gi = nxg - 1; gj = 1 + tc - 2 * nxg - (nyg - 2); }
         }
     }
-    __syncthreads();
-    for (int l = 1; l <= top; l++) {
-        const RestrictGeo G = A->G[l];
-        const LvArgs<T> L = A->L[l];
-        T *x = A->x[l];
-        const T *b = A->b[l], *xc = A->x[l - 1];
-        const size_t nf = (size_t)G.nxgf * G.nygf * G.nzgf;
-        for (size_t q = threadIdx.x; q < nf; q += blockDim.x) prolong_point(G, q, xc, x);
-        __syncthreads();
-        bottom_smooth<T, NZ>(L, nu2, x, b);
+    __device__ __forceinline__ void column(Column &C, int c) {   // of colour c
+        const int nxg = L.nxg, nyg = L.nyg, th = (int)threadIdx.x;
+        const int ni = bottom_inner(nxg, nyg, D3), nip = (ni + 63) / 64 * 64, hw = cmax((nxg - 3) / 2, 1);
+        if (!edge) {
+            const int r = D3 ? th / hw : 0, t = th - r * hw;
+            C.j = D3 ? 2 + r : 0;
+            C.i = 2 + ((C.j & 1) != c ? 1 : 0) + 2 * t;
+            C.on = th < ni && C.i <= nxg - 3;
+        } else {   // south row, north row, then west and east column
+            const int l = ((th - nip) >> 6) * 32 + ((th - nip) & 31), bx = D3 ? (nxg - 1) / 2 : 0, by = D3 ? (nyg - 1) / 2 : 1;
+            if (D3 && l < 2 * bx) {
+                const bool first = l < bx;
+                C.j = first ? 1 : nyg - 2;
+                C.i = 1 + (((1 + C.j) & 1) != c ? 1 : 0) + 2 * (first ? l : l - bx);
+                C.on = C.i <= nxg - 2 && (first || nyg > 3);
+            } else {
+                const int q = l - 2 * bx;
+                const bool first = q < by;
+                C.i = first ? 1 : nxg - 2;
+                C.j = (D3 ? 1 : 0) + (((C.i + (D3 ? 1 : 0)) & 1) != c ? 1 : 0) + 2 * (first ? q : q - by);
+                C.on = q < 2 * by && C.j <= (D3 ? nyg - 2 : 0) && (first || nxg > 3) && !(D3 && (C.j == 1 || C.j == nyg - 2));
+            }
+        }
+        const int i = C.on ? C.i : 1, j = C.on ? C.j : (D3 ? 1 : 0);   // (idle lanes load a valid column)
+        const int r = (int)Rec::index(nxg, nyg, i, j);
+#pragma unroll
+        for (int q = 0; q < Rec::N / Rec::W; q++) {
+            T v[Rec::W];
+            load_record(L.fac + (q * L.facq + r) * Rec::W, v);
+#pragma unroll
+            for (int m = 0; m < Rec::W; m++) C.rec[q * Rec::W + m] = v[m];
+        }
+    }
+    __device__ __forceinline__ void planes(int c) {
+#pragma unroll
+        for (int q = 0; q < 6; q++) cp[q] = L.col[q * L.nxy + c];
+    }
+    __device__ __forceinline__ T *at(T *v, int i, int j) const { return v + (j * L.nxg + i) * NZP; }
+    __device__ __forceinline__ void ghost_pass(bool zero) {   // k_mg_sweep's
+        if (gi < 0) return;
+        T *d = at(X, gi, gj);
+        const T *gp = at(B, gi, gj);
+        const int nxg = L.nxg, nyg = L.nyg;
+        const bool gx = gi == 0 || gi == nxg - 1, gy = D3 && (gj == 0 || gj == nyg - 1);
+        const bool low = gx ? gi == 0 : gj == 0;
+        const T *S = gx ? L.sx + (low ? 1 : nxg - 2) * 6 : L.sy + (low ? 1 : nyg - 2) * 6;
+        const T *xa = gx ? at(X, low ? 1 : nxg - 3, gj) : at(X, gi, low ? 1 : nyg - 3);
+        const T *xb = gx ? at(X, low ? 2 : nxg - 2, gj) : at(X, gi, low ? 2 : nyg - 2);
+        halves([&](auto h) {
+#pragma clang fp contract(off)
+            constexpr int K0 = h.value ? HALF : 0, K1 = h.value ? NZ : HALF;
+            T v[NZ];
+#pragma unroll
+            for (int k = K0; k < K1; k++) v[k] = zero ? T(0) : gp[k];
+            if (!zero && !(gx && gy)) {
+                const T w0 = S[0], w1 = S[1], w2 = S[2];
+                const T dg = low ? w0 : w2, wa = low ? w1 : w0, wb = low ? w2 : w1;
+                T a[NZ], b[NZ];
+#pragma unroll
+                for (int k = cmax(K0, 1); k < K1; k++) { a[k] = xa[k]; b[k] = xb[k]; }
+#pragma unroll
+                for (int k = cmax(K0, 1); k < K1; k++) {
+                    const T sum = fma1(wb, b[k], wa * a[k]);
+                    v[k] = (v[k] - sum) / dg;
+                }
+            }
+#pragma unroll
+            for (int k = K0; k < K1; k++) d[k] = v[k];
+        });
+    }
+    __device__ __forceinline__ void half(const Column &C, bool zero) {   // zero: all neighbours are
+        if (!C.on) return;
+        T *d = at(X, C.i, C.j);
+        const T *bp = at(B, C.i, C.j);
+        T f[NZ], up[NZ], inv[NZ], rh[NZ], x[NZ], bw[4], b[NZ];
+        const T c3 = C.rec[Rec::C3], c4 = C.rec[Rec::C4];
+#pragma unroll
+        for (int k = 0; k < NZ; k++) b[k] = bp[k];
+#pragma unroll
+        for (int q = 0; q < 4; q++) bw[q] = C.rec[Rec::BW + q];
+#pragma unroll
+        for (int k = 0; k < NZ - 1; k++) { f[k] = C.rec[k]; up[k] = C.rec[NZ - 1 + k]; inv[k] = C.rec[2 * NZ - 2 + k]; }
+        if (zero) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) rh[k] = b[k];
+        } else if (!edge && L.uni) {
+            line_rhs_uniform<T, NZ, D3, NZP>(L, c3, c4, bw, d, L.nxg * NZP, b, rh);
+        } else {
+            LineRows<T, D3> R;
+            R.load(L, C.i, C.j);
+            if (edge) line_rhs_pair<T, NZ, D3, NZP>(L, C.i, C.j, upper, R, c3, c4, bw, d, L.nxg * NZP, b, rh);
+            else line_rhs_general<T, NZ, D3, NZP>(L, C.i, C.j, R, c3, c4, bw, d, L.nxg * NZP, b, rh);
+        }
+        line_solve<T, NZ>(f, up, inv, rh, x);
+        if (!upper) {
+#pragma unroll
+            for (int k = 0; k < NZ; k++) d[k] = x[k];
+        }
+    }
+    // nu sweeps, from zero before a descent; a ghost pass before each, and after the last one of a descent
+    __device__ __forceinline__ void smooth(int nu, bool down) {
+#pragma unroll 1
+        for (int it = 0; it < nu + (down ? 1 : 0); it++) {
+            const bool zero = down && it == 0;
+            ghost_pass(zero);
+            lds_barrier();
+            if (it == nu) break;
+            if (it > 0) { column(cur, 0); column(nxt, 1); }
+#pragma unroll 1
+            for (int c = 0; c < 2; c++) {   // (one copy of the code: the kernel stays within the reach of short branches)
+                half(cur, zero && c == 0);
+                lds_barrier();
+                cur = nxt;
+            }
+        }
+    }
+    // residual into r, restricted onto the coarse right-hand side (cb, column stride cs)
+    __device__ __forceinline__ void descend(const BottomLevel<T> &V, T *r, T *cb, int cs) {
+        const int nxg = L.nxg, nyg = L.nyg, th = (int)threadIdx.x;
+        halves([&](auto h) {
+            constexpr int K0 = h.value ? HALF : 0, K1 = h.value ? NZ : HALF;
+#pragma unroll 1
+            for (int c = th & (NC - 1); c < L.nxy; c += NC) {
+                const int j = D3 ? c / nxg : 0, i = c - j * nxg;
+                T b[NZ], o[NZ], cc[6];
+#pragma unroll
+                for (int q = 0; q < 6; q++) cc[q] = cp[q];
+                planes(cmin(c + NC, L.nxy - 1));
+                LineRows<T, D3> R;
+                R.load(L, cclamp(i, 1, nxg - 2), D3 ? cclamp(j, 1, nyg - 2) : 0);
+#pragma unroll
+                for (int k = 0; k < NZ; k++) b[k] = B[c * NZP + k];
+                residual_rows<T, NZ, D3, NZP>(L, i, j, R, cc, X + c * NZP, nxg * NZP, b, o);   // (the other half's rows are dead code)
+#pragma unroll
+                for (int k = K0; k < K1; k++) r[c * NZP + k] = o[k];
+            }
+        });
+        lds_barrier();
+        if ((D3 ? V.xc && V.yc : V.xc) && !V.zc) restrict_columns(V, r, cb, cs);
+        else restrict_points(V, r, cb, cs);
+        lds_barrier();
+    }
+    // Coarse column c of the restriction (restrict_at's and k_mg_restrict_tab's arithmetic).  FULL: x and, in 3D, y are coarsened.
+    template <bool FULL>
+    struct Coarse {
+        const T *q;          // its residual column
+        T wx[4], wy[4];
+        int row, py, ny;     // fine row, row pitch, rows
+        bool in, xc, yc;     // in: no wall ghost column (those are zero)
+        __device__ __forceinline__ void set(const BottomStep &S, const BottomLevel<T> &V, const T *r, int c) {
+            const int jc = D3 ? c / V.nxgc : 0, ic = c - jc * V.nxgc;
+            xc = FULL || V.xc; yc = D3 && (FULL || V.yc);
+            in = ic >= 1 && ic <= V.nxgc - 2 && (!D3 || (jc >= 1 && jc <= V.nygc - 2));
+            const int fi = in ? (xc ? 2 * ic - 1 : ic) : 1;
+            row = in ? (yc ? 2 * jc - 1 : jc) : (D3 ? 1 : 0);   // (ghost columns read a valid one)
+            py = S.L.nxg * NZP; ny = S.L.nyg;
+            q = r + row * py + fi * NZP;
+#pragma unroll
+            for (int m = 0; m < 4; m++) { wx[m] = S.tab[V.rx + 4 * ic + m]; wy[m] = D3 ? S.tab[V.ry + 4 * jc + m] : T(0); }
+        }
+        __device__ __forceinline__ T line(const T *p, int dj) const {
+#pragma clang fp contract(off)
+            p += dj * py;
+            const T r1 = p[0];
+            if (!FULL && !xc) return r1;
+            const T s = wx[3] * fma1(wx[2], p[NZP], fma1(wx[0], p[-NZP], wx[1] * r1));
+            return D3 && (row + dj < 1 || row + dj > ny - 2) ? r1 : s;
+        }
+        __device__ __forceinline__ T plane(int k) const {   // smoothed in the plane of fine level k, 1 .. NZ - 2
+#pragma clang fp contract(off)
+            if (!D3 || (!FULL && !yc)) return line(q + k, 0);
+            return wy[3] * fma1(wy[2], line(q + k, 1), fma1(wy[0], line(q + k, -1), wy[1] * line(q + k, 0)));
+        }
+    };
+    // sigma not coarsened: two threads per coarse column
+    __device__ __forceinline__ void restrict_columns(const BottomLevel<T> &V, const T *r, T *cb, int cs) {
+        halves([&](auto h) {
+            constexpr int K0 = h.value ? HALF : 0, K1 = h.value ? NZ : HALF;
+#pragma unroll 1
+            for (int c = (int)threadIdx.x & (NC - 1); c < V.nxgc * V.nygc; c += NC) {
+                Coarse<true> P;
+                P.set(*this, V, r, c);
+                T y[NZ];
+#pragma unroll
+                for (int k = K0; k < K1; k++) y[k] = k == 0 ? T(0) : k == NZ - 1 ? P.q[k] : P.plane(k);
+#pragma unroll
+                for (int k = K0; k < K1; k++) cb[c * cs + k] = P.in ? y[k] : T(0);
+            }
+        });
+    }
+    // any coarsening: a thread per coarse point (the smallest levels)
+    __device__ __forceinline__ void restrict_points(const BottomLevel<T> &V, const T *r, T *cb, int cs) {
+#pragma clang fp contract(off)
+        const int nzc = V.nzgc;
+#pragma unroll 1
+        for (int e = (int)threadIdx.x; e < V.nxgc * V.nygc * nzc; e += NT) {
+            const int c = e / nzc, k = e - c * nzc;
+            Coarse<false> P;
+            P.set(*this, V, r, c);
+            const int kf = V.zc ? 2 * k - 1 : k;
+            T v = T(0);
+            if (P.in && k > 0) {
+                if (k == nzc - 1) v = P.q[NZ - 1];
+                else {
+                    v = P.plane(kf);
+                    if (V.zc) {
+                        const T *wz = tab + V.rz + 3 * k;
+                        const T lo = kf == 1 ? P.q[0] : P.plane(kf - 1), hi = kf == NZ - 2 ? P.q[NZ - 1] : P.plane(kf + 1);
+                        v = fma1(wz[2], fma1(wz[0], lo, wz[1] * hi), T(0.5) * v);
+                    }
+                }
+            }
+            cb[c * cs + k] = v;
+        }
+    }
+    // Fine column c of the prolongation (prolong_at's and k_mg_prolong_tab's arithmetic), on the coarse correction ec.
+    struct Fine {
+        const T *ea, *eb, *el, *er;
+        T wxl, wxr, sx, wyl, wyr, sy;
+        bool in;
+        __device__ __forceinline__ void set(const BottomStep &S, const BottomLevel<T> &V, const T *ec, int cs, int c) {
+            const int nxg = S.L.nxg, j = D3 ? c / nxg : 0, i = c - j * nxg;
+            in = i >= 1 && i <= nxg - 2 && (!D3 || (j >= 1 && j <= S.L.nyg - 2));
+            const int xl = V.xc ? 1 + ((i - 1) >> 1) : i, xr = V.xc ? 1 + (i >> 1) : i;
+            const int yl = !D3 ? 0 : V.yc ? 1 + ((j - 1) >> 1) : j, yr = !D3 ? 0 : V.yc ? 1 + (j >> 1) : j;
+            wxl = S.tab[V.px + 3 * i]; wxr = S.tab[V.px + 3 * i + 1]; sx = S.tab[V.px + 3 * i + 2];
+            if constexpr (D3) { wyl = S.tab[V.py + 3 * j]; wyr = S.tab[V.py + 3 * j + 1]; sy = S.tab[V.py + 3 * j + 2]; }
+            ea = ec + (yl * V.nxgc + xl) * cs; eb = ec + (yl * V.nxgc + xr) * cs;
+            el = ec + (yr * V.nxgc + xl) * cs; er = ec + (yr * V.nxgc + xr) * cs;
+        }
+        __device__ __forceinline__ T plane(int k) const {   // interpolated in the plane of coarse level k, without the last scale
+#pragma clang fp contract(off)
+            const T lo = fma1(wxl, ea[k], wxr * eb[k]);
+            if constexpr (!D3) return lo;
+            else {
+                const T l1 = lo * sx, h1 = fma1(wxl, el[k], wxr * er[k]) * sx;
+                return fma1(wyl, l1, wyr * h1);
+            }
+        }
+        __device__ __forceinline__ T scale() const {
+            if constexpr (D3) return sy;
+            else return sx;
+        }
+    };
+    // adds the prolongated coarse correction (ec, column stride cs)
+    __device__ __forceinline__ void ascend(const BottomLevel<T> &V, const T *ec, int cs) {
+        if (!V.zc) {   // two threads per column
+            halves([&](auto h) {
+#pragma clang fp contract(off)
+                constexpr int K0 = h.value ? HALF : 1, K1 = h.value ? NZ - 1 : HALF;
+#pragma unroll 1
+                for (int c = (int)threadIdx.x & (NC - 1); c < L.nxy; c += NC) {
+                    Fine P;
+                    P.set(*this, V, ec, cs, c);
+                    if (!P.in) continue;
+                    T *d = X + c * NZP;
+                    T x[NZ], m[NZ];
+#pragma unroll
+                    for (int k = K0; k < K1; k++) { x[k] = d[k]; m[k] = P.plane(k); }
+#pragma unroll
+                    for (int k = K0; k < K1; k++) d[k] = V.tab ? fma1(m[k], P.scale(), x[k]) : x[k] + m[k] * P.scale();
+                }
+            });
+        } else {   // a thread per point (the smallest levels)
+#pragma clang fp contract(off)
+#pragma unroll 1
+            for (int e = (int)threadIdx.x; e < L.nxy * (NZ - 2); e += NT) {
+                const int c = e / (NZ - 2), k = 1 + e - c * (NZ - 2), kc = (k + 1) / 2;
+                Fine P;
+                P.set(*this, V, ec, cs, c);
+                if (!P.in) continue;
+                T *d = X + c * NZP + k;
+                const T *wz = tab + V.pz + 3 * k;
+                const bool odd = k % 2;   // on coarse level kc; else between kc and kc + 1 (none on the surface)
+                const T lo = P.plane(kc) * P.scale();
+                T hi = T(0);
+                if (!odd && kc + 1 < NZH - 1) hi = P.plane(kc + 1) * P.scale();
+                *d = *d + (odd ? lo : fma1(wz[0], lo, wz[1] * hi) * wz[2]);
+            }
+        }
+        lds_barrier();
+    }
+};
+
+// Runs `f` with the column depth nzg, one of NZ and its sigma coarsenings.
+template <int NZ, class F>
+__device__ __forceinline__ void bottom_depth(int nzg, const F &f) {
+    if (nzg == NZ) f(std::integral_constant<int, NZ>{});
+    else if constexpr (NZ % 2 == 0 && NZ >= 4) bottom_depth<(NZ - 2) / 2 + 2>(nzg, f);
+}
+
+// x = Minv b in one workgroup, k_mg_coarse's arithmetic: a wave takes RB rows at a time, and the reductions over its lanes
+// pass half of the rows to the other half of the lanes at each of the first three steps (sums of the same pairs).
+template <typename T, typename M>
+__device__ __forceinline__ void bottom_dense(int n, int pitch, const M *__restrict__ minv, const T *b, T *x) {
+    constexpr int V = 16 / (int)sizeof(M), RB = 8;
+    const int lane = (int)threadIdx.x & 63;
+    for (int r0 = ((int)threadIdx.x >> 6) * RB; r0 < n; r0 += MG_BOTTOM_NT / 64 * RB) {
+        T s[RB];
+#pragma unroll
+        for (int q = 0; q < RB; q++) s[q] = T(0);
+        for (int c0 = lane * V; c0 < n; c0 += 64 * V) {
+#pragma unroll
+            for (int q = 0; q < RB; q++) s[q] += coarse_chunk<T, M>(minv + cmin(r0 + q, n - 1) * pitch, b, c0);
+        }
+#pragma unroll
+        for (int h = RB / 2, off = 32; h > 0; h >>= 1, off >>= 1) {
+#pragma unroll
+            for (int q = 0; q < h; q++) {
+                const T keep = pick((lane & off) != 0, s[q + h], s[q]), give = pick((lane & off) != 0, s[q], s[q + h]);
+                s[q] = keep + __shfl_xor(give, off, 64);
+            }
+        }
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) s[0] += __shfl_xor(s[0], off, 64);
+        const int r = r0 + ((lane & 32) ? 4 : 0) + ((lane & 16) ? 2 : 0) + ((lane & 8) ? 1 : 0);
+        if ((lane & 7) == 0 && r < n) x[r] = s[0];
+    }
+}
+
+// PART 0: the whole; 1: down to the right-hand side of level 0; 2: from its solution upwards.
+template <typename T, int NZ, bool D3>
+__global__ __launch_bounds__(MG_BOTTOM_NT) void k_mg_bottom(const BottomArgs<T> *__restrict__ args, const int *skip, int part) {
+    constexpr int NT = MG_BOTTOM_NT;
+    extern __shared__ double bottom_lds[];
+    T *lds = (T *)bottom_lds;
+    const BottomArgs<T> *A = ro(args);
+    const int top = A->nlev - 1, th = (int)threadIdx.x;
+    const bool done = solve_done(skip);
+    T *ltab = lds + A->tab;
+    const T *tables = ro(A->tables);
+    for (int e = th; e < A->ntab; e += NT) ltab[e] = tables[e];
+    if (done) return;
+    if (part == 2) {
+        const T *img = ro((const T *)A->img), *x0 = ro((const T *)A->x0);
+        for (int e = th; e < A->image; e += NT) lds[e] = img[e];
+        lds_barrier();
+        for (int e = th; e < A->n0; e += NT) lds[A->lev[0].x + e] = x0[e];
+    } else {   // the right-hand side, and level 0's zeros up to the inverse's pitch
+        const T *b = ro((const T *)A->b);
+        T *B = lds + A->lev[top].b;
+        for (int c = th; c < A->lev[top].L.nxy; c += NT) {
+            T v[NZ];
+            load_column<NZ>(b + c * NZ, v);
+#pragma unroll
+            for (int k = 0; k < NZ; k++) B[c * (NZ | 1) + k] = v[k];
+        }
+        for (int e = A->n0 + th; e < A->pitch0; e += NT) lds[A->lev[0].b + e] = T(0);
+    }
+    lds_barrier();
+    // levels top .. 1 downwards, 0, and 1 .. top upwards
+    const int last = part == 1 ? top - 1 : 2 * top;
+    for (int st = part == 2 ? top + 1 : 0; st <= last; st++) {
+        const bool down = st < top;
+        const int l = down ? top - st : st - top;
+        if (l == 0) {
+            const T *b = lds + A->lev[0].b;
+            T *x = lds + A->lev[0].x;
+            if (sizeof(T) == 4 && A->half0) bottom_dense<T, __half>(A->n0, A->pitch0, ro((const __half *)A->minv), b, x);
+            else bottom_dense<T, T>(A->n0, A->pitch0, ro((const T *)A->minv), b, x);
+            lds_barrier();
+            continue;
+        }
+        const BottomLevel<T> &V = A->lev[l], &C = A->lev[l - 1];
+        const int cs = l == 1 ? C.L.nzg : (C.L.nzg | 1);   // level 0 is unpadded
+        bottom_depth<NZ>(V.L.nzg, [&](auto depth) {
+            BottomStep<T, decltype(depth)::value, D3> S;
+            S.load(V, lds, ltab, down);
+            if (!down) S.ascend(V, lds + C.x, cs);
+            S.smooth(down ? A->nu1 : A->nu2, down);
+            if (down) S.descend(V, lds + A->r, lds + C.b, cs);
+        });
+    }
+    if (part == 1) {
+        T *img = A->img, *b0 = A->b0;
+        for (int e = th; e < A->image; e += NT) img[e] = lds[e];
+        for (int e = th; e < A->n0; e += NT) b0[e] = lds[A->lev[0].b + e];
+        return;
+    }
+    const T *X = lds + A->lev[top].x;
+    T *out = A->x;
+    for (int c = th; c < A->lev[top].L.nxy; c += NT) {
+        T v[NZ];
+#pragma unroll
+        for (int k = 0; k < NZ; k++) v[k] = X[c * (NZ | 1) + k];
+        store_column<NZ>(out + (size_t)c * NZ, v);
     }
 }
 

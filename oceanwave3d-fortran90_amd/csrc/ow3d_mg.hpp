@@ -290,6 +290,7 @@ int mg_build(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg) {
         L->args.fac = nullptr;
         if (k > 0 && has_records(g)) {
             HIPCHK(L->fac.alloc(line_records<T>(g.nxg, g.nyg, g.nzg)));
+            L->args.facq = k <= t->bot_top ? (int)LineRecord<T, 3>::count(g.nxg, g.nyg) : 0;
             if (factor_launch<T>(L->args, L->fac.p, s)) { err() = "multigrid level depth outside 3..14"; return -1; }
             HIPCHK(hipGetLastError());
             L->args.fac = L->fac.p;
@@ -365,6 +366,18 @@ inline RestrictGeo geo(const Grid &f, const Grid &c, const double *xf, const dou
 }
 
 template <typename T>
+using BottomKernel = void (*)(const BottomArgs<T> *, const int *, int);
+template <typename T>
+BottomKernel<T> bottom_kernel(int nzg, bool d3) {
+    switch (nzg) {
+#define OW3D_NZ(N) case N: return d3 ? k_mg_bottom<T, N, true> : k_mg_bottom<T, N, false>;
+        OW3D_NZ(3) OW3D_NZ(4) OW3D_NZ(5) OW3D_NZ(6) OW3D_NZ(7) OW3D_NZ(8) OW3D_NZ(9) OW3D_NZ(10)
+        OW3D_NZ(11) OW3D_NZ(12) OW3D_NZ(13) OW3D_NZ(14)
+#undef OW3D_NZ
+    }
+    return nullptr;
+}
+template <typename T>
 int fill_bottom(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, BottomArgs<T> &A, DevBuf<BottomArgs<T>> &dA) {
     A = BottomArgs<T>{};
     if (t->bot_top < 0) return 0;
@@ -372,13 +385,76 @@ int fill_bottom(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, Bott
     A.nu1 = t->cfg.nu1; A.nu2 = t->cfg.nu2;
     A.n0 = (int)mg[0]->g.n;
     A.pitch0 = mg[0]->minv_pitch;
-    A.minv = mg[0]->minv.p;
+    A.half0 = mg[0]->minv16.p != nullptr;
+    A.minv = A.half0 ? (const void *)mg[0]->minv16.p : (const void *)mg[0]->minv.p;
+    std::vector<T> tab;
+    auto put = [&](T v) { tab.push_back(v); };
+    // the weights are the ones restrict_at and prolong_at form per point
+    auto rows = [&](const std::vector<double> &s, int n) { const int o = (int)tab.size(); for (int q = 0; q < n; q++) put((T)s[q]); return o; };
+    auto restrict_w = [&](const std::vector<double> &x, int nc, int g, int ncin, int c, bool high) {
+        const int o = (int)tab.size();
+        for (int ic = 0; ic < nc; ic++) {
+            T lo = T(0), hi = T(0);
+            if (c && ic >= g && ic < g + ncin) { const int i = g + 2 * (ic - g); lo = (T)(x[i] - x[i - 1]); hi = (T)(x[i + 1] - x[i]); }
+            put(lo); put(high ? hi + lo : lo + hi); put(hi); put(lo + hi != T(0) ? T(0.5) * (T(1) / (lo + hi)) : T(0));
+        }
+        return o;
+    };
+    auto prolong_w = [&](const std::vector<double> &x, int n, int g, int nin, int c) {
+        const int o = (int)tab.size();
+        for (int i = 0; i < n; i++) {
+            if (c && i >= g && i < g + nin && (i - g) % 2) {
+                const T lo = (T)(x[i] - x[i - 1]), hi = (T)(x[i + 1] - x[i]);
+                put(hi); put(lo); put(T(1) / (lo + hi));
+            } else { put(T(1)); put(T(0)); put(T(1)); }
+        }
+        return o;
+    };
     for (int k = 0; k <= t->bot_top; k++) {
         MgLevel<T> &L = *mg[k];
-        A.L[k] = L.args; A.x[k] = L.x.p; A.b[k] = L.b.p; A.r[k] = L.r.p;
-        if (k >= 1) A.G[k] = geo(L.g, mg[k - 1]->g, L.xf.p, L.yf.p, L.zf.p, t->done());
+        BottomLevel<T> &V = A.lev[k];
+        V.L = L.args;
+        if (k == 0) continue;
+        const Grid &f = L.g, &c = mg[k - 1]->g;
+        V.xc = c.xc; V.yc = f.ny > 1 && c.yc; V.zc = c.zc; V.tab = L.ptab;
+        V.nxgc = c.nxg; V.nygc = c.nyg; V.nzgc = c.nzg;
+        V.sx = rows(f.sx, f.nxg * 6);
+        V.rx = restrict_w(f.x, c.nxg, f.gx, c.nx, c.xc, false);
+        V.px = prolong_w(f.x, f.nxg, f.gx, f.nx, c.xc);
+        if (f.ny > 1) {
+            V.sy = rows(f.sy, f.nyg * 6);
+            V.ry = restrict_w(f.y, c.nyg, f.gy, c.ny, c.yc, true);
+            V.py = prolong_w(f.y, f.nyg, f.gy, f.ny, c.yc);
+        }
+        V.rz = (int)tab.size();   // coarse level kc lies on fine level 2 kc - 1
+        for (int kc = 0; kc < c.nzg; kc++) {
+            T lo = T(0), hi = T(0);
+            if (c.zc && kc >= 1 && 2 * kc < f.nzg) { lo = (T)(f.z[2 * kc - 1] - f.z[2 * kc - 2]); hi = (T)(f.z[2 * kc] - f.z[2 * kc - 1]); }
+            put(lo); put(hi); put(lo + hi != T(0) ? T(0.5) * (T(1) / (lo + hi)) : T(0));
+        }
+        V.pz = (int)tab.size();
+        for (int k2 = 0; k2 < f.nzg; k2++) {
+            T lo = T(0), hi = T(0);
+            if (c.zc && k2 >= 1 && k2 < f.nzg - 1) { lo = (T)(f.z[k2] - f.z[k2 - 1]); hi = (T)(f.z[k2 + 1] - f.z[k2]); }
+            put(hi); put(lo); put(lo + hi != T(0) ? T(1) / (lo + hi) : T(0));
+        }
     }
-    A.skip = t->done();
+    MgLevel<T> &B = *mg[t->bot_top];
+    A.b = B.b.p; A.x = B.x.p;
+    A.b0 = mg[0]->b.p; A.x0 = mg[0]->x.p;
+    A.ntab = (int)tab.size();
+    t->bot_lds = bottom_layout<T>(t->levels, t->bot_top, &A) * sizeof(T);
+    if (bottom_tables(t->levels, t->bot_top) < tab.size()) { err() = "bottom tables exceed their place in LDS"; return -1; }
+    HIPCHK(t->bot_tab.alloc((tab.size() * sizeof(T) + 7) / 8));
+    HIPCHK(hipMemcpy(t->bot_tab.p, tab.data(), tab.size() * sizeof(T), hipMemcpyHostToDevice));
+    A.tables = (const T *)t->bot_tab.p;
+    if (t->bot_split) {
+        HIPCHK(t->bot_img.alloc(((size_t)A.image * sizeof(T) + 7) / 8));
+        A.img = (T *)t->bot_img.p;
+    }
+    const BottomKernel<T> kernel = bottom_kernel<T>(B.g.nzg, B.args.dim3);
+    if (!kernel) { err() = "bottom level depth outside 3..14"; return -1; }
+    HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)t->bot_lds));
     HIPCHK(dA.alloc(1));
     HIPCHK(hipMemcpy(dA.p, &A, sizeof(A), hipMemcpyHostToDevice));
     return 0;
@@ -564,13 +640,16 @@ template <typename T>
 int vcycle(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, int k, const T *b, T *&cur, hipStream_t s,
            const double *r0 = nullptr, double *uout = nullptr) {
     MgLevel<T> &L = *mg[k];
-    if (k == t->bot_top) {   // in place on L.x
-        switch (L.g.nzg) {
-#define OW3D_NZ(N) case N: hipLaunchKernelGGL((k_mg_bottom<T, N>), dim3(1), dim3(512), 0, s, bottom_args<T>(t)); break;
-            OW3D_NZ(3) OW3D_NZ(4) OW3D_NZ(5) OW3D_NZ(6) OW3D_NZ(7) OW3D_NZ(8) OW3D_NZ(9) OW3D_NZ(10)
-            OW3D_NZ(11) OW3D_NZ(12) OW3D_NZ(13) OW3D_NZ(14)
-#undef OW3D_NZ
-            default: err() = "bottom level depth outside 3..14"; return -1;
+    if (k == t->bot_top) {
+        auto part = [&](int p) {
+            hipLaunchKernelGGL(bottom_kernel<T>(L.g.nzg, L.args.dim3), dim3(1), dim3(MG_BOTTOM_NT), t->bot_lds, s, bottom_args<T>(t), t->done(), p);
+        };
+        if (!t->bot_split) part(0);
+        else {
+            part(1);
+            T *c0 = nullptr;
+            if (vcycle<T>(t, mg, 0, mg[0]->b.p, c0, s)) return -1;
+            part(2);
         }
         cur = L.x.p;
         return 0;
@@ -591,7 +670,7 @@ int vcycle(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, int k, co
     RestrictGeo G = geo(L.g, C.g, L.xf.p, L.yf.p, L.zf.p, t->done());
     G.spec = L.args.spec;
     // the coarse iterate is cleared where something reads it: not by the dense solve, nor by a first sweep from zero
-    T *xz = t->bot_top < 0 && (k == 1 || (t->fused_rb && t->cfg.nu1 >= 1)) ? nullptr : C.x.p;
+    T *xz = k == 1 || (t->fused_rb && t->cfg.nu1 >= 1) ? nullptr : C.x.p;
     if (!resrestrict_launch<T>(L, G, cur, b, C.b.p, xz, s)) {
         if (!L.r.p) { err() = "multigrid level has no residual buffer"; return -1; }   // needs_r says otherwise
         if (mg_launch<T>(L.args, 0, 0, cur, b, L.r.p, s)) return -1;
@@ -624,7 +703,7 @@ int precond_body(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, con
     MgLevel<T> &F = *mg[top];
     // with fused sweeps and pre-smoothing above the coarsest level, the first sweep sets b = (T) r from
     // x = 0 itself; otherwise one pass does it first
-    const bool fused = t->fused_rb && top >= 1 && top != t->bot_top;
+    const bool fused = t->fused_rb && top >= 1;
     const bool fuse_in = fused && t->cfg.nu1 >= 1, fuse_out = fused && u && t->cfg.nu2 >= 1;
     // FP64: r itself is the finest level's right-hand side (needs_b; r stays unchanged through the application)
     const T *b = F.b.p;
