@@ -41,6 +41,45 @@ __device__ __forceinline__ void lds_barrier() {
 // nullptr: always run.
 __device__ __forceinline__ bool solve_done(const int *skip) { return skip != nullptr && *skip != 0; }
 
+// Columns between HBM and registers, two values per load or store where every column starts on an even element.
+template <typename S>
+struct alignas(2 * sizeof(S)) ColPair { S a, b; };
+template <int NZ, typename S, typename T>
+__device__ __forceinline__ void load_column(const S *__restrict__ p, T (&v)[NZ]) {
+    if constexpr (NZ % 2 == 0) {
+        const ColPair<S> *q = reinterpret_cast<const ColPair<S> *>(p);
+#pragma unroll
+        for (int k = 0; k < NZ / 2; k++) { const ColPair<S> w = q[k]; v[2 * k] = (T)w.a; v[2 * k + 1] = (T)w.b; }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NZ; k++) v[k] = (T)p[k];
+    }
+}
+// N values (a multiple of 16 bytes) from a 16-byte aligned address.
+template <int N, typename T>
+__device__ __forceinline__ void load_record(const T *__restrict__ p, T (&v)[N]) {
+    constexpr int W = 16 / sizeof(T);
+    struct alignas(16) Quad { T e[W]; };
+    static_assert(N % W == 0, "whole 16-byte loads");
+#pragma unroll
+    for (int q = 0; q < N / W; q++) {
+        const Quad w = reinterpret_cast<const Quad *>(p)[q];
+#pragma unroll
+        for (int e = 0; e < W; e++) v[q * W + e] = w.e[e];
+    }
+}
+template <int NZ, typename T, typename O>
+__device__ __forceinline__ void store_column(O *__restrict__ p, const T (&v)[NZ]) {
+    if constexpr (NZ % 2 == 0) {
+        ColPair<O> *q = reinterpret_cast<ColPair<O> *>(p);
+#pragma unroll
+        for (int k = 0; k < NZ / 2; k++) q[k] = ColPair<O>{(O)v[2 * k], (O)v[2 * k + 1]};
+    } else {
+#pragma unroll
+        for (int k = 0; k < NZ; k++) p[k] = (O)v[k];
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // High-order matvec  (BuildLinearSystem.f90:1-290)
 // ---------------------------------------------------------------------------------------------
@@ -313,203 +352,32 @@ __global__ __launch_bounds__(NT) void k_matvec3p(MvArgs g, const double *__restr
     }
 }
 
-// 3D, one thread per sigma column: block = 16 x TY columns.  The tile and its (alpha+1)-wide halo are
-// staged level-major in LDS (sP[k*PS + column], PS odd), so the 16 lanes of a tile row read consecutive
-// words at every stencil tap (conflict-free) and the column's x- and y-derivatives stay in registers for
-// the mixed derivatives.  Sigma-stencil rows and levels are uniform across the block (scalar loads);
-// the coefficient planes of the tile are staged with the window.  Results are written back through LDS
-// as coalesced row segments.
-template <int NZ, int A, int TY>
-__global__ __launch_bounds__(16 * TY) void k_matvec3c(MvArgs g, const double *__restrict__ phi, double *__restrict__ out) {
-    if (solve_done(g.skip)) return;
-    constexpr int TX = 16, NT = TX * TY, RA = 2 * A + 1, R = A + 1, WX = TX + 2 * R, WY = TY + 2 * R;
-    constexpr int PS = (WX * WY) | 1;
-    __shared__ double sP[NZ * PS];
-    __shared__ double sSX[(TX + 2) * 2 * RA];
-    __shared__ double sSY[(TY + 2) * 2 * RA];
-    const int nxg = g.nxg, nyg = g.nyg, nxy = g.nxy;
-    const int gxt = (nxg + TX - 1) / TX;
-    const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-    const int i0 = (tile % gxt) * TX, j0 = (tile / gxt) * TY;
-    const int lox = cmax(cmin(i0 - R, nxg - 2 - 2 * A), 0);
-    const int loy = cmax(cmin(j0 - R, nyg - 2 - 2 * A), 0);
-    const int wx = cmin(WX, nxg - lox), wy = cmin(WY, nyg - loy);
-    {
-        // every HBM load of the block first: the phi window (stored level-major) and the stencil rows of
-        // its columns and rows (each thread reads its own column's coefficient planes where it uses them)
-        constexpr int RL = WX * NZ, TOT = WY * RL, PER = (TOT + NT - 1) / NT;
-        double v[PER];
-        const double *src = phi + ((size_t)loy * nxg + lox) * NZ;
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = (int)threadIdx.x + q * NT, r = e / RL, c = e - r * RL;
-            v[q] = (e < TOT && r < wy && c < wx * NZ) ? src[(size_t)r * nxg * NZ + c] : 0.0;
-        }
-        for (int e = threadIdx.x; e < (TX + 2) * 2 * RA; e += NT) {
-            const int r = e / (2 * RA), ii = i0 - 1 + r;
-            if (ii >= 0 && ii < nxg) sSX[e] = g.sx[(size_t)ii * 2 * RA + (e - r * 2 * RA)];
-        }
-        for (int e = threadIdx.x; e < (TY + 2) * 2 * RA; e += NT) {
-            const int r = e / (2 * RA), jj = j0 - 1 + r;
-            if (jj >= 0 && jj < nyg) sSY[e] = g.sy[(size_t)jj * 2 * RA + (e - r * 2 * RA)];
-        }
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = (int)threadIdx.x + q * NT, r = e / RL, c = e - r * RL;
-            if (e < TOT && r < wy && c < wx * NZ) {
-                const int cc = c / NZ, k = c - cc * NZ;
-                sP[k * PS + r * WX + cc] = v[q];
-            }
-        }
-    }
-    __syncthreads();
-    auto P = [&](int k, int ii, int jj) -> double { return sP[k * PS + (jj - loy) * WX + (ii - lox)]; };
-    auto SX = [&](int ii) -> const double * { return sSX + (ii - (i0 - 1)) * 2 * RA; };
-    auto SY = [&](int jj) -> const double * { return sSY + (jj - (j0 - 1)) * 2 * RA; };
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    const int i = i0 + tx, j = j0 + ty;
-    const bool active = (i < nxg) && (j < nyg);
-    double o[NZ];
-    if (active) {
-        const bool wxl = (i == 0 || i == nxg - 1), wyl = (j == 0 || j == nyg - 1);
-        if (wxl && wyl) {
-#pragma unroll
-            for (int k = 0; k < NZ; k++) o[k] = P(k, i, j);
-        } else if (wxl || wyl) {
-            // wall ghost column: first derivative across the wall at the adjacent node, identity at k = 0
-            const int ib = wxl ? ((i == 0) ? 1 : nxg - 2) : ((j == 0) ? 1 : nyg - 2);
-            const int ws = wxl ? cclamp(ib - A, 0, nxg - RA) : cclamp(ib - A, 0, nyg - RA);
-            const double *S = wxl ? SX(ib) : SY(ib);
-            o[0] = P(0, i, j);
-#pragma unroll
-            for (int k = 1; k < NZ; k++) {
-                double s = 0.0;
-#pragma unroll
-                for (int m = 0; m < RA; m++) s += S[m] * (wxl ? P(k, ws + m, j) : P(k, i, ws + m));
-                o[k] = s;
-            }
-        } else {
-            double dx[NZ], dy[NZ], pc[NZ];
-            const int wsx = cclamp(i - A, 0, nxg - RA), wsy = cclamp(j - A, 0, nyg - RA);
-            {
-                const double *S1 = SX(i), *S2 = S1 + RA;
-#pragma unroll
-                for (int k = 0; k < NZ; k++) {
-                    double d1 = 0.0, d2 = 0.0;
-#pragma unroll
-                    for (int m = 0; m < RA; m++) { const double v = P(k, wsx + m, j); d1 += S1[m] * v; d2 += S2[m] * v; }
-                    dx[k] = d1; o[k] = d2;
-                }
-            }
-            {
-                const double *S1 = SY(j), *S2 = S1 + RA;
-#pragma unroll
-                for (int k = 0; k < NZ; k++) {
-                    double d1 = 0.0, d2 = 0.0;
-#pragma unroll
-                    for (int m = 0; m < RA; m++) { const double v = P(k, i, wsy + m); d1 += S1[m] * v; d2 += S2[m] * v; }
-                    dy[k] = d1; o[k] += d2;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < NZ; k++) pc[k] = P(k, i, j);
-            // corner-corrected first pass on the sigma ghost level (ConstructTableCrossDerivatives.f90:173-186)
-            double dxc0 = dx[0], dyc0 = dy[0];
-            {
-                int sh = 0;
-                if (wsx == 0) sh = 1;
-                if (wsx + RA - 1 == nxg - 1) sh = -1;
-                if (sh != 0) {
-                    const double *S = SX(i - sh);
-                    double t = 0.0;
-#pragma unroll
-                    for (int m = 0; m < RA; m++) t += S[m] * P(0, wsx + sh + m, j);
-                    dxc0 = t;
-                }
-                sh = 0;
-                if (wsy == 0) sh = 1;
-                if (wsy + RA - 1 == nyg - 1) sh = -1;
-                if (sh != 0) {
-                    const double *S = SY(j - sh);
-                    double t = 0.0;
-#pragma unroll
-                    for (int m = 0; m < RA; m++) t += S[m] * P(0, i, wsy + sh + m);
-                    dyc0 = t;
-                }
-            }
-            const double *cfp = g.cf + i + (size_t)nxg * j;
-            const double A2 = cfp[0], B2 = cfp[nxy], A4 = cfp[2 * (size_t)nxy], B4 = cfp[3 * (size_t)nxy];
-            const double A3 = cfp[4 * (size_t)nxy], B3 = cfp[5 * (size_t)nxy], S5 = cfp[6 * (size_t)nxy];
-            double obot;
-            {
-                constexpr int wz = (1 - A) < 0 ? 0 : (1 - A);
-                const double *Z1 = g.sz + (1 * 2) * RA;
-                double dz = 0.0;
-#pragma unroll
-                for (int m = 0; m < RA; m++) dz += Z1[m] * pc[wz + m];
-                // h_x = A2 * d and h_y = A4 * d with d = 1 / S5
-                const double sg = g.zs[1], d = 1.0 / S5, hx = A2 * d, hy = A4 * d;
-                obot = (S5 + hx * (A2 + sg * B2) + hy * (A4 + sg * B4)) * dz + hx * dx[1] + hy * dy[1];
-            }
-#pragma unroll
-            for (int k = 1; k < NZ - 1; k++) {
-                const int wz = cclamp(k - A, 0, NZ - RA);
-                const double *Z1 = g.sz + (k * 2) * RA, *Z2 = Z1 + RA;
-                double dz = 0.0, dzz = 0.0, dxz = 0.0, dyz = 0.0;
-#pragma unroll
-                for (int m = 0; m < RA; m++) {
-                    const double z1 = Z1[m], cv = pc[wz + m];
-                    dz += z1 * cv;
-                    dzz += Z2[m] * cv;
-                    dxz += z1 * ((wz + m == 0) ? dxc0 : dx[wz + m]);
-                    dyz += z1 * ((wz + m == 0) ? dyc0 : dy[wz + m]);
-                }
-                const double sg = g.zs[k];
-                const double s2 = A2 + sg * B2, s4 = A4 + sg * B4, s3 = A3 + sg * B3;
-                o[k] = o[k] + s3 * dz + 2.0 * (s2 * dxz + s4 * dyz) + (s2 * s2 + s4 * s4 + S5 * S5) * dzz;
-            }
-            o[0] = obot;
-            o[NZ - 1] = pc[NZ - 1];
-        }
-    }
-    __syncthreads();
-    if (active) {
-#pragma unroll
-        for (int k = 0; k < NZ; k++) sP[k * PS + (j - loy) * WX + (i - lox)] = o[k];
-    }
-    __syncthreads();
-    {
-        const int ie = cmin(i0 + TX, nxg), je = cmin(j0 + TY, nyg);
-        for (int jj = j0; jj < je; jj++) {
-            double *dst = out + ((size_t)jj * nxg + i0) * NZ;
-            for (int e = threadIdx.x; e < (ie - i0) * NZ; e += NT) {
-                const int ii = e / NZ, k = e - ii * NZ;
-                dst[e] = sP[k * PS + (jj - loy) * WX + (i0 + ii - lox)];
-            }
-        }
-    }
-}
-
 // The column matvec with the work of each column split between two waves: a block of TX x TY columns
 // has 2 TX TY threads; the first TX TY take the x-side of column t (d/dx, d2/dx2, the first sigma
 // derivative of phi and the mixed x-sigma term, the bottom row), the others the y-side of column
-// t - TX TY (d/dy, d2/dy2, the second sigma derivative and the mixed y-sigma term): four
-// 2A+1-point stencils per level on each side.  The y-side leaves its part of every row in LDS; the x-side
-// adds it.  Each thread holds half the live values of the one-thread-per-column kernel and a block has
-// twice the waves.  Same terms as k_matvec3c; the x and y parts are summed in another order (results agree
-// to rounding).  The live values of a column take about 210 VGPRs (two waves per SIMD), so a block of
-// 4 waves lets two blocks share a CU and one block's window loads overlap the other's arithmetic.  On a
-// 515 x 515 x 10 grid (6th order): 16 x 8 tiles 29.6 us, 32 x 4 32.5 us, 16 x 4 33.1 us, 16 x 16 (one
-// block per CU) 36.3 us.
-template <int NZ, int A, int TX = 16, int TY = 8>
+// t - TX TY (d/dy, d2/dy2, the mixed y-sigma term).  The y-side leaves its part of every row in LDS; the x-side
+// adds it.  Each thread holds half the live values of a one-thread-per-column kernel and a block has
+// twice the waves.  ORDER 0: a row is summed as d2x + d2y, then s3 dz, 2 (s2 dxz + s4 dyz) and the second sigma
+// derivative's term, which the x-side forms; 1: the y-side forms its whole part, with the second sigma derivative,
+// and the x-side adds it last (both are rounding of the same sum; solves that amplify rounding keep the one they use).
+// The live values of a column take about 220 VGPRs (two waves per SIMD), so two blocks share a CU and one block's loads
+// overlap the other's arithmetic; with registers for three it spills (46-56 us where it takes 30).  Bound by the chain of
+// one tile (loads, LDS, four stencils per level, LDS, stores: 8.5 us), four and a half times in a row at 513^2.  With
+// 10 levels, 6th order, at 33^2, 97 x 161, 257^2, 513^2: one thread per column and 16 x 16 tiles 15.5, 14.2, 21.9 and
+// 47.7 us; ORDER 0 10.1, 8.6, 14.3 and 31.6 us; ORDER 1 with the test of the done flag before the loads, the planes
+// loaded where they are used and row-by-row stores 10.7, 8.9, 15.7 and 33.0 us, now 10.0, 8.3, 14.1 and 30.4 us.
+template <int NZ, int A, int TX, int TY, int ORDER>
+struct MvSplit {
+    static constexpr int NC = TX * TY, NT = 2 * NC, RA = 2 * A + 1, R = A + 1, WX = TX + 2 * R, WY = TY + 2 * R, PS = (WX * WY) | 1;
+    static constexpr int YP = ORDER == 0 ? 2 : 1;   // values per row that the y-side passes on
+    static constexpr int ROWS = (TX + 2 + TY + 2) * 2 * RA, LDS = NZ * PS + ROWS + YP * NZ * NC;   // in doubles
+};
+template <int NZ, int A, int TX, int TY, int ORDER>
 __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double *__restrict__ phi, double *__restrict__ out) {
-    if (solve_done(g.skip)) return;
-    constexpr int NC = TX * TY, NT = 2 * NC, RA = 2 * A + 1, R = A + 1, WX = TX + 2 * R, WY = TY + 2 * R;
-    constexpr int PS = (WX * WY) | 1;
-    __shared__ double sP[NZ * PS];
-    __shared__ double sSX[(TX + 2) * 2 * RA];
-    __shared__ double sSY[(TY + 2) * 2 * RA];
-    __shared__ double sYp[NZ * NC];   // y-side part of each row: [k][column]
+    using G = MvSplit<NZ, A, TX, TY, ORDER>;
+    constexpr int NC = G::NC, NT = G::NT, RA = G::RA, R = G::R, WX = G::WX, WY = G::WY, PS = G::PS;
+    __shared__ double lds[G::LDS];
+    double *const sP = lds, *const sSX = lds + NZ * PS, *const sSY = sSX + (TX + 2) * 2 * RA, *const sYp = lds + NZ * PS + G::ROWS;
     const int nxg = g.nxg, nyg = g.nyg, nxy = g.nxy;
     const int gxt = (nxg + TX - 1) / TX;
     const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
@@ -517,9 +385,16 @@ __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double
     const int lox = cmax(cmin(i0 - R, nxg - 2 - 2 * A), 0);
     const int loy = cmax(cmin(j0 - R, nyg - 2 - 2 * A), 0);
     const int wx = cmin(WX, nxg - lox), wy = cmin(WY, nyg - loy);
+    const bool yside = threadIdx.x >= NC;
+    const int col = yside ? (int)threadIdx.x - NC : (int)threadIdx.x;
+    const int tx = col % TX, ty = col / TX;
+    const int i = i0 + tx, j = j0 + ty;
+    const bool active = (i < nxg) && (j < nyg);
+    double cf[7];   // the column's planes A2, B2, A4, B4, A3, B3, S5
     {
-        // window values two at a time (16-byte loads) for an even NZ: rows of columns start at even
-        // offsets, so every pair is aligned and stays inside one window row
+        // every HBM load of the block first, and before the test of the done flag: the phi window (stored level-major;
+        // two values at a time for an even NZ: rows of columns start at even offsets, so every pair is aligned and
+        // stays inside one window row), the stencil rows of its columns and rows, the planes
         constexpr bool PAIRS = NZ % 2 == 0;
         constexpr int W = PAIRS ? 2 : 1;
         constexpr int RL = WX * NZ, TOT = WY * RL, PER = (TOT / W + NT - 1) / NT;
@@ -538,41 +413,47 @@ __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double
                 v[q] = ok ? src[(size_t)r * nxg * NZ + c] : 0.0;
             }
         }
-        for (int e = threadIdx.x; e < (TX + 2) * 2 * RA; e += NT) {
-            const int r = e / (2 * RA), ii = i0 - 1 + r;
-            if (ii >= 0 && ii < nxg) sSX[e] = g.sx[(size_t)ii * 2 * RA + (e - r * 2 * RA)];
+        const double *cfp = g.cf + (active ? i + (size_t)nxg * j : 0);
+#pragma unroll
+        for (int q = 0; q < 7; q++) cf[q] = cfp[(size_t)q * nxy];
+        constexpr int SXN = (TX + 2) * 2 * RA, SYN = (TY + 2) * 2 * RA, SPER = (SXN + SYN + NT - 1) / NT;
+        double sv[SPER];
+#pragma unroll
+        for (int q = 0; q < SPER; q++) {
+            const int e = (int)threadIdx.x + q * NT, f = e < SXN ? e : e - SXN, r = f / (2 * RA), m = f - r * 2 * RA;
+            const int ii = cclamp((e < SXN ? i0 : j0) - 1 + r, 0, (e < SXN ? nxg : nyg) - 1);
+            sv[q] = e < SXN + SYN ? (e < SXN ? g.sx : g.sy)[(size_t)ii * 2 * RA + m] : 0.0;
         }
-        for (int e = threadIdx.x; e < (TY + 2) * 2 * RA; e += NT) {
-            const int r = e / (2 * RA), jj = j0 - 1 + r;
-            if (jj >= 0 && jj < nyg) sSY[e] = g.sy[(size_t)jj * 2 * RA + (e - r * 2 * RA)];
+        if (solve_done(g.skip)) return;
+#pragma unroll
+        for (int q = 0; q < SPER; q++) {
+            const int e = (int)threadIdx.x + q * NT;
+            if (e < SXN + SYN) sSX[e] = sv[q];
         }
 #pragma unroll
         for (int q = 0; q < PER; q++) {
             const int e = ((int)threadIdx.x + q * NT) * W, r = e / RL, c = e - r * RL;
             if (e < TOT && r < wy && c < wx * NZ) {
                 const int cc = c / NZ, k = c - cc * NZ;
-                if constexpr (PAIRS) {
-                    sP[k * PS + r * WX + cc] = v[2 * q];
-                    if (k + 1 < NZ) sP[(k + 1) * PS + r * WX + cc] = v[2 * q + 1];
-                    else sP[r * WX + cc + 1] = v[2 * q + 1];   // level 0 of the next column
+                double *d = sP + k * PS + r * WX + cc;
+                if constexpr (PAIRS) {   // an even NZ: k is even, so k + 1 is the same column's
+                    d[0] = v[2 * q];
+                    d[PS] = v[2 * q + 1];
                 } else {
-                    sP[k * PS + r * WX + cc] = v[q];
+                    d[0] = v[q];
                 }
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
     auto P = [&](int k, int ii, int jj) -> double { return sP[k * PS + (jj - loy) * WX + (ii - lox)]; };
     auto SX = [&](int ii) -> const double * { return sSX + (ii - (i0 - 1)) * 2 * RA; };
     auto SY = [&](int jj) -> const double * { return sSY + (jj - (j0 - 1)) * 2 * RA; };
-    const bool yside = threadIdx.x >= NC;
-    const int col = yside ? (int)threadIdx.x - NC : (int)threadIdx.x;
-    const int tx = col % TX, ty = col / TX;
-    const int i = i0 + tx, j = j0 + ty;
-    const bool active = (i < nxg) && (j < nyg);
     const bool wxl = (i == 0 || i == nxg - 1), wyl = (j == 0 || j == nyg - 1);
     const bool interior = active && !wxl && !wyl;
+    const double A2 = cf[0], B2 = cf[1], A4 = cf[2], B4 = cf[3], A3 = cf[4], B3 = cf[5], S5 = cf[6];
     double o[NZ];
+    double dzk[NZ], zz[NZ], xz[NZ], dz0 = 0.0, dx1 = 0.0;   // ORDER 0: the x-side's derivatives of each row, summed once the y-side's part is there
     if (yside) {
         if (interior) {
             const int wsy = cclamp(j - A, 0, nyg - RA);
@@ -598,14 +479,13 @@ __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double
                     dyc0 = t;
                 }
             }
-            const double *cfp = g.cf + i + (size_t)nxg * j;
-            const double A2 = cfp[0], B2 = cfp[nxy], A4 = cfp[2 * (size_t)nxy], B4 = cfp[3 * (size_t)nxy];
-            const double S5 = cfp[6 * (size_t)nxy];
-            // the second sigma derivative is this side's share of the column's own terms (the x side takes
+            // ORDER 1: the second sigma derivative is this side's share of the column's own terms (the x side takes
             // the first), so that both halves of a column do the same work
             double pc[NZ];
+            if constexpr (ORDER == 1) {
 #pragma unroll
-            for (int k = 0; k < NZ; k++) pc[k] = P(k, i, j);
+                for (int k = 0; k < NZ; k++) pc[k] = P(k, i, j);
+            }
 #pragma unroll
             for (int k = 1; k < NZ - 1; k++) {
                 const int wz = cclamp(k - A, 0, NZ - RA);
@@ -614,14 +494,23 @@ __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double
 #pragma unroll
                 for (int m = 0; m < RA; m++) {
                     dyz += Z1[m] * ((wz + m == 0) ? dyc0 : dy[wz + m]);
-                    dzz += Z2[m] * pc[wz + m];
+                    if constexpr (ORDER == 1) dzz += Z2[m] * pc[wz + m];
                 }
                 const double sg = g.zs[k];
-                const double s2 = A2 + sg * B2, s4 = A4 + sg * B4;
-                o[k] = o[k] + 2.0 * (s4 * dyz) + (s2 * s2 + s4 * s4 + S5 * S5) * dzz;
+                const double s4 = A4 + sg * B4;
+                if constexpr (ORDER == 1) {
+                    const double s2 = A2 + sg * B2;
+                    o[k] = o[k] + 2.0 * (s4 * dyz) + (s2 * s2 + s4 * s4 + S5 * S5) * dzz;
+                } else {
+                    sYp[(NZ + k) * NC + col] = s4 * dyz;
+                }
             }
-            const double d = 1.0 / S5;
-            o[0] = (A4 * d) * dy[1];   // h_y dy at the bottom row (h_y = A4 d, d = 1 / S5)
+            if constexpr (ORDER == 1) {
+                const double d = 1.0 / S5;
+                o[0] = (A4 * d) * dy[1];   // h_y dy at the bottom row (h_y = A4 d, d = 1 / S5)
+            } else {
+                o[0] = dy[1];
+            }
 #pragma unroll
             for (int k = 0; k < NZ - 1; k++) sYp[k * NC + col] = o[k];
         }
@@ -669,53 +558,69 @@ __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double
                     dxc0 = t;
                 }
             }
-            const double *cfp = g.cf + i + (size_t)nxg * j;
-            const double A2 = cfp[0], B2 = cfp[nxy], A4 = cfp[2 * (size_t)nxy], B4 = cfp[3 * (size_t)nxy];
-            const double A3 = cfp[4 * (size_t)nxy], B3 = cfp[5 * (size_t)nxy], S5 = cfp[6 * (size_t)nxy];
             {
                 constexpr int wz = (1 - A) < 0 ? 0 : (1 - A);
                 const double *Z1 = g.sz + (1 * 2) * RA;
                 double dz = 0.0;
 #pragma unroll
                 for (int m = 0; m < RA; m++) dz += Z1[m] * pc[wz + m];
-                const double sg = g.zs[1], d = 1.0 / S5, hx = A2 * d, hy = A4 * d;
-                o[0] = (S5 + hx * (A2 + sg * B2) + hy * (A4 + sg * B4)) * dz + hx * dx[1];
+                if constexpr (ORDER == 1) {
+                    const double sg = g.zs[1], d = 1.0 / S5, hx = A2 * d, hy = A4 * d;
+                    o[0] = (S5 + hx * (A2 + sg * B2) + hy * (A4 + sg * B4)) * dz + hx * dx[1];
+                } else { dz0 = dz; dx1 = dx[1]; }
             }
 #pragma unroll
             for (int k = 1; k < NZ - 1; k++) {
                 const int wz = cclamp(k - A, 0, NZ - RA);
-                const double *Z1 = g.sz + (k * 2) * RA;
-                double dz = 0.0, dxz = 0.0;
+                const double *Z1 = g.sz + (k * 2) * RA, *Z2 = Z1 + RA;
+                double dz = 0.0, dxz = 0.0, dzz = 0.0;
 #pragma unroll
                 for (int m = 0; m < RA; m++) {
                     const double z1 = Z1[m];
                     dz += z1 * pc[wz + m];
+                    if constexpr (ORDER == 0) dzz += Z2[m] * pc[wz + m];
                     dxz += z1 * ((wz + m == 0) ? dxc0 : dx[wz + m]);
                 }
                 const double sg = g.zs[k];
                 const double s2 = A2 + sg * B2, s3 = A3 + sg * B3;
-                o[k] = o[k] + s3 * dz + 2.0 * (s2 * dxz);
+                if constexpr (ORDER == 1) o[k] = o[k] + s3 * dz + 2.0 * (s2 * dxz);
+                else { xz[k] = dxz; dzk[k] = dz; zz[k] = dzz; }
             }
             o[NZ - 1] = pc[NZ - 1];
         }
     }
-    __syncthreads();   // every read of the phi window and every y-side part done
-    if (!yside && active) {
-        if (interior) {
+    lds_barrier();   // every y-side part is there
+    if (!yside && interior) {
+        if constexpr (ORDER == 1) {
 #pragma unroll
             for (int k = 0; k < NZ - 1; k++) o[k] += sYp[k * NC + col];
-        }
+        } else {
+            const double d = 1.0 / S5, hx = A2 * d, hy = A4 * d, sb = g.zs[1];
+            o[0] = (S5 + hx * (A2 + sb * B2) + hy * (A4 + sb * B4)) * dz0 + hx * dx1 + hy * sYp[col];
 #pragma unroll
-        for (int k = 0; k < NZ; k++) sP[k * PS + (j - loy) * WX + (i - lox)] = o[k];
+            for (int k = 1; k < NZ - 1; k++) {
+                const double d2y = sYp[k * NC + col], yz = sYp[(NZ + k) * NC + col], sg = g.zs[k];
+                const double s2 = A2 + sg * B2, s4 = A4 + sg * B4, s3 = A3 + sg * B3;
+                o[k] = (o[k] + d2y) + s3 * dzk[k] + 2.0 * (s2 * xz[k] + yz) + (s2 * s2 + s4 * s4 + S5 * S5) * zz[k];
+            }
+        }
     }
-    __syncthreads();
+    if (!yside && active) {
+#pragma unroll
+        for (int k = 0; k < NZ; k++) sP[col * (NZ | 1) + k] = o[k];
+    }
+    lds_barrier();
     {
+        constexpr int E = NZ % 2 == 0 ? 2 : 1, CH = TX * NZ / E, PER = (TY * CH + NT - 1) / NT;
         const int ie = cmin(i0 + TX, nxg), je = cmin(j0 + TY, nyg);
-        for (int jj = j0; jj < je; jj++) {
-            double *dst = out + ((size_t)jj * nxg + i0) * NZ;
-            for (int e = threadIdx.x; e < (ie - i0) * NZ; e += NT) {
-                const int ii = e / NZ, k = e - ii * NZ;
-                dst[e] = sP[k * PS + (jj - loy) * WX + (i0 + ii - lox)];
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const int e = (int)threadIdx.x + q * NT, r = e / CH, c = (e - r * CH) * E, ii = c / NZ, k = c - ii * NZ;
+            if (r < je - j0 && i0 + ii < ie) {
+                const double *d = sP + (r * TX + ii) * (NZ | 1) + k;
+                double *g2 = out + ((size_t)(j0 + r) * nxg + i0 + ii) * NZ + k;
+                if constexpr (E == 2) *reinterpret_cast<double2 *>(g2) = make_double2(d[0], d[1]);
+                else *g2 = *d;
             }
         }
     }
@@ -2121,45 +2026,6 @@ __global__ __launch_bounds__(128) void k_mg_zebra_t(LvArgs<T> L, int colour, T *
             const int c = e / NZ, k = e - c * NZ;
             dst[e] = sX[((j0 + r - loy) * WX + (i0 + c - lox)) * NZP + k];
         }
-    }
-}
-
-// Columns between HBM and registers, two values per load or store where every column starts on an even element.
-template <typename S>
-struct alignas(2 * sizeof(S)) ColPair { S a, b; };
-template <int NZ, typename S, typename T>
-__device__ __forceinline__ void load_column(const S *__restrict__ p, T (&v)[NZ]) {
-    if constexpr (NZ % 2 == 0) {
-        const ColPair<S> *q = reinterpret_cast<const ColPair<S> *>(p);
-#pragma unroll
-        for (int k = 0; k < NZ / 2; k++) { const ColPair<S> w = q[k]; v[2 * k] = (T)w.a; v[2 * k + 1] = (T)w.b; }
-    } else {
-#pragma unroll
-        for (int k = 0; k < NZ; k++) v[k] = (T)p[k];
-    }
-}
-// N values (a multiple of 16 bytes) from a 16-byte aligned address.
-template <int N, typename T>
-__device__ __forceinline__ void load_record(const T *__restrict__ p, T (&v)[N]) {
-    constexpr int W = 16 / sizeof(T);
-    struct alignas(16) Quad { T e[W]; };
-    static_assert(N % W == 0, "whole 16-byte loads");
-#pragma unroll
-    for (int q = 0; q < N / W; q++) {
-        const Quad w = reinterpret_cast<const Quad *>(p)[q];
-#pragma unroll
-        for (int e = 0; e < W; e++) v[q * W + e] = w.e[e];
-    }
-}
-template <int NZ, typename T, typename O>
-__device__ __forceinline__ void store_column(O *__restrict__ p, const T (&v)[NZ]) {
-    if constexpr (NZ % 2 == 0) {
-        ColPair<O> *q = reinterpret_cast<ColPair<O> *>(p);
-#pragma unroll
-        for (int k = 0; k < NZ / 2; k++) q[k] = ColPair<O>{(O)v[2 * k], (O)v[2 * k + 1]};
-    } else {
-#pragma unroll
-        for (int k = 0; k < NZ; k++) p[k] = (O)v[k];
     }
 }
 

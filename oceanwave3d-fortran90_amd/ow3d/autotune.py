@@ -6,9 +6,8 @@ tank under each candidate and keeps the fastest:
 * the V-cycle schedule: the number of multigrid levels (MGmaxgrids), from the full hierarchy down to the
   fewest levels whose coarsest level the dense solve accepts (at most 4096 unknowns, ow3d.mg_plan);
   fewer levels trade launch-latency-bound small levels for a larger dense coarse solve;
-* the matvec kernel (ow3d_tune: column kernel with the widest tile, with 16 x 8 tiles, with each column
-  split over two waves, or the point kernel), timed with ow3d_time_matvec;
-* the block size of the zebra sweeps (automatic, 256 or 1024 threads).
+* the matvec kernel (ow3d_tune: the column kernel in its two summation orders, or the point kernel), timed with
+  ow3d_time_matvec.
 
 None of these changes results beyond the multigrid depth, which is the reference's own MGmaxgrids
 input (the solve still runs to its tolerance).  Choices are cached by class in tuning.json next to this
@@ -106,7 +105,7 @@ def tune_class(spec, mg_precision=1, warmup=3, steps=3, log=None):
         mv[v] = 1e3 * T.time_matvec(30)
     v_best = min(mv, key=mv.get)
     thr = {}
-    for n in (0, 256, 1024):
+    for n in (0,):   # (the sweeps' block sizes follow from their tiles)
         T.tune(v_best, n)
         thr[n] = 1e3 * _time_steps(T, dt, 1, steps)
     n_best = min(thr, key=thr.get)
