@@ -1020,19 +1020,36 @@ __global__ void k_fill(size_t n, T v, T *__restrict__ y, const int *skip) {
         y[q] = v;
 }
 
-// Block reduction of MAXK accumulators into part[blockIdx.x*MAXK + i].
-// Block sum of NA per-thread accumulators, stored at part[blockIdx.x * PSTRIDE + i] (fixed order).
+// Block sum of NA per-thread accumulators, stored at part[blockIdx.x * PSTRIDE + i] (fixed order: lanes by halves, then the
+// waves).  At each of the first steps over the lanes half of the accumulators go to the other half of the lanes, which
+// sums the same pairs: about NA exchanges for all of them where a reduction of each takes 6 NA.  k_dcgs_a with 18 vectors
+// at 513 x 513 x 10 86.7 us before, 83.9 after (bound by the basis it reads); a 33 x 33 x 9 RK4 step, where the
+// exchanges were a third of the kernel, 8.99 and 8.78 ms.
 template <int NA, int PSTRIDE>
 __device__ __forceinline__ void block_reduce_store(const double (&acc)[NA], double *part) {
+    static_assert(NA <= 64, "one accumulator or more per lane");
+    constexpr int NP = NA <= 1 ? 1 : NA <= 2 ? 2 : NA <= 4 ? 4 : NA <= 8 ? 8 : NA <= 16 ? 16 : NA <= 32 ? 32 : 64;
     __shared__ double red[NA][4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double v[NA];
 #pragma unroll
-    for (int i = 0; i < NA; i++) {
-        double v = acc[i];
+    for (int i = 0; i < NA; i++) v[i] = acc[i];
+    int mine = 0;   // the lane's accumulator
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if (lane == 0) red[i][wv] = v;
+    for (int h = NP / 2, off = 32; h > 0; h >>= 1, off >>= 1) {
+        const bool hi = (lane & off) != 0;
+#pragma unroll
+        for (int q = 0; q < h; q++) {
+            if (q >= NA) continue;
+            const bool two = q + h < NA;
+            const double give = two ? (hi ? v[q] : v[q + h < NA ? q + h : q]) : v[q], keep = two ? (hi ? v[q + h < NA ? q + h : q] : v[q]) : v[q];
+            v[q] = keep + __shfl_xor(give, off, 64);
+        }
+        mine += hi ? h : 0;
     }
+#pragma unroll
+    for (int off = 32 / NP; off > 0; off >>= 1) v[0] += __shfl_xor(v[0], off, 64);
+    if (lane % (64 / NP) == 0 && mine < NA) red[mine][wv] = v[0];
     __syncthreads();
     if (threadIdx.x < NA) {
         const int i = threadIdx.x;
@@ -1197,84 +1214,87 @@ static __global__ void k_gmres_start(KrylovState *S, const double *hv, double rt
     S->g[0] = beta;
 }
 
-// Hessenberg column k (1-based step): col[0..k-1] projections, col[k] = hn the new vector's norm, held in
-// LDS with the previous rotations (cs, sn).  One lane applies the previous rotations and the new one and
-// updates the residual estimate and the stopping test; the caller writes col back as column k - 1 of H.
-__device__ inline void gmres_column(KrylovState *S, int k, double *col, const double *cs, const double *sn, int m) {
+// Value of lane i (uniform) of a wave, in every lane.
+__device__ __forceinline__ double lane_value(double v, int i) {
+    union { double d; int w[2]; } u;
+    u.d = v;
+    u.w[0] = __builtin_amdgcn_readlane(u.w[0], i);
+    u.w[1] = __builtin_amdgcn_readlane(u.w[1], i);
+    return u.d;
+}
+// Hessenberg column k (1-based step) of one wave: lane i holds col[i] (col[0..k-1] projections, col[k] = hn the new vector's
+// norm) and the previous rotations cs[i], sn[i].  Applies the previous rotations and the new one, updates the residual
+// estimate and the stopping test, and returns the rotated column, which the caller writes as column k - 1 of H.  The
+// chain over the rotations reads the lanes' registers: from LDS each of its k steps waited for the store before it.
+// g0 = S->g[k - 1], tol = S->tol, matvecs = S->matvecs.
+__device__ __forceinline__ double gmres_column(KrylovState *S, int k, double col, double cs, double sn, int m, double g0, double tol, int matvecs) {
     constexpr int M = KRYLOV_MAXK;
-    const double hn = col[k];
+    const int t = threadIdx.x;
+    const double hn = lane_value(col, k);
+    double a = lane_value(col, 0), out = col;
     for (int i = 0; i < k - 1; i++) {
-        const double a = col[i], b = col[i + 1];
-        col[i] = cs[i] * a + sn[i] * b;
-        col[i + 1] = cs[i] * b - sn[i] * a;
+        const double b = lane_value(col, i + 1), c = lane_value(cs, i), s = lane_value(sn, i);
+        const double top = c * a + s * b;
+        a = c * b - s * a;
+        if (t == i) out = top;
     }
-    const double a = col[k - 1], b = col[k];
+    const double b = hn;
     const double rr = sqrt(a * a + b * b);
     double c = 1.0, sv = 0.0;
     if (rr > 0.0) { c = a / rr; sv = b / rr; }
-    S->cs[k - 1] = c; S->sn[k - 1] = sv;
-    col[k - 1] = rr;
-    col[k] = hn;
-    const double g0 = S->g[k - 1];
-    S->g[k] = -sv * g0;
-    S->g[k - 1] = c * g0;
-    const double est = fabs(-sv * g0);
-    S->est = est; S->k = k;
-    S->scale = hn > 0.0 ? 1.0 / hn : 1.0;
-    if (!(k < m && !(est <= S->tol) && S->matvecs < m) || hn == 0.0 || k + 1 >= M) S->done = 1;
+    if (t == k - 1) out = rr;
+    if (t == k) out = hn;
+    if (t == 0) {
+        S->cs[k - 1] = c; S->sn[k - 1] = sv;
+        S->g[k] = -sv * g0;
+        S->g[k - 1] = c * g0;
+        const double est = fabs(-sv * g0);
+        S->est = est; S->k = k;
+        S->scale = hn > 0.0 ? 1.0 / hn : 1.0;
+        if (!(k < m && !(est <= tol) && matvecs < m) || hn == 0.0 || k + 1 >= M) S->done = 1;
+    }
+    return out;
 }
 
 // Arnoldi step k, first pass: hv[0..k-1] = V_i . w, hv[k] = w . w (classical Gram-Schmidt).  Keeps the
 // column when the projection removed at most half of the squared norm, else asks for the second pass.
-// One wave: the vectors are staged in LDS by all lanes, the serial part runs on lane 0.
+// One wave: lane i holds entry i.
 static __global__ __launch_bounds__(64) void k_gmres_pass1(KrylovState *S, const double *hv, int k, int m) {
     constexpr int M = KRYLOV_MAXK;
-    __shared__ double col[M + 1], cs[M], sn[M];
-    __shared__ int second;
-    if (S->done) return;
     const int t = threadIdx.x;
-    if (t <= k) col[t] = hv[t];
-    if (t < k - 1) { cs[t] = S->cs[t]; sn[t] = S->sn[t]; }
-    __syncthreads();
-    if (t == 0) {
-        S->matvecs += 1;
-        const double nrm2 = col[k];
-        double nn = nrm2;
-        for (int i = 0; i < k; i++) nn -= col[i] * col[i];
-        second = !(nn > 0.5 * nrm2);
-        if (!second) {
-            col[k] = sqrt(nn);
-            gmres_column(S, k, col, cs, sn, m);
-        }
-        S->skip2 = second ? 0 : 1;
-    }
-    __syncthreads();
+    double col = t <= k ? hv[t] : 0.0;
+    const double cs = t < k - 1 ? S->cs[t] : 0.0, sn = t < k - 1 ? S->sn[t] : 0.0, g0 = S->g[k - 1], tol = S->tol;
+    const int matvecs = S->matvecs + 1;
+    if (S->done) return;
+    const double nrm2 = lane_value(col, k);
+    double nn = nrm2;
+    for (int i = 0; i < k; i++) { const double c = lane_value(col, i); nn -= c * c; }
+    const bool second = !(nn > 0.5 * nrm2);
+    if (t == 0) { S->matvecs = matvecs; S->skip2 = second ? 0 : 1; }
     if (second) {
-        if (t < k) S->h1[t] = col[t];
-    } else if (t <= k) {
-        S->H[t * M + (k - 1)] = col[t];
+        if (t < k) S->h1[t] = col;
+    } else {
+        if (t == k) col = sqrt(nn);
+        col = gmres_column(S, k, col, cs, sn, m, g0, tol, matvecs);
+        if (t <= k) S->H[t * M + (k - 1)] = col;
     }
 }
 
 // Arnoldi step k, second (DGKS) pass: hv holds the projections of the once-orthogonalised vector.
 static __global__ __launch_bounds__(64) void k_gmres_pass2(KrylovState *S, const double *hv, int k, int m) {
     constexpr int M = KRYLOV_MAXK;
-    __shared__ double col[M + 1], h2[M + 1], cs[M], sn[M];
-    if (S->skip2) return;
     const int t = threadIdx.x;
-    if (t <= k) h2[t] = hv[t];
-    if (t < k) col[t] = S->h1[t];
-    if (t < k - 1) { cs[t] = S->cs[t]; sn[t] = S->sn[t]; }
-    __syncthreads();
-    if (t == 0) {
-        double n2 = h2[k];
-        for (int i = 0; i < k; i++) { n2 -= h2[i] * h2[i]; col[i] = col[i] + h2[i]; }
-        col[k] = sqrt(fmax(n2, 0.0));
-        gmres_column(S, k, col, cs, sn, m);
-        S->skip2 = 1;
-    }
-    __syncthreads();
-    if (t <= k) S->H[t * M + (k - 1)] = col[t];
+    const double h2 = t <= k ? hv[t] : 0.0, h1 = t < k ? S->h1[t] : 0.0;
+    const double cs = t < k - 1 ? S->cs[t] : 0.0, sn = t < k - 1 ? S->sn[t] : 0.0, g0 = S->g[k - 1], tol = S->tol;
+    const int matvecs = S->matvecs;
+    if (S->skip2) return;
+    double n2 = lane_value(h2, k);
+    for (int i = 0; i < k; i++) { const double c = lane_value(h2, i); n2 -= c * c; }
+    double col = h1 + h2;
+    if (t == k) col = sqrt(fmax(n2, 0.0));
+    col = gmres_column(S, k, col, cs, sn, m, g0, tol, matvecs);
+    if (t == 0) S->skip2 = 1;
+    if (t <= k) S->H[t * M + (k - 1)] = col;
 }
 
 // One-reduction classical Gram-Schmidt with reorthogonalisation (DCGS2: Swirydowicz, Langou, Ananthan,
@@ -1412,30 +1432,46 @@ __global__ __launch_bounds__(256) void k_dcgs_b2(size_t n, const double *__restr
 // Step k: d = the first pass's dots (k), e = the second pass's dots and squared norm (k + 1).  Completes
 // Hessenberg column k - 1, rotates it, updates the residual estimate and the stopping test, and keeps c'
 // and the new inverse norm for the next step.
+// One wave, a chain of latencies: everything is loaded before the first wait, the rows of H go to LDS (padded), the rest
+// stays in the lanes' registers.  With one load per term of the sums and the rotations in LDS it took 6.8 us on average
+// over a 513 x 513 solve and 5.1 us at 33 x 33, now 5.4 and 4.4.
 static __global__ __launch_bounds__(64) void k_dcgs_column(KrylovState *S, const double *d, const double *e, int k, int m) {
-    constexpr int M = KRYLOV_MAXK;
-    __shared__ double col[M + 1], cs[M], sn[M];
-    if (S->done) return;
+    constexpr int M = KRYLOV_MAXK, PITCH = M + 1, PER = M * (M - 1) / 64;
+    __shared__ double sH[(M - 1) * PITCH];
     const int t = threadIdx.x;
-    if (t < k) {   // h_t = (d_t - sum_j H(t, j) c_j) ib over the columns j = t-1 .. k-2 that have row t
-        double acc = d[t];
-        for (int j = t > 0 ? t - 1 : 0; j <= k - 2; j++) acc -= S->Hr[t * M + j] * S->cv[j];
-        col[t] = acc * S->ib + e[t];
+    double hr[PER + 1];
+#pragma unroll
+    for (int q = 0; q <= PER; q++) hr[q] = t + q * 64 < k * M ? S->Hr[t + q * 64] : 0.0;
+    const double dv = t < k ? d[t] : 0.0, ev = t <= k ? e[t] : 0.0, cv = t < k - 1 ? S->cv[t] : 0.0;
+    const double cs = t < k - 1 ? S->cs[t] : 0.0, sn = t < k - 1 ? S->sn[t] : 0.0, ib = S->ib, g0 = S->g[k - 1], tol = S->tol;
+    const int matvecs = S->matvecs + 1;
+    if (S->done) return;
+#pragma unroll
+    for (int q = 0; q <= PER; q++) {
+        const int c = t + q * 64;
+        if (c < k * M) sH[c / M * PITCH + c % M] = hr[q];
     }
-    if (t < k - 1) { cs[t] = S->cs[t]; sn[t] = S->sn[t]; }
     __syncthreads();
+    // h_t = (d_t - sum_j H(t, j) c_j) ib over the columns j = t-1 .. k-2 that have row t
+    double acc = dv;
+    const double *row = sH + cmin(t, k - 1) * PITCH;
+    for (int j = 0; j <= k - 2; j++) {
+        const double c = lane_value(cv, j), h = row[j];
+        if (j >= t - 1) acc -= h * c;
+    }
+    double col = acc * ib + ev;
+    double n2 = lane_value(ev, k);
+    for (int i = 0; i < k; i++) { const double c = lane_value(ev, i); n2 -= c * c; }
+    const double hn = sqrt(fmax(n2, 0.0));
+    if (t == k) col = hn;
+    if (t <= k) S->Hr[t * M + (k - 1)] = col;
+    if (t < k) S->cv[t] = ev;
     if (t == 0) {
-        S->matvecs += 1;
-        double n2 = e[k];
-        for (int i = 0; i < k; i++) n2 -= e[i] * e[i];
-        col[k] = sqrt(fmax(n2, 0.0));
-        for (int i = 0; i <= k; i++) S->Hr[i * M + (k - 1)] = col[i];
-        for (int i = 0; i < k; i++) S->cv[i] = e[i];
-        S->ib = col[k] > 0.0 ? 1.0 / col[k] : 1.0;
-        gmres_column(S, k, col, cs, sn, m);
+        S->matvecs = matvecs;
+        S->ib = hn > 0.0 ? 1.0 / hn : 1.0;
     }
-    __syncthreads();
-    if (t <= k) S->H[t * M + (k - 1)] = col[t];
+    col = gmres_column(S, k, col, cs, sn, m, g0, tol, matvecs);
+    if (t <= k) S->H[t * M + (k - 1)] = col;
 }
 
 __device__ inline void solve_stats(KrylovState *S) {
