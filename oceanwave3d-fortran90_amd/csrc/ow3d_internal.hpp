@@ -114,6 +114,7 @@ size_t line_records(int nxg, int nyg, int nzg) {
 // k_mg_bottom on levels 0 .. top: values of its tables at most, and LDS elements of the iterate and right-hand side of each
 // level (columns padded to an odd stride above level 0), the finest one's residual and the tables, whose offsets go to
 // A (unless NULL).
+constexpr size_t BOTTOM_LDS = 160 << 10;   // bytes a workgroup may have
 inline size_t bottom_tables(const std::vector<Grid> &lv, int top) {
     size_t n = 0;
     for (int k = 1; k <= top; k++)   // rows 6, prolongation 3, restriction 4 (coarse) per column and row; 3 and 3 per level

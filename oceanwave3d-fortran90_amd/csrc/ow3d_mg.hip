@@ -18,7 +18,7 @@ bool needs_r(const ow3d_tank *t, int k) {
 }
 
 namespace {
-constexpr size_t BOTTOM_DENSE = 512 << 10, BOTTOM_LDS = 160 << 10;
+constexpr size_t BOTTOM_DENSE = 512 << 10;
 }  // namespace
 // One compute unit reads about 60-100 GB/s: an inverse of more than BOTTOM_DENSE bytes is read by all of them.
 bool bottom_split(const ow3d_tank *t) {

@@ -454,7 +454,8 @@ int fill_bottom(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, Bott
     }
     const BottomKernel<T> kernel = bottom_kernel<T>(B.g.nzg, B.args.dim3);
     if (!kernel) { err() = "bottom level depth outside 3..14"; return -1; }
-    HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)t->bot_lds));
+    // (the attribute belongs to the kernel, which tanks share: the same value for all)
+    HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BOTTOM_LDS));
     HIPCHK(dA.alloc(1));
     HIPCHK(hipMemcpy(dA.p, &A, sizeof(A), hipMemcpyHostToDevice));
     return 0;
