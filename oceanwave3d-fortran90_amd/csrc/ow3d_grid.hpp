@@ -75,6 +75,23 @@ inline void build_stencils(const std::vector<double> &x, int N, int half, std::v
     }
 }
 
+// True when the 3-point rows S[N][2][3] of nodes 2 .. N-3 are the centred rows of a uniform grid: all
+// equal (to 1e-12) to the middle node's, with a zero centre weight in the first derivative.  c receives
+// the first-derivative weight of the right neighbour, the second-derivative neighbour and centre weights.
+inline bool uniform_rows(const std::vector<double> &S, int N, double *c) {
+    if (N < 5) return false;
+    const double *R = &S[(size_t)(N / 2) * 6];
+    c[0] = R[2]; c[1] = R[3]; c[2] = R[4];
+    const double t1 = 1e-12 * std::fabs(c[0]), t2 = 1e-12 * std::fabs(c[2]);
+    for (int i = 2; i <= N - 3; i++) {
+        const double *Q = &S[(size_t)i * 6];
+        if (std::fabs(Q[0] + c[0]) > t1 || std::fabs(Q[1]) > t1 || std::fabs(Q[2] - c[0]) > t1 ||
+            std::fabs(Q[3] - c[1]) > t2 || std::fabs(Q[4] - c[2]) > t2 || std::fabs(Q[5] - c[1]) > t2)
+            return false;
+    }
+    return true;
+}
+
 inline void grid_stencils(Grid &g) {
     if (g.nx > 1) build_stencils(g.x, g.nxg, g.a, g.sx);
     if (g.ny > 1) build_stencils(g.y, g.nyg, g.b, g.sy);

@@ -2686,7 +2686,8 @@ __global__ __launch_bounds__((SweepTile<NZ, TX, TY>::NT)) void k_mg_sweep(LvArgs
             for (int k = 0; k < NZ; k++) d[k] = T(0);
         }
     }
-    if (ZB || (ZX && !wall && L.uni)) half(red, std::integral_constant<bool, ZX || ZB>{});
+    // (MODE 1 away from the walls: nothing is staged, so the red columns must not read their neighbours)
+    if (ZB || (ZX && !wall)) half(red, std::integral_constant<bool, ZX || ZB>{});
     else half(red, std::false_type{});
     lds_barrier();
     half(black, std::false_type{});
