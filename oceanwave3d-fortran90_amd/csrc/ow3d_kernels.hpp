@@ -83,6 +83,11 @@ __device__ __forceinline__ void store_column(O *__restrict__ p, const T (&v)[NZ]
 // ---------------------------------------------------------------------------------------------
 // High-order matvec  (BuildLinearSystem.f90:1-290)
 // ---------------------------------------------------------------------------------------------
+// Two values of the matvec's result as one store.  A device-pointer caller's y is only 8-byte aligned
+// (ow3d_laplace_apply_device); global memory takes 16-byte stores at any multiple of 4.
+struct OutPair { double a, b; };
+static_assert(alignof(OutPair) == 8, "y's alignment");
+
 struct MvArgs {
     int nxg, nyg, nxy;
     const double *sx, *sy, *sz;  // stencil rows [N][2][2A+1]
@@ -619,7 +624,7 @@ __global__ __launch_bounds__(2 * TX * TY) void k_matvec3s(MvArgs g, const double
             if (r < je - j0 && i0 + ii < ie) {
                 const double *d = sP + (r * TX + ii) * (NZ | 1) + k;
                 double *g2 = out + ((size_t)(j0 + r) * nxg + i0 + ii) * NZ + k;
-                if constexpr (E == 2) *reinterpret_cast<double2 *>(g2) = make_double2(d[0], d[1]);
+                if constexpr (E == 2) *reinterpret_cast<OutPair *>(g2) = OutPair{d[0], d[1]};
                 else *g2 = *d;
             }
         }
