@@ -175,6 +175,9 @@ long long ow3d_estimate_bytes(const ow3d_config *cfg);
 /* Multigrid hierarchy ow3d_create would build for cfg: number of levels and unknowns of the coarsest
  * (solved with its dense inverse; at most 4096).  Host only. */
 int ow3d_mg_plan(const ow3d_config *cfg, int *nlev, int *coarsest);
+/* Finest multigrid level that the handle's one-workgroup kernel takes, with all coarser ones (0: the coarsest level);
+ * -1: every level has launches of its own. */
+int ow3d_mg_bottom_level(const ow3d_tank *t);
 
 #ifdef __cplusplus
 }

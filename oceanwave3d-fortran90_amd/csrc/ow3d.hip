@@ -465,6 +465,8 @@ extern "C" int ow3d_dims(const ow3d_tank *t, int *nxg, int *nyg, int *nzg, int *
     return 0;
 }
 
+extern "C" int ow3d_mg_bottom_level(const ow3d_tank *t) { return t ? t->bot_top : -1; }
+
 extern "C" void *ow3d_stream(ow3d_tank *t) { return t ? (void *)t->s : nullptr; }
 
 extern "C" int ow3d_laplace_apply_device(ow3d_tank *t, const double *d_phi, double *d_y, void *stream) {

@@ -55,7 +55,7 @@ EXPORTS = ["ow3d_create", "ow3d_destroy", "ow3d_dims", "ow3d_last_error", "ow3d_
            "ow3d_rhs_free_surface", "ow3d_add_relax_zone", "ow3d_set_state", "ow3d_get_state",
            "ow3d_rk4_steps", "ow3d_stats", "ow3d_laplace_apply_device", "ow3d_stream",
            "ow3d_time_matvec", "ow3d_batch_rk4_steps", "ow3d_rk4_steps_async", "ow3d_query", "ow3d_wait",
-           "ow3d_device_bytes", "ow3d_estimate_bytes", "ow3d_step_stats", "ow3d_tune", "ow3d_mg_plan", "ow3d_kinematics", "ow3d_steps_status",
+           "ow3d_device_bytes", "ow3d_estimate_bytes", "ow3d_step_stats", "ow3d_tune", "ow3d_mg_plan", "ow3d_mg_bottom_level", "ow3d_kinematics", "ow3d_steps_status",
            "ow3d_solve_noalloc", "ow3d_kinematics_gradients", "ow3d_surface_slopes"]
 
 
@@ -106,6 +106,7 @@ def lib():
         L.ow3d_kinematics.argtypes = [P, D, D, D, D]
         L.ow3d_kinematics_gradients.argtypes = [P, D, D]
         L.ow3d_surface_slopes.argtypes = [P, D, D]
+        L.ow3d_mg_bottom_level.argtypes = [P]
         L.ow3d_mg_plan.argtypes = [ctypes.POINTER(Config), IP, IP]
         L.ow3d_step_stats.argtypes = [P, ctypes.POINTER(ctypes.c_longlong), ctypes.POINTER(ctypes.c_longlong), D]
         L.ow3d_estimate_bytes.restype = ctypes.c_longlong
@@ -265,6 +266,10 @@ class Tank:
 
     def device_bytes(self):
         return int(lib().ow3d_device_bytes(self.h))
+
+    def mg_bottom_level(self):
+        """Finest multigrid level of the one-workgroup kernel (0: the coarsest level), -1 if it is not used."""
+        return int(lib().ow3d_mg_bottom_level(self.h))
 
     def step_stats(self):
         """(replays, captures, capture_ms): speculative steps rolled back and replayed with the whole
