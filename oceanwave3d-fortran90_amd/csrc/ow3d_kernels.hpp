@@ -3293,7 +3293,8 @@ __device__ __forceinline__ void residual_rows(const LvArgs<T> &L, int i, int j, 
         const T om = T(1) - L.zs[1];
         const T s2 = om * cp[3], s4 = om * cp[4], s5 = cp[0], hx = cp[1], hy = D3 ? cp[2] : T(0);
         const T dz = dot3(Z1, xc[0], xc[1], xc[2]), cz = fma1(hy, s4, fma1(hx, s2, s5));
-        o[0] = b[0] - fma1(hy, dyl[1], fma1(cz, dz, hx * dxl[1]));
+        // (read by the restriction onto a sigma-coarsened level only: there it must round as k_mg_residual_t does)
+        o[0] = b[0] - fma1(hy, dyl[1], fma1(hx, dxl[1], cz * dz));
     }
 }
 

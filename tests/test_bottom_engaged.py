@@ -56,3 +56,31 @@ def test_v_cycle_matches_the_oracle(oracle_mod, nx, ny, nz, mg, kw):
         assert np.max(np.abs(T.precond_apply(scale * r) - scale * want)) <= TOL[mg] * abs(scale) * np.max(np.abs(want))
     T.close()
     O.close()
+
+
+def smooth(shape, rng):
+    """A residual whose V cycle lives on the coarse levels: a few long waves."""
+    j, i, k = np.meshgrid(*[np.arange(n) for n in shape], indexing="ij")
+    r = np.zeros(shape)
+    for q in range(4):
+        a = rng.uniform(0, 0.5, 3)
+        a[q % 3] *= 0.1
+        r += rng.standard_normal() * np.cos(a[0] * j + rng.uniform(0, 6)) * np.cos(a[1] * i + rng.uniform(0, 6)) * np.cos(a[2] * k + 1)
+    return r
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mg", [0, 1, 2])
+@pytest.mark.parametrize("nx,ny,nz,kw", CASES + [(25, 49, 13, dict(nu1=2, nu2=1)), (49, 33, 11, {}), (13, 13, 13, {})])
+def test_same_bits_as_one_launch_per_step(nx, ny, nz, mg, kw):
+    T, _, _ = tank(nx, ny, nz, mg, kw)
+    W, _, _ = tank(nx, ny, nz, mg, kw, bottom=False)
+    rng = np.random.default_rng(nx * ny + nz)
+    # one rounding of a coarse level reaches the finest in one vector of several only
+    for n in range(24):
+        r = smooth(T.shape3, rng) * (1.0 + (n % 2) * 0.1 * rng.standard_normal(T.shape3))
+        want = W.precond_apply(r)
+        assert np.abs(want).max() > 0
+        assert np.array_equal(T.precond_apply(r), want), n
+    T.close()
+    W.close()
