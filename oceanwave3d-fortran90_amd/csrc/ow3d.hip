@@ -1059,10 +1059,15 @@ extern "C" long long ow3d_estimate_bytes(const ow3d_config *cfg) {
         std::vector<Grid> lev;
         if (!mg_levels(g, cfg->mg_maxgrids, lev, err())) return -1;
         const long long p = cfg->mg_precision == 0 ? 8 : 4, pc = cfg->mg_precision == 2 ? 2 : p;
-        ow3d_tank probe;   // the hierarchy and the settings that needs_b and needs_r read
+        ow3d_tank probe;   // the hierarchy and the choices ow3d_create would make for it
         probe.cfg = *cfg;
         probe.levels = lev;
-        probe.bot_top = bottom_top(&probe);
+        mg_choices(&probe);
+        if (probe.bot_top >= 0) {   // tables, arguments and (around a dense solve of its own) LDS image of the one-workgroup kernel
+            BottomArgs<double> A;
+            bottom_layout<double>(lev, probe.bot_top, &A);
+            b += p * (long long)(bottom_tables(lev, probe.bot_top) + (probe.bot_split ? A.image : 0)) + (long long)(p == 8 ? sizeof(BottomArgs<double>) : sizeof(BottomArgs<float>));
+        }
         for (size_t k = 0; k < lev.size(); k++) {
             const Grid &L = lev[k];
             b += p * ((long long)L.n * (2 + needs_b(&probe, (int)k) + needs_r(&probe, (int)k)) + 6LL * L.nxy + 12LL * (L.nxg + L.nyg + L.nzg)) + 8LL * (L.nxg + L.nyg + L.nzg);

@@ -238,8 +238,9 @@ int launch_matvec(const ow3d_tank *t, const double *phi, double *y, hipStream_t 
 bool matvec_supported(int nzg, int A);
 // multigrid (ow3d_mg.hip): hierarchy set-up for t->cfg and u = M^-1 r on device vectors
 int mg_setup(ow3d_tank *t);
-int bottom_top(const ow3d_tank *t);   // t->bot_top from t->levels and the settings
-bool bottom_split(const ow3d_tank *t);   // t->bot_split
+// Choices that follow from t->cfg, t->levels and the environment: fused_rb (OW3D_MG_FUSED_RB=0: off), bot_lim
+// (OW3D_MG_BOTTOM: most points of a level of the one-workgroup kernel, 0 = none), bot_top and bot_split.
+void mg_choices(ow3d_tank *t);
 // Buffers of level k that some path uses (t->levels, t->fused_rb and t->bot_top are set): the right-hand side, except
 // on an FP64 finest level whose first sweep reads the residual itself, and the residual, except where it goes into its
 // restriction in one launch.

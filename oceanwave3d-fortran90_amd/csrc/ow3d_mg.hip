@@ -19,7 +19,6 @@ bool needs_r(const ow3d_tank *t, int k) {
 
 namespace {
 constexpr size_t BOTTOM_DENSE = 512 << 10;
-}  // namespace
 // One compute unit reads about 60-100 GB/s: an inverse of more than BOTTOM_DENSE bytes is read by all of them.
 bool bottom_split(const ow3d_tank *t) {
     const size_t n = t->levels[0].n, p = t->cfg.mg_precision == 0 ? 8 : t->cfg.mg_precision == 2 ? 2 : 4;
@@ -44,9 +43,17 @@ int bottom_top(const ow3d_tank *t) {
     }
     return top < 2 && bottom_split(t) ? -1 : top;
 }
+}  // namespace
+
+void mg_choices(ow3d_tank *t) {
+    if (const char *e = std::getenv("OW3D_MG_BOTTOM")) t->bot_lim = std::atol(e);
+    if (const char *e = std::getenv("OW3D_MG_FUSED_RB")) t->fused_rb = e[0] != '0';
+    t->bot_top = bottom_top(t);
+    t->bot_split = bottom_split(t);
+}
 
 // Multigrid hierarchy of the tank (MGPreProcess.f90:6-460 with coarsening strategy 0), level operators in
-// the precision the configuration asks for, and the levels handed to the one-workgroup kernel (OW3D_MG_BOTTOM: most points of such a level, 0 = none).
+// the precision the configuration asks for, and the levels handed to the one-workgroup kernel.
 int mg_setup(ow3d_tank *t) {
     const ow3d_config &c = t->cfg;
     if (!mg_levels(t->g, c.mg_maxgrids, t->levels, err())) return -1;
@@ -54,10 +61,7 @@ int mg_setup(ow3d_tank *t) {
     for (auto &L : t->levels)
         if (L.nzg < 3 || L.nzg > 14) { err() = "multigrid level depth outside 3..14"; return -1; }
     if (t->levels[0].n > 4096) { err() = "coarsest multigrid level too large for the dense solve"; return -1; }
-    if (const char *e = std::getenv("OW3D_MG_BOTTOM")) t->bot_lim = std::atol(e);
-    if (const char *e = std::getenv("OW3D_MG_FUSED_RB")) t->fused_rb = e[0] != '0';
-    t->bot_top = bottom_top(t);
-    t->bot_split = bottom_split(t);
+    mg_choices(t);
     if (c.mg_precision == 0 ? mg_build64(t) : mg_build32(t)) return -1;
     return c.mg_precision == 0 ? mg_fill_bottom64(t) : mg_fill_bottom32(t);
 }
