@@ -1020,7 +1020,6 @@ extern "C" int ow3d_tune(ow3d_tank *t, int matvec_variant, int sweep_threads) {
     HIPCHK(hipStreamSynchronize(t->s));
     std::lock_guard<std::mutex> lk(capture_lock());
     t->mv_variant = matvec_variant;
-    t->rb_threads = sweep_threads;
     t->drop_step_graphs();   // captured with the old launch shapes
     if (t->pg_exec) { HIPCHK(hipGraphExecDestroy(t->pg_exec)); t->pg_exec = nullptr; }
     return 0;

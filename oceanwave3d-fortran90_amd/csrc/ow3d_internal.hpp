@@ -178,10 +178,9 @@ struct ow3d_tank {
     DevBuf<double> bot_tab, bot_img;  // its tables, and its LDS image between the parts
     int bot_top = -1;                 // finest level handled by the one-workgroup bottom kernel (-1: none)
     bool fused_rb = true;             // one launch per zebra sweep (red and black halves) on the upper levels
-    // launch choices (ow3d_tune): matvec variant 0 column kernel, widest tile / 1 column kernel, 8-row
-    // tiles / 2 point kernel; zebra-sweep block size 0 / 256 / 1024 (kept for callers; the sweeps have one block size)
+    // matvec kernel (ow3d_tune): 0 and 1 split column kernel, x and y terms of a row summed first / 2 point kernel / 3 split
+    // column kernel, y terms added last
     int mv_variant = 0;
-    int rb_threads = 0;
     BottomArgs<double> bot64{};
     BottomArgs<float> bot32{};
     DevBuf<BottomArgs<double>> bot64d;   // device copies read by the bottom kernel

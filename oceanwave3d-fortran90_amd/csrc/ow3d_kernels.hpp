@@ -1617,7 +1617,6 @@ struct CoefLds {
 // Stages the coefficients of the window [lox, lox+wcols) x [loy, loy+wrows) (row length MW) into buf
 // (CoefLds<MW, MH, NZ>::TOTAL elements) and returns the accessor.  Each segment is one predicated load per
 // element with no branches around it, so all loads of a thread are in flight together.
-// CoefRegs holds the two halves separately (load into registers, store to LDS), as WindowRegs.
 template <typename T, int NZ, int MW, int MH, int NT>
 struct CoefRegs {
     using S = CoefLds<MW, MH, NZ>;
@@ -1667,13 +1666,6 @@ struct CoefRegs {
         return C;
     }
 };
-template <typename T, int NZ, int MW, int MH, int NT>
-__device__ __forceinline__ CoefS<T> stage_coefs(const LvArgs<T> &L, int lox, int loy, int wcols, int wrows, T *buf) {
-    CoefRegs<T, NZ, MW, MH, NT> c;
-    c.load(L, lox, loy, wcols, wrows);
-    return c.store(buf);
-}
-
 // Coefficients of the linearised (eta = 0) level operator at sigma level k: with eta = 0 the sigma
 // coefficients (DetermineTransformationConstantsArray.f90:190-201) are (1 - sigma) times per-column
 // constants, precomputed at set-up (planes 3, 4, 5 and 0 of col).
@@ -3187,40 +3179,6 @@ __global__ void k_mg_prolong_add_t(RestrictGeo G, const T *__restrict__ ec, T *_
     xf[q] = x0 + e;
 }
 
-// Restriction onto a coarse level coarsened in x and y but not in sigma (kc = kf), with the 3-point weights
-// of each coarse column and row from tables (restrict_at's values: the fine residual smoothed along x on
-// the coarse point's row and its two neighbour rows, injected on wall ghost rows, then along y; injected on
-// the top level; zero on coarse ghost points).  Also clears the coarse iterate.
-template <typename T, int NZC>
-__global__ void k_mg_restrict_tab(RestrictGeo G, const T *__restrict__ rxw, const T *__restrict__ ryw, const T *__restrict__ rf,
-                                  T *__restrict__ rc, T *__restrict__ xz) {
-    if (!G.spec && solve_done(G.skip)) return;
-    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (t >= G.nxgc * NZC) return;
-    const int ic = t / NZC, k = t - ic * NZC, jc = (int)blockIdx.y;
-    const int icn = ic - G.gx, jcn = jc - G.gy;
-    T v = T(0);
-    if (k >= 1 && icn >= 0 && icn < G.nxc && jcn >= 0 && jcn < G.nyc) {
-        const int i = G.gx + 2 * icn, j = G.gy + 2 * jcn;
-        auto R = [&](int ii, int jj) -> T { return rf[((size_t)jj * G.nxgf + ii) * NZC + k]; };
-        if (k <= G.nzf - 1) {
-            const T x0 = rxw[4 * ic], x1 = rxw[4 * ic + 1], x2 = rxw[4 * ic + 2], ax = rxw[4 * ic + 3];
-            auto Xv = [&](int jj) -> T {
-                if (jj < G.gy || jj > G.nyf + G.gy - 1) return R(i, jj);
-                return ax * ((x0 * R(i - 1, jj) + x1 * R(i, jj)) + x2 * R(i + 1, jj));
-            };
-            const T y0 = ryw[4 * jc], y1 = ryw[4 * jc + 1], y2 = ryw[4 * jc + 2], ay = ryw[4 * jc + 3];
-            v = ay * ((y0 * Xv(j - 1) + y1 * Xv(j)) + y2 * Xv(j + 1));
-        } else {
-            v = R(i, j);
-        }
-    }
-    if (G.spec && solve_done(G.skip)) return;
-    const size_t q = (size_t)jc * G.nxgc * NZC + t;
-    if (xz) xz[q] = T(0);
-    rc[q] = v;
-}
-
 // Residual of a column from its rows (residual_column's arithmetic, its roundings written out): c its level 0 in
 // LDS, x- and y-neighbours at +- SXS and +- SYS; i, j the column (wall columns take the rows of the
 // column beside them).
@@ -3305,7 +3263,7 @@ struct ResRestrictLds {
     static constexpr int TOTAL = WX * WY * NZP;
 };
 // Residual of a level and its restriction onto a coarse level coarsened in x and y but not in sigma, in one
-// launch (k_mg_residual_t followed by k_mg_restrict_tab, same arithmetic).  A block owns CX x CY coarse
+// launch (the arithmetic of k_mg_residual_t, then of restrict_at with the weights from tables).  A block owns CX x CY coarse
 // columns (ghost columns included); it computes the fine residual on the (2 CX + 1) x (2 CY + 1) fine columns
 // their restriction stencils reach, one thread per column (the fine column between two tiles is computed by
 // both), keeps it in LDS over the staged x window and restricts from there, so the fine residual never goes
@@ -3374,7 +3332,8 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(LvArgs<T> L, Restri
         for (int k = 0; k < NZ; k++) dst[k] = o[k];
     }
     lds_barrier();
-    // restriction (k_mg_restrict_tab's arithmetic)
+    // restriction: smoothed along x on the coarse point's row and its two neighbour rows (injected on wall ghost rows),
+    // then along y; injected on the top level; zero on coarse ghost points
 #pragma unroll
     for (int q = 0; q < RES; q++) {
         const Point &p = pt[q];
@@ -3709,7 +3668,7 @@ struct BottomStep {
         else restrict_points(V, r, cb, cs);
         lds_barrier();
     }
-    // Coarse column c of the restriction (restrict_at's and k_mg_restrict_tab's arithmetic).  FULL: x and, in 3D, y are coarsened.
+    // Coarse column c of the restriction (restrict_at's arithmetic).  FULL: x and, in 3D, y are coarsened.
     template <bool FULL>
     struct Coarse {
         const T *q;          // its residual column

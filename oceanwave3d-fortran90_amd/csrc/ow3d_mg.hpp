@@ -7,7 +7,7 @@
 namespace ow3d_host {
 namespace mg {
 
-// LDS bytes of the tiled residual (16 x TY columns) and of the fused sweep (32 x TY columns).
+// LDS bytes of the tiled residual (16 x TY columns).
 template <typename T, int NZ, int TY>
 constexpr size_t residual_lds() {
     constexpr int WX = 20, WY = TY + 4, RS2 = 16 * TY + 4, LX = WX * WY > RS2 ? WX * WY : RS2;
@@ -463,38 +463,24 @@ void restrict_launch(const RestrictGeo &G, const T *rf, T *rc, T *xz, hipStream_
     }
     hipLaunchKernelGGL((k_mg_restrict<T>), dim3(grid_blocks((size_t)G.nxgc * G.nygc * G.nzgc)), dim3(256), 0, s, G, rf, rc, xz);
 }
-// Restriction from fine level F with its weight tables (F.ptab).
-template <typename T>
-void restrict_tab_launch(const RestrictGeo &G, const MgLevel<T> &F, const T *rf, T *rc, T *xz, hipStream_t s) {
-    switch (G.nzgc) {
-#define OW3D_NZ(N) case N: hipLaunchKernelGGL((k_mg_restrict_tab<T, N>), dim3((G.nxgc * N + 255) / 256, G.nygc), dim3(256), 0, s, G, \
-                                          (const T *)F.rxw.p, (const T *)F.ryw.p, rf, rc, xz); return;
-        OW3D_NZ(3) OW3D_NZ(4) OW3D_NZ(5) OW3D_NZ(6) OW3D_NZ(7) OW3D_NZ(8) OW3D_NZ(9) OW3D_NZ(10)
-        OW3D_NZ(11) OW3D_NZ(12) OW3D_NZ(13) OW3D_NZ(14)
-#undef OW3D_NZ
-    }
-    hipLaunchKernelGGL((k_mg_restrict<T>), dim3(grid_blocks((size_t)G.nxgc * G.nygc * G.nzgc)), dim3(256), 0, s, G, rf, rc, xz);
-}
-// Residual of level F and its restriction in one launch (k_mg_residual_restrict, F.ptab levels); false where it does not
-// apply (the caller then launches the two).  Coarse tiles of 8 x 7 columns: 17 x 15 fine columns, one per thread of 256.
+// Residual of level F and its restriction in one launch (k_mg_residual_restrict), on levels with weight tables (F.ptab).
+// Coarse tiles of 8 x 7 columns: 17 x 15 fine columns, one per thread of 256.
 template <typename T, int NZ>
-bool resrestrict_nz(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
+void resrestrict_nz(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
     constexpr int CX = 8, CY = 7;
     static_assert(ResRestrictLds<NZ, CX, CY>::TOTAL * sizeof(T) <= 65536, "residual tile exceeds 64 KiB of LDS");
     hipLaunchKernelGGL((k_mg_residual_restrict<T, NZ, CX, CY, 256>), dim3((G.nxgc + CX - 1) / CX, (G.nygc + CY - 1) / CY), dim3(256), 0, s,
                        F.args, G, (const T *)F.rxw.p, (const T *)F.ryw.p, x, b, rc, xz);
-    return true;
 }
 template <typename T>
-bool resrestrict_launch(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
-    if (!F.ptab || !F.args.dim3 || G.gx != 1 || G.gy != 1 || G.nzgc != F.g.nzg) return false;
+int resrestrict_launch(const MgLevel<T> &F, const RestrictGeo &G, const T *x, const T *b, T *rc, T *xz, hipStream_t s) {
     switch (F.g.nzg) {
-#define OW3D_NZ(N) case N: return resrestrict_nz<T, N>(F, G, x, b, rc, xz, s);
+#define OW3D_NZ(N) case N: resrestrict_nz<T, N>(F, G, x, b, rc, xz, s); return 0;
         OW3D_NZ(3) OW3D_NZ(4) OW3D_NZ(5) OW3D_NZ(6) OW3D_NZ(7) OW3D_NZ(8) OW3D_NZ(9) OW3D_NZ(10)
         OW3D_NZ(11) OW3D_NZ(12) OW3D_NZ(13) OW3D_NZ(14)
 #undef OW3D_NZ
     }
-    return false;
+    return -1;
 }
 // Prolongation onto fine level F from its interpolation tables (F.ptab), else prolong_launch.
 template <typename T>
@@ -655,11 +641,12 @@ int vcycle(ow3d_tank *t, std::vector<std::unique_ptr<MgLevel<T>>> &mg, int k, co
     G.spec = L.args.spec;
     // the coarse iterate is cleared where something reads it: not by the dense solve, nor by a first sweep from zero
     T *xz = k == 1 || (t->fused_rb && t->cfg.nu1 >= 1) ? nullptr : C.x.p;
-    if (!resrestrict_launch<T>(L, G, cur, b, C.b.p, xz, s)) {
+    if (L.ptab) {
+        if (resrestrict_launch<T>(L, G, cur, b, C.b.p, xz, s)) return -1;
+    } else {
         if (!L.r.p) { err() = "multigrid level has no residual buffer"; return -1; }   // needs_r says otherwise
         if (mg_launch<T>(L.args, 0, 0, cur, b, L.r.p, s)) return -1;
-        if (L.ptab) restrict_tab_launch<T>(G, L, (const T *)L.r.p, C.b.p, xz, s);
-        else restrict_launch<T>(G, (const T *)L.r.p, C.b.p, xz, s);
+        restrict_launch<T>(G, (const T *)L.r.p, C.b.p, xz, s);
     }
     T *ccur = C.x.p;
     if (vcycle<T>(t, mg, k - 1, C.b.p, ccur, s)) return -1;

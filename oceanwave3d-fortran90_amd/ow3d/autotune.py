@@ -104,16 +104,12 @@ def tune_class(spec, mg_precision=1, warmup=3, steps=3, log=None):
         T.time_matvec(3)
         mv[v] = 1e3 * T.time_matvec(30)
     v_best = min(mv, key=mv.get)
-    thr = {}
-    for n in (0,):   # (the sweeps' block sizes follow from their tiles)
-        T.tune(v_best, n)
-        thr[n] = 1e3 * _time_steps(T, dt, 1, steps)
-    n_best = min(thr, key=thr.get)
+    T.tune(v_best, 0)
+    ms = 1e3 * _time_steps(T, dt, 1, steps)
     T.close()
-    choice = {"mg_maxgrids": L, "matvec_variant": v_best, "sweep_threads": n_best,
-              "ms_per_step": round(thr[n_best], 3), "levels_ms": {str(k): round(v, 3) for k, v in per_levels.items()},
-              "matvec_us": {str(k): round(v, 2) for k, v in mv.items()},
-              "sweep_threads_ms": {str(k): round(v, 3) for k, v in thr.items()}}
+    choice = {"mg_maxgrids": L, "matvec_variant": v_best, "sweep_threads": 0,   # (ow3d_tune: no effect)
+              "ms_per_step": round(ms, 3), "levels_ms": {str(k): round(v, 3) for k, v in per_levels.items()},
+              "matvec_us": {str(k): round(v, 2) for k, v in mv.items()}}
     if log:
         log(f"{class_key(base)}: {choice}")
     return choice
