@@ -2724,8 +2724,9 @@ __device__ __forceinline__ void store_rows(O *__restrict__ dst, size_t pitch, co
 }
 
 // k_mg_sweep for large 3D levels (same modes, same arithmetic): there the sweep is bound by the throughput of its
-// HBM accesses and by its arithmetic, not by latency (513^2 x 10, FP32: 28 us, of which 12 are the loads, 12 the line
-// solves and 2 the stores; 46 us with the row-per-thread form; FP64 39-42 us against 71-73).  All fields move through LDS in whole rows (column by column,
+// HBM accesses and by its arithmetic, not by latency (513^2 x 10, first / last sweep of an application, FP32: 30.0 /
+// 28.4 us, of which 12 are the loads, 12 the line solves and 2 the stores, 46-48 with the row-per-thread form; FP64
+// 39.6 / 49.8 us, 71-73 before).  All fields move through LDS in whole rows (column by column,
 // each lane's 40 bytes apart, the address units were busy 60% of a 513^2 sweep's 26 us), the line matrices are
 // formed in registers (reading the records costs more bytes than the arithmetic costs time), the coarse window and
 // then the right-hand sides share one LDS region, and the columns next to a wall are a second pass of the tiles
@@ -3635,7 +3636,7 @@ struct BottomStep {
             if (it == nu) break;
             if (it > 0) { column(cur, 0); column(nxt, 1); }
 #pragma unroll 1
-            for (int c = 0; c < 2; c++) {   // (one copy of the code: the kernel stays within the reach of short branches)
+            for (int c = 0; c < 2; c++) {   // (one copy of the code: see k_mg_bottom)
                 half(cur, zero && c == 0);
                 lds_barrier();
                 cur = nxt;
@@ -3847,6 +3848,10 @@ __device__ __forceinline__ void bottom_dense(int n, int pitch, const M *__restri
 }
 
 // PART 0: the whole; 1: down to the right-hand side of level 0; 2: from its solution upwards.
+// Size: at most 97 KB of code (FP64, 14 levels), less than the 128 KiB that a branch instruction reaches, in every
+// instance; the loops over sweeps, colours and columns stay rolled for it.  A build with 235 KB (four unrolled copies of the
+// residual), whose branches go through register-indirect jumps, gave wrong FP64 values with 10 sigma levels and right
+// ones elsewhere.  Why is not known: the source was the same up to the unrolling, and the jumps are suspected only.
 template <typename T, int NZ, bool D3>
 __global__ __launch_bounds__(MG_BOTTOM_NT) void k_mg_bottom(const BottomArgs<T> *__restrict__ args, const int *skip, int part) {
     constexpr int NT = MG_BOTTOM_NT;

@@ -540,14 +540,16 @@ void sweep_tiles(const LvArgs<T> &L, const T *xin, T *xout, const T *b, hipStrea
 }
 // Levels whose column records are kept (up to SWEEP_RECORD_POINTS points, and all x-z levels) take the latency-bound
 // kernel, larger ones the tiled one.  At 257^2 x 10 the first takes 8.4 / 9.4 us (from zero / with the correction; FP64
-// 12.3 / 18.5) and the second 13 / 18 (18 / 23); at 513^2 x 10 both take 27-28 us in FP32, and in FP64 45-49 us and
-// 39-42, the records' 76 MB being the difference.
+// 12.3 / 18.5) and the second 13 / 18 (18 / 23).  At 513^2 x 10 (first / last sweep of an application) the first takes
+// 28.0 / 29.9 us in FP32 and 44.0 / 60.0 in FP64, the second 30.0 / 28.4 and 39.6 / 49.8: the same sum in FP32, where
+// the records would only take memory, and 14 us less in FP64, where they are 76 MB more to read.
 template <typename T, int NZ>
 void sweep_nz(const LvArgs<T> &L, const T *xin, T *xout, const T *b, hipStream_t s, const double *r0, T *bout, double *uout,
               const ProArgs<T> *pro, bool zero, bool ghosts) {
     if (!L.dim3) sweep_tiles<T, NZ, 66, 1, false>(L, xin, xout, b, s, r0, bout, uout, nullptr, zero, ghosts);
     else if (L.fac) sweep_tiles<T, NZ, 18, 8, false>(L, xin, xout, b, s, r0, bout, uout, pro, zero, ghosts);
-    // 36 x 8 columns fill 190 of 192 threads of the red half; in FP64 such a tile would exceed 64 KiB
+    // 36 x 8 columns fill 190 of 192 threads of the red half.  FP64 takes 18 x 8 (41 KB of LDS): 36 x 8 is 76 KB, still two
+    // blocks per CU, and took 41.4 / 51.6 us at 513^2 x 10 where 18 x 8 takes 39.6 / 49.8
     else sweep_tiles<T, NZ, sizeof(T) == 4 ? 36 : 18, 8, true>(L, xin, xout, b, s, r0, bout, uout, pro, zero, ghosts);
 }
 
