@@ -169,7 +169,8 @@ int ow3d_step_stats(const ow3d_tank *t, long long *replays, long long *captures,
  * and has no effect (a sweep's block follows from its tile).
  * Results do not depend on them beyond rounding. */
 int ow3d_tune(ow3d_tank *t, int matvec_variant, int sweep_threads);
-/* Device memory held by a handle, and what ow3d_create would allocate for cfg (admission control). */
+/* Device memory held by a handle, and what ow3d_create would allocate for cfg (admission control; under the environment
+ * switches OW3D_MG_BOTTOM and OW3D_MG_FUSED_RB as ow3d_create reads them). */
 long long ow3d_device_bytes(const ow3d_tank *t);
 long long ow3d_estimate_bytes(const ow3d_config *cfg);
 /* Multigrid hierarchy ow3d_create would build for cfg: number of levels and unknowns of the coarsest
